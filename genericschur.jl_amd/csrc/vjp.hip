@@ -9,8 +9,11 @@
 //     Abar = Re( sum_k c_k y_k x_k^H ),   c_k = gbar_k / conj(y_k^H x_k),
 // i.e. Re(X^{-H} diag(gbar) X^H).  The eigenvectors are recomputed from the
 // Schur factors by the eigenvector kernels (normalised, any scaling cancels
-// in c_k y_k x_k^H); this kernel forms c_k and the rank-n sum, one
-// workgroup per matrix, with the two n x n complex factors staged in LDS.
+// in c_k y_k x_k^H); the kernels here form c_k and the rank-n sum: one
+// workgroup per matrix with the two n x n complex factors staged in LDS, or,
+// above the LDS-resident orders, as FP64 MFMA tiles.
+#include <algorithm>
+
 #include "dev_common.h"
 #include "internal.h"
 
@@ -75,42 +78,132 @@ template <int NT> __global__ void __launch_bounds__(NT) vjp_assemble_kernel(VjpA
   if (tid == 0) a.info[m] = *bad;
 }
 
-// Orders whose two factors do not fit LDS: c_k for one matrix, one
-// wavefront per column, with the factors split into planes for a real GEMM:
-// P = [Re(Y C) | Im(Y C)] and Q = [Re X | Im X] (n x 2n each, column-major,
-// ld = n), so that Abar = Re(Y C X^H) = P Q^T.  info = 1 when some
-// y_k^H x_k vanished.
-__global__ void __launch_bounds__(256) vjp_planes_kernel(int n, const zd* VR, const zd* VL, const zd* g,
-                                                         double* P, double* Q, int32_t* info) {
+// Orders whose two factors do not fit LDS, every matrix of a size class in
+// two launches.  First, in place in the left vectors' buffer, y_k := c_k y_k
+// (one wavefront per column); info = 1 when some y_k^H x_k vanished.
+__global__ void __launch_bounds__(256) vjp_scale_kernel(VjpArgs a, zd* VL) {
+  const int m = a.order[blockIdx.y];
+  const int n = a.n[m];
   const int lane = threadIdx.x & 63;
   const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (k >= n) return;
-  const zd* x = VR + (int64_t)k * n;
-  const zd* y = VL + (int64_t)k * n;
+  const zd* x = reinterpret_cast<const zd*>(a.VR) + a.off[m] + (int64_t)k * n;
+  zd* y = VL + a.off[m] + (int64_t)k * n;
   zd s = zr(0.0);
   for (int i = lane; i < n; i += 64) s = s + zconj(y[i]) * x[i];
   s = wave_zsum(s);
   const zd d = zconj(s);
   const bool zero = d.x == 0.0 && d.y == 0.0;
-  const zd c = zero ? zr(0.0) : g[k] / d;
-  if (zero && lane == 0) *info = 1;
-  const int64_t nn = (int64_t)n * n;
-  for (int i = lane; i < n; i += 64) {
-    const zd t = c * y[i];
-    P[i + (int64_t)k * n] = t.x;
-    P[nn + i + (int64_t)k * n] = t.y;
-    Q[i + (int64_t)k * n] = x[i].x;
-    Q[nn + i + (int64_t)k * n] = x[i].y;
-  }
+  const zd c = zero ? zr(0.0) : (reinterpret_cast<const zd*>(a.gbar) + a.woff[m])[k] / d;
+  if (zero && lane == 0) a.info[m] = 1;
+  for (int i = lane; i < n; i += 64) y[i] = c * y[i];
 }
 
-hipError_t launch_vjp_planes(int n, const double* VR, const double* VL, const double* g, double* P, double* Q,
-                             int32_t* info, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(vjp_planes_kernel, dim3((n + 3) / 4), dim3(256), 0, s, n, reinterpret_cast<const zd*>(VR),
-                     reinterpret_cast<const zd*>(VL), reinterpret_cast<const zd*>(g), P, Q, info);
+// Then Abar(r, s) = sum_k Re(y_k[r] conj(x_k[s])), an n x n x 2n real
+// product of the interleaved factors (k and the real / imaginary part are
+// the contraction index) on v_mfma_f64_16x16x4_f64 (operand layout in
+// dgemm.hip).  One workgroup of four wavefronts owns a 64 x 64 tile of one
+// matrix, each wavefront 32 x 32; slabs of 8 vectors (16 contraction
+// entries) through two LDS buffers, the next slab's loads in flight during
+// the current slab's MFMAs.  Bound by the reads of the two factors (16
+// bytes per 2 flops and tile side).  One launch covers every matrix of the
+// class instead of a GEMM per matrix, whose single 128 x 128 tile left 255
+// CUs idle: 4096 real matrices n ~ U{16..128}, the 2119 of order above 70
+// took 105 ms
+// more in 6357 launches (forward and backward 146.9 -> 42.3 ms).
+constexpr int VT = 64, VKB = 8, VLD = VT + 16;
+__global__ void __launch_bounds__(256) vjp_gemm_kernel(VjpArgs a) {
+  __shared__ double As[2][2 * VKB * VLD], Bs[2][2 * VKB * VLD];
+  typedef double v4d __attribute__((ext_vector_type(4)));
+  const int m = a.order[blockIdx.z];
+  const int n = a.n[m];
+  const int r0 = blockIdx.x * VT, s0 = blockIdx.y * VT;
+  if (r0 >= n || s0 >= n) return;
+  const zd* Y = reinterpret_cast<const zd*>(a.VL) + a.off[m];
+  const zd* X = reinterpret_cast<const zd*>(a.VR) + a.off[m];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = (wave & 1) * 32, wc = (wave >> 1) * 32;
+  const int ty = min(r0 + lane, n - 1), tx = min(s0 + lane, n - 1);
+  const bool vy = r0 + lane < n, vx = s0 + lane < n;
+  zd ry[2], rx[2];
+  // unconditional loads from clamped addresses; entries outside the factors
+  // are zeroed when staged
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int64_t k = min(k0 + wave + 4 * q, n - 1);
+      ry[q] = Y[ty + k * n];
+      rx[q] = X[tx + k * n];
+    }
+  };
+  auto stage = [&](int k0, int buf) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int kk = wave + 4 * q;
+      const bool vk = k0 + kk < n;
+      As[buf][(2 * kk) * VLD + lane] = (vk && vy) ? ry[q].x : 0.0;
+      As[buf][(2 * kk + 1) * VLD + lane] = (vk && vy) ? ry[q].y : 0.0;
+      Bs[buf][(2 * kk) * VLD + lane] = (vk && vx) ? rx[q].x : 0.0;
+      Bs[buf][(2 * kk + 1) * VLD + lane] = (vk && vx) ? rx[q].y : 0.0;
+    }
+  };
+  v4d acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  const int ns = (n + VKB - 1) / VKB;
+  fetch(0);
+  stage(0, 0);
+  for (int sl = 0; sl < ns; ++sl) {
+    const int buf = sl & 1;
+    __syncthreads();
+    fetch((sl + 1) * VKB);
+#pragma unroll
+    for (int k4 = 0; k4 < 2 * VKB / 4; ++k4) {
+      const int kk = 4 * k4 + (lane >> 4);
+      double af[2], bf[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) af[i] = As[buf][kk * VLD + wr + 16 * i + (lane & 15)];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) bf[j] = Bs[buf][kk * VLD + wc + 16 * j + (lane & 15)];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j], af[i], acc[i][j], 0, 0, 0);
+    }
+    if (sl + 1 < ns) stage((sl + 1) * VKB, buf ^ 1);
+  }
+  double* Ab = a.Abar + a.off[m];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gr = r0 + wr + 16 * i + (lane & 15), gc = s0 + wc + 16 * j + (lane >> 4) + 4 * r;
+        if (gr < n && gc < n) Ab[gr + (int64_t)gc * n] = acc[i][j][r];
+      }
+}
+
+// a.order lists matrices whose orders need the same number of tiles; VL is
+// a.VL, writable (scaled in place)
+hipError_t launch_vjp_class(const VjpArgs& a, double* VL, int nmax, hipStream_t s) {
+  if (a.count <= 0 || nmax <= 0) return hipSuccess;
+  const int nt = (nmax + VT - 1) / VT;
+  // grid dimensions y and z hold at most 65535
+  for (int first = 0; first < a.count; first += 65535) {
+    VjpArgs b = a;
+    b.order = a.order + first;
+    b.count = std::min(a.count - first, 65535);
+    hipLaunchKernelGGL(vjp_scale_kernel, dim3((nmax + 3) / 4, b.count), dim3(256), 0, s, b,
+                       reinterpret_cast<zd*>(VL));
+    hipLaunchKernelGGL(vjp_gemm_kernel, dim3(nt, nt, b.count), dim3(256), 0, s, b);
+  }
   return hipGetLastError();
 }
+
+int vjp_tiles(int n) { return (n + VT - 1) / VT; }
 
 __global__ void vjp_info_clear_kernel(int32_t* info, int count) {
   const int i = blockIdx.x * 256 + threadIdx.x;

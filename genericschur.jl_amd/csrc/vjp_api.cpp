@@ -125,41 +125,35 @@ extern "C" int gs_eig_vjp_batched_d(gs_handle* h, int64_t count, const int32_t* 
     if ((e = launch_dtrevc(t, nsmall, s)) != hipSuccess) return handle_fail_hip(h, e, "eigenvector launch");
   }
   // orders whose two factors fit LDS: one workgroup per matrix; larger
-  // ones (first in the descending order): c_k and the planes of each
-  // matrix, then Abar = P Q^T as one FP64 MFMA GEMM of n x n x 2n
+  // ones (first in the descending order) two launches for each run of
+  // matrices with the same number of tiles, their info cleared first (the
+  // tiles only raise it)
   int64_t nlarge = 0;
   while (nlarge < count && vjp_lds_bytes(n[order[nlarge]]) > 160 * 1024) ++nlarge;
+  VjpArgs v;
+  v.n = d_n;
+  v.off = d_off;
+  v.woff = d_woff;
+  v.VR = static_cast<const double*>(bVR.p);
+  v.VL = static_cast<const double*>(bVL.p);
+  v.gbar = dG;
+  v.Abar = dA;
+  v.info = dI;
+  if (nlarge > 0 && (e = launch_vjp_info_clear(dI, (int)count, s)) != hipSuccess)
+    return handle_fail_hip(h, e, "VJP launch");
+  for (int64_t q = 0; q < nlarge;) {
+    int64_t q1 = q + 1;
+    while (q1 < nlarge && vjp_tiles(n[order[q1]]) == vjp_tiles(n[order[q]])) ++q1;
+    v.order = d_order + q;
+    v.count = (int)(q1 - q);
+    if ((e = launch_vjp_class(v, static_cast<double*>(bVL.p), n[order[q]], s)) != hipSuccess)
+      return handle_fail_hip(h, e, "VJP launch");
+    q = q1;
+  }
   if (nlarge < count) {
-    VjpArgs v;
     v.order = d_order + nlarge;
     v.count = (int)(count - nlarge);
-    v.n = d_n;
-    v.off = d_off;
-    v.woff = d_woff;
-    v.VR = static_cast<const double*>(bVR.p);
-    v.VL = static_cast<const double*>(bVL.p);
-    v.gbar = dG;
-    v.Abar = dA;
-    v.info = dI;
     if ((e = launch_vjp_assemble(v, n[order[nlarge]], s)) != hipSuccess) return handle_fail_hip(h, e, "VJP launch");
-  }
-  if (nlarge > 0) {
-    const int nl = n[order[0]];
-    DevBuf& planes = handle_buf(h, 12);
-    if ((e = planes.ensure(8 * 4 * (size_t)nl * nl)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
-    double* P = static_cast<double*>(planes.p);
-    double* Q = P + 2 * (size_t)nl * nl;
-    const double* vr = static_cast<const double*>(bVR.p);
-    const double* vl = static_cast<const double*>(bVL.p);
-    for (int64_t q = 0; q < nlarge; ++q) {
-      const int32_t mi = order[q];
-      const int nm = n[mi];
-      if ((e = launch_vjp_info_clear(dI + mi, 1, s)) != hipSuccess ||
-          (e = launch_vjp_planes(nm, vr + 2 * off[mi], vl + 2 * off[mi], dG + 2 * woff[mi], P, Q, dI + mi, s)) !=
-              hipSuccess ||
-          (e = launch_dgemm(false, true, nm, nm, 2 * nm, 1.0, P, nm, Q, nm, 0.0, dA + off[mi], nm, s)) != hipSuccess)
-        return handle_fail_hip(h, e, "VJP launch");
-    }
   }
   if (!dev) {
     std::vector<double> ha((size_t)span);

@@ -214,3 +214,24 @@ def test_order_above_1024(gs, oracle):
     d = np.sum(Y.conj() * X, axis=0)
     ref = np.real((Y * (g / np.conj(d))) @ X.conj().T)
     assert np.abs(Ab - ref).max() <= 1e-7 * max(1.0, np.abs(ref).max())
+
+
+def test_assembly_tile_edges(gs):
+    """The tiled assembly (orders above 70) at its tiles' edges, several tile
+    counts and an empty matrix in one batch, against the same sum formed from
+    this library's eigenvectors; each entry sums n terms of modulus at most
+    |c_k| (unit vectors), so the bound is 8 n eps sum |c_k|."""
+    orders = (71, 0, 72, 127, 128, 129, 64, 192, 193, 96)
+    mats = [_sep_ginibre(n, 14) if n else np.zeros((0, 0)) for n in orders]
+    Ss = [gs.gschur(A) if A.size else _forward(gs, [A])[0] for A in mats]
+    rng = np.random.default_rng(17)
+    gbars = [rng.standard_normal(n) + 1j * rng.standard_normal(n) for n in orders]
+    Abs = _vjp(gs, mats, Ss, gbars)
+    for n, S, g, Ab in zip(orders, Ss, gbars, Abs):
+        print(f"case vjp tiles n={n}", flush=True)
+        if n == 0:
+            continue
+        X, Y = gs.geigvecs(S), gs.geigvecs(S, left=True)
+        c = g / np.conj(np.sum(Y.conj() * X, axis=0))
+        ref = np.real((Y * c) @ X.conj().T)
+        assert np.abs(Ab - ref).max() <= 8 * n * np.finfo(np.float64).eps * np.abs(c).sum()
