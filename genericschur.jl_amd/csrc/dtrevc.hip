@@ -5,157 +5,209 @@
 //   1x1 / 2x2 solves  _xsolve util.jl:698-751, _safe_lu_solve! :603-687
 //   unit 2-norm, largest entry real: _enormalize! util.jl:572-592
 //
-// Same organisation as the complex kernel: T (upper triangle plus the
-// subdiagonal of the 2x2 blocks) in LDS, one eigenvector (or conjugate
-// pair) per wavefront with the complex solution in registers, solutions
-// parked in V, then back-transform by Z and normalisation.  The conjugate
-// partner of a complex pair is written last as the conjugate of the
-// finished column, which equals the reference's copy-then-normalise.
-#include <type_traits>
+// Same organisation as the complex kernels (trevc_grid.h): one wavefront per
+// eigenvector (or conjugate pair) with the complex solution in its lanes.
+// The conjugate partner of a complex pair is written last as the conjugate
+// of the finished column, which equals the reference's copy-then-normalise.
+#include <algorithm>
 
 #include "dev_common.h"
 #include "internal.h"
-#include "trevc_big.h"
+#include "trevc_grid.h"
 #include "wavevec.h"
 
 namespace gs {
 
-
-GS_DEV int trd(int i, int j) { return (j * (j + 1)) / 2 + i; }
-
-// Entry (i, j), i <= j, of T: from the compact copy in LDS, or from T in
-// global memory for orders whose triangle does not fit a CU's LDS.
-struct TriLdsD {
-  const double* p;
-  GS_DEV double operator()(int i, int j) const { return p[trd(i, j)]; }
+// One step of a substitution, (a A - lam I) x = s B for the 1 x 1 or 2 x 2
+// diagonal block A at the step (_xsolve, util.jl:698-751, _safe_lu_solve!
+// :603-687, complete pivoting), split in two: what does not depend on B is
+// factored for the 64 rows of a chunk at once, one row per lane (DFac in
+// LDS); a step then reads its factors as broadcasts and applies them to B.
+// The operations on B are those of the unsplit form, in its order.  The
+// factorization's moduli and divisions are most of a step's instructions,
+// and every lane used to repeat them at every step.
+struct DFac {
+  zd l;       // 2 x 2: A21 / A11 after pivoting; 1 x 1: Smith's (ratio, denominator)
+  zd u;       // 2 x 2: A12 / A11
+  zd t0, t1;  // 2 x 2: 1 / A11, 1 / A22
+  double a0, a3;  // 2 x 2: |A11|, |A22|; 1 x 1: a0 = abs1 of the pivot
+  double beta;    // the column norm(s) of the overflow guard
+  double flags;   // bits below
 };
-struct GlobD {
-  const double* p;
-  int64_t ld;
-  GS_DEV double operator()(int i, int j) const { return p[i + (int64_t)j * ld]; }
-};
+enum { DF_TWO = 1, DF_IP = 2, DF_JP = 4, DF_SMALL = 8, DF_SWAP = 16 };
 
-// T entry (0-based) from compact upper storage + subdiagonal
-template <class TA> GS_DEV double Tat(const TA& Tc, const double* sub, int i, int j) {
-  if (i <= j) return Tc(i, j);
-  if (i == j + 1) return sub[j];
-  return 0.0;
+GS_DEV void dfac1(DFac& f, double diag, zd lam, double smin, double beta) {
+  smin = fmax(smin, 2.0 * GS_FMIN);
+  double csr = diag - lam.x, csi = -lam.y;
+  double cnorm = fabs(csr) + fabs(csi);
+  if (cnorm < smin) {
+    csr = smin;
+    csi = 0.0;
+    cnorm = smin;
+  }
+  // Smith's division by (csr, csi): the part without the numerator
+  const bool sw = fabs(csi) > fabs(csr);
+  const double r = sw ? csr / csi : csi / csr;
+  const double d = sw ? csr * r + csi : csr + csi * r;
+  f.l = zmk(r, d);
+  f.a0 = cnorm;
+  f.beta = beta;
+  f.flags = sw ? (double)DF_SWAP : 0.0;
 }
 
-// _safe_lu_solve! (util.jl:603-687) for a complex 2x2 system; A column-major
-// (a11, a21, a12, a22), b in/out.  Returns the scale.
-GS_DEV double safe_lu2(zd* A, zd* b) {
-  const double smallnum = GS_FMIN / GS_EPS;
-  double smin = 0.0;
-  for (int i = 0; i < 4; ++i) smin = fmax(smin, zabs(A[i]));
-  smin = fmax(GS_EPS * smin, smallnum);
-  // complete pivoting for i = 1: the last maximal entry in (ip, jp) order
-  int ipsv = 0, jpsv = 0;
-  double xmax = 0.0;
-  for (int ip = 0; ip < 2; ++ip)
-    for (int jp = 0; jp < 2; ++jp)
-      if (zabs(A[ip + 2 * jp]) >= xmax) {
-        xmax = zabs(A[ip + 2 * jp]);
-        ipsv = ip;
-        jpsv = jp;
-      }
-  if (ipsv != 0) {
-    for (int j = 0; j < 2; ++j) {
-      const zd t = A[0 + 2 * j];
-      A[0 + 2 * j] = A[1 + 2 * j];
-      A[1 + 2 * j] = t;
-    }
-    const zd t = b[0];
-    b[0] = b[1];
-    b[1] = t;
-  }
-  if (jpsv != 0) {
-    for (int j = 0; j < 2; ++j) {
-      const zd t = A[j + 0];
-      A[j + 0] = A[j + 2];
-      A[j + 2] = t;
-    }
-  }
-  if (zabs(A[0]) < smin) A[0] = zr(smin);
-  A[1] = A[1] / A[0];
-  b[1] = b[1] - A[1] * b[0];
-  A[3] = A[3] - A[1] * A[2];
-  if (zabs(A[3]) < smin) A[3] = zr(smin);
-  double scale = 1.0;
-  const double a8 = 8.0 * smallnum;
-  bool needscl = (a8 * zabs(b[0]) > zabs(A[0])) || (a8 * zabs(b[1]) > zabs(A[3]));
-  if (needscl) {
-    scale = (1.0 / 8.0) / fmax(zabs(b[0]), zabs(b[1]));
-    b[0] = b[0] * scale;
-    b[1] = b[1] * scale;
-  }
-  {
-    const zd t = zdiv(zr(1.0), A[3]);
-    b[1] = b[1] * t;
-  }
-  {
-    const zd t = zdiv(zr(1.0), A[0]);
-    b[0] = b[0] * t;
-    b[0] = b[0] - (t * A[2]) * b[1];
-  }
-  if (jpsv != 0) {
-    const zd t = b[0];
-    b[0] = b[1];
-    b[1] = t;
-  }
-  return scale;
-}
-
-// _xsolve (util.jl:698-751): (a A - bw I) x = s B, na = 1 or 2, A column-major.
-GS_DEV double xsolve_dev(int na, const double* Ae, zd bw, zd* B, double smin, double& xnorm) {
-  double s = 1.0;
-  const double small = 2.0 * GS_FMIN;
-  const double bignum = s / small;
-  smin = fmax(smin, small);
-  if (na == 1) {
-    double csr = Ae[0] - bw.x;
-    double csi = -bw.y;
-    double cnorm = fabs(csr) + fabs(csi);
-    if (cnorm < smin) {
-      csr = smin;
-      csi = 0.0;
-      cnorm = smin;
-    }
-    const double bnorm = zabs1(B[0]);
-    if (cnorm < 1.0 && bnorm > 1.0 && bnorm > bignum * cnorm) s = 1.0 / bnorm;
-    const zd x = (B[0] * s) / zmk(csr, csi);
-    xnorm = zabs1(x);
-    B[0] = x;
-    return s;
-  }
-  zd M[4];
-  double cmax = 0.0;
-  for (int j = 0; j < 2; ++j)
-    for (int i = 0; i < 2; ++i) {
-      zd z = zr(Ae[i + 2 * j]);
-      if (i == j) z = z - bw;
-      M[i + 2 * j] = z;
-      cmax = fmax(cmax, zabs1(z));
-    }
+// A column-major: a11, a21, a12, a22
+GS_DEV void dfac2(DFac& f, double a11, double a21, double a12, double a22, zd lam, double smin, double beta) {
+  smin = fmax(smin, 2.0 * GS_FMIN);
+  zd A[4] = {zr(a11) - lam, zr(a21), zr(a12), zr(a22) - lam};
+  int fl = DF_TWO;
+  const double cmax = fmax(fmax(zabs1(A[0]), zabs1(A[1])), fmax(zabs1(A[2]), zabs1(A[3])));
+  f.beta = beta;
   if (cmax < smin) {
+    f.flags = (double)(fl | DF_SMALL);
+    return;
+  }
+  const double m0 = zabs(A[0]), m1 = zabs(A[1]), m2 = zabs(A[2]), m3 = zabs(A[3]);
+  const double sm = fmax(GS_EPS * fmax(fmax(m0, m1), fmax(m2, m3)), GS_FMIN / GS_EPS);
+  // complete pivoting: the last maximal entry in (row, column) order
+  int ip = 0, jp = 0;
+  double xm = 0.0;
+  if (m0 >= xm) { xm = m0; ip = 0; jp = 0; }
+  if (m2 >= xm) { xm = m2; ip = 0; jp = 1; }
+  if (m1 >= xm) { xm = m1; ip = 1; jp = 0; }
+  if (m3 >= xm) { xm = m3; ip = 1; jp = 1; }
+  if (ip) {
+    const zd t = A[0], u = A[2];
+    A[0] = A[1];
+    A[1] = t;
+    A[2] = A[3];
+    A[3] = u;
+    fl |= DF_IP;
+  }
+  if (jp) {
+    const zd t = A[0], u = A[1];
+    A[0] = A[2];
+    A[2] = t;
+    A[1] = A[3];
+    A[3] = u;
+    fl |= DF_JP;
+  }
+  if (zabs(A[0]) < sm) A[0] = zr(sm);
+  A[1] = A[1] / A[0];
+  A[3] = A[3] - A[1] * A[2];
+  if (zabs(A[3]) < sm) A[3] = zr(sm);
+  f.l = A[1];
+  f.t1 = zdiv(zr(1.0), A[3]);
+  f.t0 = zdiv(zr(1.0), A[0]);
+  f.u = f.t0 * A[2];
+  f.a0 = zabs(A[0]);
+  f.a3 = zabs(A[3]);
+  f.flags = (double)fl;
+}
+
+GS_DEV double dapply1(const DFac& f, int fl, zd& B, double& xnorm) {
+  const double bignum = 1.0 / (2.0 * GS_FMIN);
+  double s = 1.0;
+  const double bnorm = zabs1(B);
+  if (f.a0 < 1.0 && bnorm > 1.0 && bnorm > bignum * f.a0) s = 1.0 / bnorm;
+  const zd a = B * s;
+  const bool sw = (fl & DF_SWAP) != 0;
+  const double p = sw ? a.y : a.x, q = sw ? a.x : a.y;
+  const double x = (p + q * f.l.x) / f.l.y, y = (q - p * f.l.x) / f.l.y;
+  B = zmk(x, sw ? -y : y);
+  xnorm = zabs1(B);
+  return s;
+}
+
+GS_DEV double dapply2(const DFac& f, int fl, zd* B, double smin, double& xnorm) {
+  double s = 1.0;
+  if (fl & DF_SMALL) {
+    const double bignum = 1.0 / (2.0 * GS_FMIN);
+    smin = fmax(smin, 2.0 * GS_FMIN);
     const double bnorm = fmax(zabs1(B[0]), zabs1(B[1]));
     if (smin < 1.0 && bnorm > 1.0 && bnorm > bignum * smin) s = 1.0 / bnorm;
-    const double t1 = s / smin;
-    B[0] = B[0] * t1;
-    B[1] = B[1] * t1;
+    const double t = s / smin;
+    B[0] = B[0] * t;
+    B[1] = B[1] * t;
   } else {
-    s = safe_lu2(M, B);
+    if (fl & DF_IP) {
+      const zd t = B[0];
+      B[0] = B[1];
+      B[1] = t;
+    }
+    B[1] = B[1] - f.l * B[0];
+    const double a8 = 8.0 * (GS_FMIN / GS_EPS);
+    // |b| <= abs1(b): the moduli only where the cheap bound cannot decide
+    if (!(a8 * zabs1(B[0]) <= f.a0 && a8 * zabs1(B[1]) <= f.a3) &&
+        ((a8 * zabs(B[0]) > f.a0) || (a8 * zabs(B[1]) > f.a3))) {
+      s = (1.0 / 8.0) / fmax(zabs(B[0]), zabs(B[1]));
+      B[0] = B[0] * s;
+      B[1] = B[1] * s;
+    }
+    B[1] = B[1] * f.t1;
+    B[0] = B[0] * f.t0;
+    B[0] = B[0] - f.u * B[1];
+    if (fl & DF_JP) {
+      const zd t = B[0];
+      B[0] = B[1];
+      B[1] = t;
+    }
   }
   xnorm = sqrt(zabs2(B[0]) + zabs2(B[1]));
   return s;
 }
+
+// The columns of T a substitution reads.  Up to R = 8 entries per lane the two
+// that the next step needs are loaded a step ahead; above, each entry is read
+// where it is used.
+template <int R, class TA, bool LEFT> struct DCols {
+  static constexpr bool PF = R <= 8;
+  static constexpr int NR = PF ? R : 1;
+  const TA& Tc;
+  int n;  // rows and columns that may be read
+  double ca[NR], cb[NR], na[NR], nb[NR];
+  // line j: column j (right) or row j (left) of T, lanes along it
+  GS_DEV double at(int i, int j) const { return LEFT ? Tc(j, i) : Tc(i, j); }
+  GS_DEV void load(double (&c)[NR], int j) const {
+    if constexpr (PF) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) c[q] = at(min((int)(threadIdx.x & 63) + 64 * q, n - 1), min(max(j, 0), n - 1));
+    }
+  }
+  static constexpr int D = LEFT ? 1 : -1;
+  // lines j and j + D in ca, cb; the two after them on the way
+  GS_DEV void start(int j) {
+    load(ca, j);
+    load(cb, j + D);
+  }
+  GS_DEV void ahead(int j) {
+    load(na, j + 2 * D);
+    load(nb, j + 3 * D);
+  }
+  GS_DEV void advance(bool two) {
+    if constexpr (PF) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        ca[q] = two ? na[q] : cb[q];
+        cb[q] = two ? nb[q] : na[q];
+      }
+    }
+  }
+  GS_DEV double first(int q, int i, int j) const {
+    if constexpr (PF) return ca[q];
+    else return at(i, j);
+  }
+  GS_DEV double second(int q, int i, int j) const {
+    if constexpr (PF) return cb[q];
+    else return at(i, j);
+  }
+};
 
 // ------------------------------------------------------------- right
 // Solution for column ki (0-based) with ip = 0 (real wr) or -1 (pair,
 // lambda = wr + i wi, ki the second row of the block).  Entries 0..ki hold
 // the vector on exit.
 template <int R, class TA, class VEC> GS_DEV void dsolve_right(const TA& Tc, const double* sub, const double* tnorms, int ki,
-                                                     int ip, double smallnum, double bignum, VEC& v) {
+                                                     int ip, double smallnum, double bignum, VEC& v, DFac* fac) {
   const int lane = threadIdx.x & 63;
   const double ulp = GS_EPS;
   const double wr = Tc(ki, ki);
@@ -191,56 +243,66 @@ template <int R, class TA, class VEC> GS_DEV void dsolve_right(const TA& Tc, con
     jtop = ki - 2;
   }
   int j = jtop;
+  DCols<R, TA, false> dc{Tc, ki + 1};
+  if (j >= 0) dc.start(j);
+  int chunk = -1;  // the 64 rows whose factors are in fac
   while (j >= 0) {
-    const bool two = (j > 0) && (sub[j - 1] != 0.0);
+    dc.ahead(j);
+    if ((j >> 6) != chunk) {
+      chunk = j >> 6;
+      const int i = 64 * chunk + lane;
+      wsync();
+      if (i <= j) {
+        DFac f;
+        if (i > 0 && sub[i - 1] != 0.0)
+          dfac2(f, Tc(i - 1, i - 1), sub[i - 1], Tc(i - 1, i), Tc(i, i), lam, smin, fmax(tnorms[i - 1], tnorms[i]));
+        else
+          dfac1(f, Tc(i, i), lam, smin, tnorms[i]);
+        fac[lane] = f;
+      }
+      wsync();
+    }
+    const DFac f = fac[j & 63];
+    const int fl = __builtin_amdgcn_readfirstlane((int)f.flags);
+    const bool two = (fl & DF_TWO) != 0;
+    zd B[2] = {v.get(j), zr(0.0)};
+    double t1, vscale;
     if (!two) {
-      zd B[1] = {v.get(j)};
-      const double Ae[1] = {Tc(j, j)};
-      double t1;
-      double vscale = xsolve_dev(1, Ae, lam, B, smin, t1);
-      if (t1 > 1.0 && tnorms[j] > bignum / t1) {
-        B[0] = B[0] / t1;
-        vscale /= t1;
-      }
-      if (vscale != 1.0) {
+      vscale = dapply1(f, fl, B[0], t1);
+    } else {
+      B[1] = B[0];
+      B[0] = v.get(j - 1);
+      vscale = dapply2(f, fl, B, smin, t1);
+    }
+    // t1 > 1 && beta > bignum / t1, the quotient only near the limit
+    if (t1 > 1.0 && !(f.beta * t1 <= 0.5 * bignum) && f.beta > bignum / t1) {
+      B[0] = B[0] / t1;
+      if (two) B[1] = B[1] / t1;
+      vscale /= t1;
+    }
+    if (vscale != 1.0) {
 #pragma unroll
-        for (int q = 0; q < R; ++q)
-          if (lane + 64 * q <= ki) v.v[q] = v.v[q] * vscale;
-      }
+      for (int q = 0; q < R; ++q)
+        if (lane + 64 * q <= ki) v.v[q] = v.v[q] * vscale;
+    }
+    if (!two) {
       v.set(j, B[0]);
 #pragma unroll
       for (int q = 0; q < R; ++q) {
         const int i = lane + 64 * q;
-        if (i < j) v.v[q] = v.v[q] - B[0] * Tc(i, j);
+        if (i < j) v.v[q] = v.v[q] - B[0] * dc.first(q, i, j);
       }
-      j -= 1;
     } else {
-      zd B[2] = {v.get(j - 1), v.get(j)};
-      const double Ae[4] = {Tc(j - 1, j - 1), sub[j - 1], Tc(j - 1, j), Tc(j, j)};
-      double t1;
-      double vscale = xsolve_dev(2, Ae, lam, B, smin, t1);
-      if (t1 > 1.0) {
-        const double beta = fmax(tnorms[j - 1], tnorms[j]);
-        if (beta > bignum / t1) {
-          B[0] = B[0] / t1;
-          B[1] = B[1] / t1;
-          vscale /= t1;
-        }
-      }
-      if (vscale != 1.0) {
-#pragma unroll
-        for (int q = 0; q < R; ++q)
-          if (lane + 64 * q <= ki) v.v[q] = v.v[q] * vscale;
-      }
       v.set(j - 1, B[0]);
       v.set(j, B[1]);
 #pragma unroll
       for (int q = 0; q < R; ++q) {
         const int i = lane + 64 * q;
-        if (i < j - 1) v.v[q] = (v.v[q] - B[0] * Tc(i, j - 1) - B[1] * Tc(i, j));
+        if (i < j - 1) v.v[q] = (v.v[q] - B[0] * dc.second(q, i, j - 1) - B[1] * dc.first(q, i, j));
       }
-      j -= 2;
     }
+    j -= two ? 2 : 1;
+    dc.advance(two);
   }
 }
 
@@ -250,7 +312,8 @@ template <int R, class TA, class VEC> GS_DEV void dsolve_right(const TA& Tc, con
 // Forward substitution in axpy form; the reference's overflow guards
 // (vmax, vcrit) and the j1 = j + 1 quirk of vectors.jl:627 are kept.
 template <int R, class TA, class VEC> GS_DEV void dsolve_left(const TA& Tc, const double* sub, const double* tnorms, int n,
-                                                    int ki, int ip, double smallnum, double bignum, VEC& v) {
+                                                    int ki, int ip, double smallnum, double bignum, VEC& v,
+                                                    DFac* fac) {
   const int lane = threadIdx.x & 63;
   const double ulp = GS_EPS;
   const double wr = Tc(ki, ki);
@@ -288,69 +351,76 @@ template <int R, class TA, class VEC> GS_DEV void dsolve_left(const TA& Tc, cons
     lam = zmk(wr, -wi);
   }
   const bool pair = (ip != 0);
-  double vmax = 1.0, vcrit = bignum;
+  double vmax = 1.0;  // the reference's vcrit is bignum / vmax
   int j = jstart;
+  DCols<R, TA, true> dc{Tc, n};
+  if (j < n) dc.start(j);
+  int chunk = -1;
   while (j < n) {
-    const bool blk = (j < n - 1) && (sub[j] != 0.0);
-    if (!blk) {
-      if (tnorms[j] > vcrit) {
-        const double t1 = 1.0 / vmax;
-#pragma unroll
-        for (int q = 0; q < R; ++q)
-          if (lane + 64 * q >= ki) v.v[q] = v.v[q] * t1;
-        vmax = 1.0;
-        vcrit = bignum;
+    dc.ahead(j);
+    if ((j >> 6) != chunk) {
+      chunk = j >> 6;
+      const int i = 64 * chunk + lane;
+      wsync();
+      if (i >= j && i < n) {
+        DFac f;
+        // with a pair the 2 x 2 guard reads tnorms[i-1]
+        if (i < n - 1 && sub[i] != 0.0)
+          dfac2(f, Tc(i, i), Tc(i, i + 1), sub[i], Tc(i + 1, i + 1), lam, smin,
+                fmax(tnorms[pair ? i - 1 : i + 1], tnorms[i]));
+        else
+          dfac1(f, Tc(i, i), lam, smin, tnorms[i]);
+        fac[lane] = f;
       }
-      zd B[1] = {v.get(j)};
-      const double Ae[1] = {Tc(j, j)};
-      double xn;
-      const double vscale = xsolve_dev(1, Ae, lam, B, smin, xn);
-      if (vscale != 1.0) {
-#pragma unroll
-        for (int q = 0; q < R; ++q)
-          if (lane + 64 * q >= ki) v.v[q] = v.v[q] * vscale;
-      }
-      v.set(j, B[0]);
-      vmax = fmax(pair ? zabs1(B[0]) : zabs(B[0]), vmax);
-      vcrit = bignum / vmax;
-      // remove x from the later right-hand sides
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int i = lane + 64 * q;
-        if (i > j && i < n) v.v[q] = v.v[q] - B[0] * Tc(j, i);
-      }
-      j += 1;
-    } else {
-      // 2x2 block at rows j, j+1; with a pair the guard reads tnorms[j-1]
-      const double beta = pair ? fmax(tnorms[j - 1], tnorms[j]) : fmax(tnorms[j + 1], tnorms[j]);
-      if (beta > vcrit) {
-        const double t1 = 1.0 / vmax;
-#pragma unroll
-        for (int q = 0; q < R; ++q)
-          if (lane + 64 * q >= ki) v.v[q] = v.v[q] * t1;
-        vmax = 1.0;
-        vcrit = bignum;
-      }
-      zd B[2] = {v.get(j), v.get(j + 1)};
-      const double Ae[4] = {Tc(j, j), Tc(j, j + 1), sub[j], Tc(j + 1, j + 1)};
-      double xn;
-      const double vscale = xsolve_dev(2, Ae, lam, B, smin, xn);
-      if (vscale != 1.0) {
-#pragma unroll
-        for (int q = 0; q < R; ++q)
-          if (lane + 64 * q >= ki) v.v[q] = v.v[q] * vscale;
-      }
-      v.set(j, B[0]);
-      v.set(j + 1, B[1]);
-      vmax = pair ? fmax(fmax(zabs1(B[0]), zabs1(B[1])), vmax) : fmax(fmax(zabs(B[0]), zabs(B[1])), vmax);
-      vcrit = bignum / vmax;
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int i = lane + 64 * q;
-        if (i > j + 1 && i < n) v.v[q] = v.v[q] - B[0] * Tc(j, i) - B[1] * Tc(j + 1, i);
-      }
-      j += 2;
+      wsync();
     }
+    const DFac f = fac[j & 63];
+    const int fl = __builtin_amdgcn_readfirstlane((int)f.flags);
+    const bool two = (fl & DF_TWO) != 0;
+    // beta > bignum / vmax, the quotient only near the limit
+    if (!(f.beta * vmax <= 0.5 * bignum) && f.beta > bignum / vmax) {
+      const double t1 = 1.0 / vmax;
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (lane + 64 * q >= ki) v.v[q] = v.v[q] * t1;
+      vmax = 1.0;
+    }
+    zd B[2] = {v.get(j), zr(0.0)};
+    double xn;
+    double vscale;
+    if (!two) {
+      vscale = dapply1(f, fl, B[0], xn);
+    } else {
+      B[1] = v.get(j + 1);
+      vscale = dapply2(f, fl, B, smin, xn);
+    }
+    if (vscale != 1.0) {
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (lane + 64 * q >= ki) v.v[q] = v.v[q] * vscale;
+    }
+    // abs1 bounds the modulus
+    const double b1 = two ? fmax(zabs1(B[0]), zabs1(B[1])) : zabs1(B[0]);
+    if (pair) vmax = fmax(b1, vmax);
+    else if (!(b1 <= vmax)) vmax = fmax(two ? fmax(zabs(B[0]), zabs(B[1])) : zabs(B[0]), vmax);
+    // remove x from the later right-hand sides
+    v.set(j, B[0]);
+    if (!two) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int i = lane + 64 * q;
+        if (i > j && i < n) v.v[q] = v.v[q] - B[0] * dc.first(q, i, j);
+      }
+    } else {
+      v.set(j + 1, B[1]);
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int i = lane + 64 * q;
+        if (i > j + 1 && i < n) v.v[q] = v.v[q] - B[0] * dc.first(q, i, j) - B[1] * dc.second(q, i, j + 1);
+      }
+    }
+    j += two ? 2 : 1;
+    dc.advance(two);
   }
 }
 
@@ -412,289 +482,90 @@ template <int R, class VEC> GS_DEV void enormalize_w(VEC& v, int n) {
   v.set(bi, zr(r0.x));
 }
 
-template <int NT, int R, bool GLOB> __global__ void __launch_bounds__(NT) dtrevc_kernel(TrevcArgsD a) {
+// Column norms, subdiagonal and block kinds, one wavefront per column.
+// kind: 0 a real eigenvalue; the row of a 2 x 2 block that solves its pair
+// (right: the second, -1; left: the first, 1); 2 its partner.  The reference
+// walks ki = n..1 (right) or 1..n (left) and skips the partner of each pair,
+// so within a run of nonzero subdiagonal entries (one entry, for a
+// quasi-triangular T) the distance from the end where the walk enters it
+// decides.
+__global__ void __launch_bounds__(256) dtrevc_norms_kernel(TrevcArgs a) {
+  const TrevcMat<double> t = trevc_mat<double>(a, blockIdx.y);
+  const int n = t.n;
+  const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (j >= n) return;
+  double s = 0.0;
+  for (int i = lane; i < j; i += 64) s += fabs(t.T[i + (int64_t)j * t.ldt]);
+  s = wave_sum(s);
+  if (lane != 0) return;
+  auto sub = [&](int i) { return (i >= 0 && i + 1 < n) ? t.T[(i + 1) + (int64_t)i * t.ldt] : 0.0; };
+  t.cn[j] = s;
+  t.sub[j] = sub(j);
+  int d = 0;
+  if (a.left) {
+    while (sub(j - 1 - d) != 0.0) ++d;
+    t.kind[j] = (d & 1) ? 2 : (sub(j) != 0.0 ? 1 : 0);
+  } else {
+    while (sub(j + d) != 0.0) ++d;
+    t.kind[j] = (d & 1) ? 2 : (sub(j - 1) != 0.0 ? -1 : 0);
+  }
+}
+
+// workgroup (t, matrix) solves column n-1-t (right) or t (left): the longest
+// solves are dispatched first
+template <int R, bool LEFT> __global__ void __launch_bounds__(64) dtrevc_solve_kernel(TrevcArgs a) {
   extern __shared__ double smem[];
-  const int b = blockIdx.x;
-  if (b >= a.count) return;
-  const int m = a.order ? a.order[b] : b;
-  const int n = a.n[m];
-  if (n <= 0) return;
-  const int64_t o = a.off[m];
-  const int64_t ldt = a.ldt > 0 ? a.ldt : n;
-  const int64_t ldz = a.ldz > 0 ? a.ldz : n;
-  const int64_t ldv = a.ldv > 0 ? a.ldv : n;
-  const double* Tg = a.T + o;
-  const double* Zg = a.Z ? a.Z + o : nullptr;
-  zd* Vg = reinterpret_cast<zd*>(a.V) + o;
-  double* Tl = smem;
-  double* sub = GLOB ? smem : Tl + (n * (n + 1)) / 2;
-  double* tnorms = sub + n;
-  int* kind = reinterpret_cast<int*>(tnorms + n);  // per column: 0 real, -1/+1 pair rows
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  constexpr int NW = NT / 64;
-  const bool left = a.left != 0;
-  if (!GLOB)
-    for (int j = 0; j < n; ++j)
-      for (int i = tid; i <= j; i += NT) Tl[trd(i, j)] = Tg[i + j * ldt];
-  for (int j = tid; j < n; j += NT) sub[j] = (j + 1 < n) ? Tg[(j + 1) + j * ldt] : 0.0;
-  __syncthreads();
-  typedef typename std::conditional<GLOB, GlobD, TriLdsD>::type TA;
-  TA Tc;
-  if constexpr (GLOB) Tc = GlobD{Tg, ldt};
-  else Tc = TriLdsD{Tl};
-  for (int j = tid; j < n; j += NT) {
-    double s = 0.0;
-    for (int i = 0; i < j; ++i) s += fabs(Tc(i, j));
-    tnorms[j] = s;
-    // right: the second row of a pair (T[j, j-1] != 0) solves; left: the first
-    const bool pr = (j > 0) && (sub[j - 1] != 0.0);
-    const bool pl = (j + 1 < n) && (sub[j] != 0.0);
-    kind[j] = left ? (pl ? 1 : 0) : (pr ? -1 : 0);
-  }
-  __syncthreads();
-  // the reference walks ki = n..1 (right) or 1..n (left) and skips the
-  // partner of each pair; mark the partners (ip == 1 / ip == -1 rows)
-  if (tid == 0) {
-    if (!left) {
-      for (int ki = n - 1; ki >= 0; --ki)
-        if (kind[ki] == -1) {
-          if (ki - 1 >= 0) kind[ki - 1] = 2;
-          --ki;
-        }
-    } else {
-      for (int ki = 0; ki < n; ++ki)
-        if (kind[ki] == 1) {
-          if (ki + 1 < n) kind[ki + 1] = 2;
-          ++ki;
-        }
-    }
-  }
-  __syncthreads();
-  const double ulp = GS_EPS;
-  const double smallnum = GS_FMIN * ((double)n / ulp);  // vectors.jl:146,475
-  const double bignum = (1.0 - ulp) / smallnum;
-  for (int t = w; t < n; t += NW) {
-    const int ki = left ? t : n - 1 - t;
-    const int kd = kind[ki];
-    if (kd == 2) continue;
-    WaveVecZ<R> v;
-    if (!left) dsolve_right<R>(Tc, sub, tnorms, ki, kd, smallnum, bignum, v);
-    else dsolve_left<R>(Tc, sub, tnorms, n, ki, kd, smallnum, bignum, v);
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int i = lane + 64 * q;
-      if (i < n) Vg[i + ki * ldv] = v.v[q];
-    }
-  }
-  __syncthreads();
-  for (int t = w; t < n; t += NW) {
-    const int ki = t;
-    const int kd = kind[ki];
-    if (kd == 2) continue;
-    WaveVecZ<R> x;
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int i = lane + 64 * q;
-      x.v[q] = (i < n) ? Vg[i + ki * ldv] : zr(0.0);
-    }
-    // solution support: right 0..ki, left ki..n-1
-    const int lo = left ? ki : 0, hi = left ? n : ki + 1;
-    WaveVecZ<R> y;
-    if (Zg) {
-      if ((!left && ki == 0 && kd == 0) || (left && ki == n - 1 && kd == 0)) {
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-          const int r = lane + 64 * q;
-          y.v[q] = (r < n) ? zr(Zg[r + (int64_t)ki * ldz]) : zr(0.0);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < R; ++q) y.v[q] = zr(0.0);
-        for (int i = lo; i < hi; ++i) {
-          const zd xi = x.get(i);
-#pragma unroll
-          for (int q = 0; q < R; ++q) {
-            const int r = lane + 64 * q;
-            if (r < n) y.v[q] = y.v[q] + Zg[r + (int64_t)i * ldz] * xi;
-          }
-        }
-        scale_by_max<R>(y, 0, n, false);
-        if (!left && kd == -1) {
-#pragma unroll
-          for (int q = 0; q < R; ++q) y.v[q] = zconj(y.v[q]);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int i = lane + 64 * q;
-        y.v[q] = (i >= lo && i < hi) ? x.v[q] : zr(0.0);
-      }
-      if (kd == 0) {
-        scale_by_max<R>(y, lo, hi, false);
-      } else {
-        if (!left) {
-#pragma unroll
-          for (int q = 0; q < R; ++q) y.v[q] = zconj(y.v[q]);
-        }
-        scale_by_max<R>(y, lo, hi, true);
-      }
-    }
-    if (a.normalize) enormalize_w<R>(y, n);
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int r = lane + 64 * q;
-      if (r < n) Vg[r + ki * ldv] = y.v[q];
-    }
-    // the conjugate partner of a pair
-    if (kd != 0) {
-      const int pk = left ? ki + 1 : ki - 1;
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = lane + 64 * q;
-        if (r < n) Vg[r + pk * ldv] = zconj(y.v[q]);
-      }
-    }
-  }
-}
-
-size_t dtrevc_lds_bytes(int n) { return 8 * ((size_t)n * (n + 1) / 2 + 2 * (size_t)n) + 4 * (size_t)n + 64; }
-static size_t dtrevc_glob_lds_bytes(int n) { return 8 * 2 * (size_t)n + 4 * (size_t)n + 64; }
-
-template <int NT, int R, bool GLOB> static void launch_dtrevc_t(const TrevcArgsD& a, size_t lds, hipStream_t s) {
-  (void)hipFuncSetAttribute((const void*)dtrevc_kernel<NT, R, GLOB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds);
-  hipLaunchKernelGGL((dtrevc_kernel<NT, R, GLOB>), dim3(a.count), dim3(NT), lds, s, a);
-}
-
-// Orders up to 192 keep T's triangle in LDS; above, T is read from global
-// memory (subdiagonal, column norms and block kinds in LDS), up to
-// dtrevc_max_n().
-hipError_t launch_dtrevc(const TrevcArgsD& a, int nmax, hipStream_t s) {
-  if (a.count <= 0) return hipSuccess;
-  if (nmax <= 64) launch_dtrevc_t<256, 1, false>(a, dtrevc_lds_bytes(nmax), s);
-  else if (nmax <= 128) launch_dtrevc_t<256, 2, false>(a, dtrevc_lds_bytes(nmax), s);
-  else if (nmax <= 192) launch_dtrevc_t<256, 3, false>(a, dtrevc_lds_bytes(nmax), s);
-  else if (nmax <= 256) launch_dtrevc_t<512, 4, true>(a, dtrevc_glob_lds_bytes(nmax), s);
-  else if (nmax <= 512) launch_dtrevc_t<512, 8, true>(a, dtrevc_glob_lds_bytes(nmax), s);
-  else if (nmax <= 1024) launch_dtrevc_t<256, 16, true>(a, dtrevc_glob_lds_bytes(nmax), s);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-int dtrevc_max_n() { return 1024; }
-
-// ------------------------------------------------------- larger orders
-// One matrix of order 1024 < n <= trevc_big_max_n() over the whole GPU:
-// the block kinds and column norms in global memory, one solve per
-// workgroup (a single wavefront whose solution vector lives in LDS,
-// WaveVecL), the solutions in a planar workspace X = [Re | Im] (n x 2n),
-// the back-transform [Re | Im] of Z X as one FP64 MFMA GEMM, then one
-// wavefront per column scales, normalises and writes V.  The per-column
-// steps are those of dtrevc_kernel.
-struct DBig {
-  int n, left, normalize;
-  const double* T;
-  int64_t ldt;
-  const double* Tt;  // T's transpose (left solves), ld n
-  const double* Z;   // may be null
-  int64_t ldz;
-  zd* V;
-  int64_t ldv;
-  double* sub;
-  double* tnorms;
-  int* kind;
-  double* X;  // n x 2n, ld n
-  double* Y;  // n x 2n, ld n
-};
-
-// subdiagonal and block kinds (as in dtrevc_kernel), one workgroup
-__global__ void __launch_bounds__(1024) dtrevc_big_kinds(DBig a) {
-  extern __shared__ double smem[];
-  int* kl = reinterpret_cast<int*>(smem);
-  const int n = a.n, tid = threadIdx.x;
-  const bool left = a.left != 0;
-  for (int j = tid; j < n; j += 1024) {
-    const double sj = (j + 1 < n) ? a.T[(j + 1) + (int64_t)j * a.ldt] : 0.0;
-    const double sp = (j > 0) ? a.T[j + (int64_t)(j - 1) * a.ldt] : 0.0;
-    a.sub[j] = sj;
-    kl[j] = left ? (sj != 0.0 ? 1 : 0) : (sp != 0.0 ? -1 : 0);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    if (!left) {
-      for (int ki = n - 1; ki >= 0; --ki)
-        if (kl[ki] == -1) {
-          if (ki - 1 >= 0) kl[ki - 1] = 2;
-          --ki;
-        }
-    } else {
-      for (int ki = 0; ki < n; ++ki)
-        if (kl[ki] == 1) {
-          if (ki + 1 < n) kl[ki + 1] = 2;
-          ++ki;
-        }
-    }
-  }
-  __syncthreads();
-  for (int j = tid; j < n; j += 1024) a.kind[j] = kl[j];
-}
-
-// workgroup t solves column n-1-t (right) or t (left): the longest solves
-// are dispatched first
-template <int R, class TA> __global__ void __launch_bounds__(64) dtrevc_big_solve(DBig a, TA Tc) {
-  extern __shared__ double smem[];
-  const int n = a.n, lane = threadIdx.x & 63, t = blockIdx.x;
-  const bool left = a.left != 0;
-  const int ki = left ? t : n - 1 - t;
-  const int kd = a.kind[ki];
-  double* xr = a.X + (int64_t)ki * n;
-  double* xi = xr + (int64_t)n * n;
+  const TrevcMat<double> t = trevc_mat<double>(a, blockIdx.y);
+  const int n = t.n, lane = threadIdx.x & 63, b = blockIdx.x;
+  if (b >= n) return;
+  const int ki = LEFT ? b : n - 1 - b;
+  const int kd = t.kind[ki];
+  zd* xo = t.X + (int64_t)ki * n;
   if (kd == 2) {
-    for (int i = lane; i < n; i += 64) {
-      xr[i] = 0.0;
-      xi[i] = 0.0;
-    }
+    for (int i = lane; i < n; i += 64) xo[i] = zr(0.0);
     return;
   }
   const double ulp = GS_EPS;
   const double smallnum = GS_FMIN * ((double)n / ulp);  // vectors.jl:146,475
   const double bignum = (1.0 - ulp) / smallnum;
-  WaveVecL<R> v{{reinterpret_cast<zd*>(smem)}};
-  if (!left) dsolve_right<R>(Tc, a.sub, a.tnorms, ki, kd, smallnum, bignum, v);
-  else dsolve_left<R>(Tc, a.sub, a.tnorms, n, ki, kd, smallnum, bignum, v);
+  WaveVec<R> v;
+  wavevec_bind(v.v, smem);
+  typedef typename std::conditional<LEFT, TransG<double>, ColG<double>>::type TA;
+  const TA Tc = LEFT ? TA{t.Tt, n} : TA{t.T, t.ldt};
+  __shared__ DFac fac[64];
+  if (!LEFT) dsolve_right<R>(Tc, t.sub, t.cn, ki, kd, smallnum, bignum, v, fac);
+  else dsolve_left<R>(Tc, t.sub, t.cn, n, ki, kd, smallnum, bignum, v, fac);
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int i = lane + 64 * q;
-    if (i < n) {
-      const zd z = v.v[q];
-      xr[i] = z.x;
-      xi[i] = z.y;
-    }
+    if (i < n) xo[i] = v.v[q];
   }
 }
 
-template <int R> __global__ void __launch_bounds__(64) dtrevc_big_finish(DBig a) {
+template <int R> __global__ void __launch_bounds__(64) dtrevc_finish_kernel(TrevcArgs a) {
   extern __shared__ double smem[];
-  const int n = a.n, lane = threadIdx.x & 63, ki = blockIdx.x;
+  const TrevcMat<double> t = trevc_mat<double>(a, blockIdx.y);
+  const int n = t.n, lane = threadIdx.x & 63, ki = blockIdx.x;
+  if (ki >= n) return;
   const bool left = a.left != 0;
-  const int kd = a.kind[ki];
+  const int kd = t.kind[ki];
   if (kd == 2) return;
-  WaveVecL<R> y{{reinterpret_cast<zd*>(smem)}};
+  WaveVec<R> y;
+  wavevec_bind(y.v, smem);
   const int lo = left ? ki : 0, hi = left ? n : ki + 1;
-  if (a.Z) {
+  zd* vo = t.V + (int64_t)ki * t.ldv;
+  if (t.Z) {
     if ((!left && ki == 0 && kd == 0) || (left && ki == n - 1 && kd == 0)) {
 #pragma unroll
       for (int q = 0; q < R; ++q) {
         const int r = lane + 64 * q;
-        y.v[q] = (r < n) ? zr(a.Z[r + (int64_t)ki * a.ldz]) : zr(0.0);
+        y.v[q] = (r < n) ? zr(t.Z[r + (int64_t)ki * t.ldz]) : zr(0.0);
       }
     } else {
-      const double* yr = a.Y + (int64_t)ki * n;
-      const double* yi = yr + (int64_t)n * n;
 #pragma unroll
       for (int q = 0; q < R; ++q) {
         const int r = lane + 64 * q;
-        y.v[q] = (r < n) ? zmk(yr[r], yi[r]) : zr(0.0);
+        y.v[q] = (r < n) ? vo[r] : zr(0.0);
       }
       scale_by_max<R>(y, 0, n, false);
       if (!left && kd == -1) {
@@ -703,12 +574,11 @@ template <int R> __global__ void __launch_bounds__(64) dtrevc_big_finish(DBig a)
       }
     }
   } else {
-    const double* xr = a.X + (int64_t)ki * n;
-    const double* xi = xr + (int64_t)n * n;
+    const zd* xo = t.X + (int64_t)ki * n;
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int i = lane + 64 * q;
-      y.v[q] = (i >= lo && i < hi) ? zmk(xr[i], xi[i]) : zr(0.0);
+      y.v[q] = (i >= lo && i < hi) ? xo[i] : zr(0.0);
     }
     if (kd == 0) {
       scale_by_max<R>(y, lo, hi, false);
@@ -721,85 +591,115 @@ template <int R> __global__ void __launch_bounds__(64) dtrevc_big_finish(DBig a)
     }
   }
   if (a.normalize) enormalize_w<R>(y, n);
-  const int pk = left ? ki + 1 : ki - 1;
+  zd* po = t.V + (int64_t)(left ? ki + 1 : ki - 1) * t.ldv;
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int r = lane + 64 * q;
     if (r < n) {
       const zd z = y.v[q];
-      a.V[r + (int64_t)ki * a.ldv] = z;
-      if (kd != 0) a.V[r + (int64_t)pk * a.ldv] = zconj(z);
+      vo[r] = z;
+      // the conjugate partner of a pair
+      if (kd != 0) po[r] = zconj(z);
     }
   }
 }
 
-size_t dtrevc_big_ws_bytes(int n) {
-  const size_t nn = (size_t)n * n;
-  return 2 * trevc_seg(8 * (size_t)n) + trevc_seg(4 * (size_t)n) + trevc_seg(8 * nn) + 2 * trevc_seg(16 * nn);
-}
-
-template <int R> static hipError_t launch_dbig_r(const DBig& b, hipStream_t s) {
-  const int n = b.n;
-  const size_t lds = 64 * R * sizeof(zd);
-  if (b.left) {
-    auto k = dtrevc_big_solve<R, TransG<double>>;
-    (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(k, dim3(n), dim3(64), lds, s, b, TransG<double>{b.Tt, n});
+template <int R> static hipError_t launch_dtrevc_r(const TrevcArgs& a, int nmax, hipStream_t s) {
+  const size_t lds = wavevec_lds_bytes<R>();
+  const int nt = (nmax + 63) / 64;
+  hipLaunchKernelGGL(dtrevc_norms_kernel, dim3((nmax + 3) / 4, a.count), dim3(256), 0, s, a);
+  if (a.left) {
+    hipLaunchKernelGGL(trevc_transpose_kernel<double>, dim3((nmax + 31) / 32, (nmax + 31) / 32, a.count), dim3(256),
+                       0, s, a);
+    hipLaunchKernelGGL((dtrevc_solve_kernel<R, true>), dim3(nmax, a.count), dim3(64), lds, s, a);
   } else {
-    auto k = dtrevc_big_solve<R, GlobD>;
-    (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(k, dim3(n), dim3(64), lds, s, b, GlobD{b.T, b.ldt});
+    hipLaunchKernelGGL((dtrevc_solve_kernel<R, false>), dim3(nmax, a.count), dim3(64), lds, s, a);
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (b.Z) {
-    e = launch_dgemm(false, false, n, 2 * n, n, 1.0, b.Z, b.ldz, b.X, n, 0.0, b.Y, n, s);
-    if (e != hipSuccess) return e;
-  }
-  (void)hipFuncSetAttribute((const void*)dtrevc_big_finish<R>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(dtrevc_big_finish<R>, dim3(n), dim3(64), lds, s, b);
+  if (a.Z) hipLaunchKernelGGL(trevc_back_kernel<double>, dim3(nt, nt, a.count), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(dtrevc_finish_kernel<R>, dim3(nmax, a.count), dim3(64), lds, s, a);
   return hipGetLastError();
 }
 
-// a.T, a.Z, a.V point at the matrix (no offsets), ld from a.ldt/ldz/ldv;
-// ws holds dtrevc_big_ws_bytes(n)
-hipError_t launch_dtrevc_big(const TrevcArgsD& a, int n, void* ws, hipStream_t s) {
-  if (n <= dtrevc_max_n() || n > trevc_big_max_n() || !ws) return hipErrorInvalidValue;
-  const size_t nn = (size_t)n * n;
-  char* p = static_cast<char*>(ws);
-  DBig b;
-  b.n = n;
-  b.left = a.left;
-  b.normalize = a.normalize;
-  b.T = a.T;
-  b.ldt = a.ldt > 0 ? a.ldt : n;
-  b.Z = a.Z;
-  b.ldz = a.ldz > 0 ? a.ldz : n;
-  b.V = reinterpret_cast<zd*>(a.V);
-  b.ldv = a.ldv > 0 ? a.ldv : n;
-  b.sub = reinterpret_cast<double*>(p);
-  p += trevc_seg(8 * (size_t)n);
-  b.tnorms = reinterpret_cast<double*>(p);
-  p += trevc_seg(8 * (size_t)n);
-  b.kind = reinterpret_cast<int*>(p);
-  p += trevc_seg(4 * (size_t)n);
-  double* tt = reinterpret_cast<double*>(p);
-  b.Tt = tt;
-  p += trevc_seg(8 * nn);
-  b.X = reinterpret_cast<double*>(p);
-  p += trevc_seg(16 * nn);
-  b.Y = reinterpret_cast<double*>(p);
-  hipLaunchKernelGGL(dtrevc_big_kinds, dim3(1), dim3(1024), 4 * (size_t)n, s, b);
-  hipLaunchKernelGGL(trevc_colnorm_kernel<double>, dim3((n + 3) / 4), dim3(256), 0, s, n, b.T, b.ldt, false,
-                     b.tnorms);
-  if (b.left)
-    hipLaunchKernelGGL(trevc_transpose_kernel<double>, dim3((n + 31) / 32, (n + 31) / 32), dim3(256), 0, s, n, b.T,
-                       b.ldt, tt);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return n <= 2048 ? launch_dbig_r<32>(b, s) : launch_dbig_r<64>(b, s);
+hipError_t launch_dtrevc(const TrevcArgs& a, int nmax, hipStream_t s) {
+  switch (trevc_class(nmax)) {
+    case 1: return launch_dtrevc_r<1>(a, nmax, s);
+    case 2: return launch_dtrevc_r<2>(a, nmax, s);
+    case 4: return launch_dtrevc_r<4>(a, nmax, s);
+    case 8: return launch_dtrevc_r<8>(a, nmax, s);
+    case 16: return launch_dtrevc_r<16>(a, nmax, s);
+    case 32: return launch_dtrevc_r<32>(a, nmax, s);
+    case 64: return launch_dtrevc_r<64>(a, nmax, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
-int trevc_big_max_n() { return 4096; }
+int trevc_max_n() { return 4096; }
+
+// Workspace of one launch group, per matrix: X (16 n^2), the transpose
+// (left), and 8 n + 8 n + 4 n for norms, subdiagonal and kinds; each array
+// 256-byte aligned.  A group ends where the next matrix needs another class,
+// would take the workspace above kGroupBytes, or fills the grid's z
+// dimension.
+constexpr size_t kGroupBytes = size_t(1) << 30;
+constexpr int kGroupCount = 32768;
+static size_t seg(size_t bytes) { return (bytes + 255) & ~size_t(255); }
+
+void trevc_groups(const int32_t* n, const int32_t* order, int64_t count, bool cplx, TrevcPlan& p) {
+  const size_t es = cplx ? 16 : 8;
+  p.groups.clear();
+  p.wsn.assign((size_t)count, 0);
+  p.wsnn.assign((size_t)count, 0);
+  p.bytes = 0;
+  for (int64_t q = 0; q < count;) {
+    if (n[order[q]] <= 0) break;  // descending: only empty matrices remain
+    TrevcGroup g;
+    g.first = q;
+    g.nmax = n[order[q]];
+    const int cls = trevc_class(g.nmax);
+    int64_t sn = 0, snn = 0;
+    int64_t k = q;
+    for (; k < count && k - q < kGroupCount; ++k) {
+      const int64_t m = n[order[k]];
+      if (m <= 0 || trevc_class((int)m) != cls) break;
+      if (k > q && (16 + es) * (size_t)(snn + m * m) > kGroupBytes) break;
+      p.wsn[k] = sn;
+      p.wsnn[k] = snn;
+      sn += m;
+      snn += m * m;
+    }
+    g.count = k - q;
+    g.sn = sn;
+    g.snn = snn;
+    p.groups.push_back(g);
+    p.bytes = std::max(p.bytes, seg(16 * (size_t)snn) + seg(es * (size_t)snn) + 2 * seg(8 * (size_t)sn) +
+                                    seg(4 * (size_t)sn));
+    q = k;
+  }
+}
+
+hipError_t launch_trevc(bool cplx, TrevcArgs a, const TrevcPlan& p, void* ws, hipStream_t s) {
+  const int32_t* order = a.order;
+  const int64_t *wsn = a.wsn, *wsnn = a.wsnn;
+  const size_t es = cplx ? 16 : 8;
+  for (const TrevcGroup& g : p.groups) {
+    char* w = static_cast<char*>(ws);
+    a.wX = w;
+    w += seg(16 * (size_t)g.snn);
+    a.wT = w;
+    w += seg(es * (size_t)g.snn);
+    a.wcn = reinterpret_cast<double*>(w);
+    w += seg(8 * (size_t)g.sn);
+    a.wsub = reinterpret_cast<double*>(w);
+    w += seg(8 * (size_t)g.sn);
+    a.wkind = reinterpret_cast<int*>(w);
+    a.order = order + g.first;
+    a.wsn = wsn + g.first;
+    a.wsnn = wsnn + g.first;
+    a.count = (int)g.count;
+    const hipError_t e = cplx ? launch_ztrevc(a, g.nmax, s) : launch_dtrevc(a, g.nmax, s);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
 
 }  // namespace gs

@@ -110,10 +110,10 @@ hipError_t launch_zqrw_single(const BatchArgs& a, int nt, hipStream_t s);
 hipError_t launch_zlog_rows(int n, double* Z, int64_t ld, const double* lg, const int64_t* llen, hipStream_t s);
 hipError_t launch_dschur_global(const SingleArgs& a, int nt, hipStream_t s);
 
-// Eigenvector kernels (one workgroup per matrix).  T, Z at element offset
-// off[m] (complex elements for the complex kernel), V (complex) at complex
-// offset off[m].  ld* > 0 gives leading dimensions for a single matrix;
-// 0 means ld = n.
+// Eigenvector kernels over a list of matrices in descending order (matrix
+// order[q] is entry q).  T, Z at element offset off[m] (complex elements for
+// the complex kernels), V (complex) at complex offset off[m].  ld* > 0 gives
+// leading dimensions for a single matrix; 0 means ld = n.
 struct TrevcArgs {
   const int32_t* order;
   int count;
@@ -125,27 +125,34 @@ struct TrevcArgs {
   int left;
   int normalize;
   int64_t ldt, ldz, ldv;
+  // workspace offsets of entry q (in rows and in entries; device copies of
+  // TrevcPlan's), and the arrays, set by launch_trevc
+  const int64_t* wsn;
+  const int64_t* wsnn;
+  void* wX;
+  void* wT;
+  double* wcn;
+  double* wsub;
+  int* wkind;
 };
-typedef TrevcArgs TrevcArgsD;
-
-size_t ztrevc_lds_bytes(int n);
-size_t dtrevc_lds_bytes(int n);
-// largest order the eigenvector kernels take (T in global memory above the
-// LDS-resident orders 128 complex / 192 real)
-int ztrevc_max_n();
-int dtrevc_max_n();
+// Launch groups of a list: orders of one class, a bounded workspace.
+struct TrevcGroup {
+  int64_t first, count;
+  int nmax;
+  int64_t sn, snn;  // sums of n and n^2
+};
+struct TrevcPlan {
+  std::vector<TrevcGroup> groups;
+  std::vector<int64_t> wsn, wsnn;
+  size_t bytes = 0;  // workspace
+};
+void trevc_groups(const int32_t* n, const int32_t* order, int64_t count, bool cplx, TrevcPlan& p);
+int trevc_max_n();
+// a: order, wsn, wsnn whole device arrays; ws holds p.bytes of device memory
+hipError_t launch_trevc(bool cplx, TrevcArgs a, const TrevcPlan& p, void* ws, hipStream_t s);
+// one group (a.order .. a.wkind the group's own)
 hipError_t launch_ztrevc(const TrevcArgs& a, int nmax, hipStream_t s);
-hipError_t launch_dtrevc(const TrevcArgsD& a, int nmax, hipStream_t s);
-// One matrix of order z/dtrevc_max_n() < n <= trevc_big_max_n() over the
-// whole GPU (solves one per workgroup with the vector in LDS, the
-// back-transform as FP64 MFMA GEMMs).  a.T, a.Z, a.V point at the matrix,
-// a.ld* its leading dimensions (0: n); order/count/n/off are not read.
-// ws: z/dtrevc_big_ws_bytes(n) bytes of device memory.
-int trevc_big_max_n();
-size_t dtrevc_big_ws_bytes(int n);
-size_t ztrevc_big_ws_bytes(int n);
-hipError_t launch_dtrevc_big(const TrevcArgsD& a, int n, void* ws, hipStream_t s);
-hipError_t launch_ztrevc_big(const TrevcArgs& a, int n, void* ws, hipStream_t s);
+hipError_t launch_dtrevc(const TrevcArgs& a, int nmax, hipStream_t s);
 
 // Eigenvalue VJP assembly: VR, VL (complex) at complex offset off[m], gbar
 // (complex) at woff[m], Abar (real) at off[m].

@@ -26,10 +26,7 @@ int run_trevc(gs_handle* h, bool cplx, int64_t count, const int32_t* n, const in
   int nmax = 0;
   for (int64_t i = 0; i < count; ++i) nmax = std::max(nmax, (int)n[i]);
   if (nmax == 0) return GS_OK;
-  // orders above the one-workgroup kernels' limit run one matrix at a time
-  // through the whole-GPU path, up to trevc_big_max_n()
-  const int lim = cplx ? ztrevc_max_n() : dtrevc_max_n();
-  if (nmax > trevc_big_max_n()) return handle_fail(h, GS_E_UNSUPPORTED, "order above the eigenvector kernel limit");
+  if (nmax > trevc_max_n()) return handle_fail(h, GS_E_UNSUPPORTED, "order above the eigenvector kernel limit");
   std::lock_guard<std::mutex> lk(handle_mutex(h));
   hipError_t e = hipSetDevice(handle_device(h));
   if (e != hipSuccess) return handle_fail_hip(h, e, "hipSetDevice");
@@ -49,17 +46,22 @@ int run_trevc(gs_handle* h, bool cplx, int64_t count, const int32_t* n, const in
   for (int64_t i = 0; i < count; ++i) order[i] = (int32_t)i;
   std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return n[x] > n[y]; });
   DevBuf& meta = handle_buf(h, 0);
-  const size_t mbytes = sizeof(int32_t) * 2 * count + sizeof(int64_t) * count + 64;
+  TrevcPlan plan;
+  trevc_groups(n, order.data(), count, cplx, plan);
+  const size_t mbytes = sizeof(int32_t) * 2 * count + sizeof(int64_t) * 3 * count;
   if ((e = meta.ensure(mbytes)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
   char* mp = static_cast<char*>(meta.p);
   int64_t* d_off = reinterpret_cast<int64_t*>(mp);
-  int32_t* d_n = reinterpret_cast<int32_t*>(mp + sizeof(int64_t) * count);
+  int32_t* d_n = reinterpret_cast<int32_t*>(d_off + 3 * count);
   int32_t* d_order = d_n + count;
   std::vector<char> hm(mbytes);
-  std::memcpy(hm.data(), off, sizeof(int64_t) * count);
-  std::memcpy(hm.data() + sizeof(int64_t) * count, n, sizeof(int32_t) * count);
-  std::memcpy(hm.data() + sizeof(int64_t) * count + sizeof(int32_t) * count, order.data(), sizeof(int32_t) * count);
-  if ((e = hipMemcpyAsync(meta.p, hm.data(), mbytes - 64, hipMemcpyHostToDevice, s)) != hipSuccess)
+  const size_t c8 = sizeof(int64_t) * count, c4 = sizeof(int32_t) * count;
+  std::memcpy(hm.data(), off, c8);
+  std::memcpy(hm.data() + c8, plan.wsn.data(), c8);
+  std::memcpy(hm.data() + 2 * c8, plan.wsnn.data(), c8);
+  std::memcpy(hm.data() + 3 * c8, n, c4);
+  std::memcpy(hm.data() + 3 * c8 + c4, order.data(), c4);
+  if ((e = hipMemcpyAsync(meta.p, hm.data(), mbytes, hipMemcpyHostToDevice, s)) != hipSuccess)
     return handle_fail_hip(h, e, "hipMemcpyAsync");
   const double *dT = T, *dZ = Z;
   double* dV = V;
@@ -101,33 +103,11 @@ int run_trevc(gs_handle* h, bool cplx, int64_t count, const int32_t* n, const in
   a.ldt = single ? ldt : 0;
   a.ldz = single ? ldz : 0;
   a.ldv = single ? ldv : 0;
-  // the order array lists the matrices largest first: those above lim lead
-  int64_t nbig = 0;
-  while (nbig < count && n[order[nbig]] > lim) ++nbig;
-  if (nbig > 0) {
-    DevBuf& ws = handle_buf(h, 4);
-    const size_t wsb = cplx ? ztrevc_big_ws_bytes(nmax) : dtrevc_big_ws_bytes(nmax);
-    if ((e = ws.ensure(wsb)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
-    const int64_t ew = cplx ? 2 : 1;  // doubles per element of T and Z
-    for (int64_t b = 0; b < nbig; ++b) {
-      const int32_t m = order[b];
-      TrevcArgs one = a;
-      one.T = dT + ew * off[m];
-      one.Z = dZ ? dZ + ew * off[m] : nullptr;
-      one.V = dV + 2 * off[m];
-      one.ldt = single ? ldt : n[m];
-      one.ldz = single ? ldz : n[m];
-      one.ldv = single ? ldv : n[m];
-      e = cplx ? launch_ztrevc_big(one, n[m], ws.p, s) : launch_dtrevc_big(one, n[m], ws.p, s);
-      if (e != hipSuccess) return handle_fail_hip(h, e, "kernel launch");
-    }
-  }
-  if (nbig < count && n[order[nbig]] > 0) {
-    a.order = d_order + nbig;
-    a.count = (int)(count - nbig);
-    e = cplx ? launch_ztrevc(a, n[order[nbig]], s) : launch_dtrevc(a, n[order[nbig]], s);
-    if (e != hipSuccess) return handle_fail_hip(h, e, "kernel launch");
-  }
+  a.wsn = d_off + count;
+  a.wsnn = d_off + 2 * count;
+  DevBuf& ws = handle_buf(h, 4);
+  if ((e = ws.ensure(plan.bytes)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
+  if ((e = launch_trevc(cplx, a, plan, ws.p, s)) != hipSuccess) return handle_fail_hip(h, e, "kernel launch");
   if (!dev) {
     if (single) {
       e = copy_cols(V, 16 * ldv, dV, 16 * ldv, 16 * n[0], n[0], hipMemcpyDeviceToHost, s);

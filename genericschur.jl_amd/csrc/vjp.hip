@@ -109,8 +109,8 @@ __global__ void __launch_bounds__(256) vjp_scale_kernel(VjpArgs a, zd* VL) {
 // bytes per 2 flops and tile side).  One launch covers every matrix of the
 // class instead of a GEMM per matrix, whose single 128 x 128 tile left 255
 // CUs idle: 4096 real matrices n ~ U{16..128}, the 2119 of order above 70
-// took 105 ms
-// more in 6357 launches (forward and backward 146.9 -> 42.3 ms).
+// took
+// 105 ms more in 6357 launches (forward and backward 146.9 -> 42.3 ms).
 constexpr int VT = 64, VKB = 8, VLD = VT + 16;
 __global__ void __launch_bounds__(256) vjp_gemm_kernel(VjpArgs a) {
   __shared__ double As[2][2 * VKB * VLD], Bs[2][2 * VKB * VLD];

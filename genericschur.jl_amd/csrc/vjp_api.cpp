@@ -29,7 +29,7 @@ extern "C" int gs_eig_vjp_batched_d(gs_handle* h, int64_t count, const int32_t* 
     woff[i] = wtot;
     wtot += n[i];
   }
-  if (nmax > trevc_big_max_n()) return handle_fail(h, GS_E_UNSUPPORTED, "order above the VJP kernel limit");
+  if (nmax > trevc_max_n()) return handle_fail(h, GS_E_UNSUPPORTED, "order above the VJP kernel limit");
   std::lock_guard<std::mutex> lk(handle_mutex(h));
   hipError_t e = hipSetDevice(handle_device(h));
   if (e != hipSuccess) return handle_fail_hip(h, e, "hipSetDevice");
@@ -39,19 +39,23 @@ extern "C" int gs_eig_vjp_batched_d(gs_handle* h, int64_t count, const int32_t* 
   for (int64_t i = 0; i < count; ++i) order[i] = (int32_t)i;
   std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return n[x] > n[y]; });
   DevBuf& meta = handle_buf(h, 4);
-  const size_t mbytes = sizeof(int64_t) * 2 * count + sizeof(int32_t) * 2 * count;
+  TrevcPlan plan;
+  trevc_groups(n, order.data(), count, false, plan);
+  const size_t mbytes = sizeof(int64_t) * 4 * count + sizeof(int32_t) * 2 * count;
   if ((e = meta.ensure(mbytes + 64)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
   char* mp = static_cast<char*>(meta.p);
   int64_t* d_off = reinterpret_cast<int64_t*>(mp);
   int64_t* d_woff = d_off + count;
-  int32_t* d_n = reinterpret_cast<int32_t*>(d_woff + count);
+  int32_t* d_n = reinterpret_cast<int32_t*>(d_off + 4 * count);
   int32_t* d_order = d_n + count;
   std::vector<char> hm(mbytes);
-  std::memcpy(hm.data(), off, sizeof(int64_t) * count);
-  std::memcpy(hm.data() + sizeof(int64_t) * count, woff.data(), sizeof(int64_t) * count);
-  std::memcpy(hm.data() + sizeof(int64_t) * 2 * count, n, sizeof(int32_t) * count);
-  std::memcpy(hm.data() + sizeof(int64_t) * 2 * count + sizeof(int32_t) * count, order.data(),
-              sizeof(int32_t) * count);
+  const size_t c8 = sizeof(int64_t) * count, c4 = sizeof(int32_t) * count;
+  std::memcpy(hm.data(), off, c8);
+  std::memcpy(hm.data() + c8, woff.data(), c8);
+  std::memcpy(hm.data() + 2 * c8, plan.wsn.data(), c8);
+  std::memcpy(hm.data() + 3 * c8, plan.wsnn.data(), c8);
+  std::memcpy(hm.data() + 4 * c8, n, c4);
+  std::memcpy(hm.data() + 4 * c8 + c4, order.data(), c4);
   if ((e = hipMemcpyAsync(meta.p, hm.data(), mbytes, hipMemcpyHostToDevice, s)) != hipSuccess)
     return handle_fail_hip(h, e, "hipMemcpyAsync");
   DevBuf& bVR = handle_buf(h, 5);
@@ -91,38 +95,16 @@ extern "C" int gs_eig_vjp_batched_d(gs_handle* h, int64_t count, const int32_t* 
   t.Z = dZ;
   t.normalize = 1;
   t.ldt = t.ldz = t.ldv = 0;
-  // right and left eigenvectors: matrices above the one-workgroup kernels'
-  // orders (first in the descending order) one at a time on the whole-GPU
-  // path, the rest in one launch per side
-  int64_t nbigv = 0;
-  while (nbigv < count && n[order[nbigv]] > dtrevc_max_n()) ++nbigv;
-  if (nbigv > 0) {
-    DevBuf& ws = handle_buf(h, 13);
-    if ((e = ws.ensure(dtrevc_big_ws_bytes(nmax))) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
-    for (int64_t b = 0; b < nbigv; ++b) {
-      const int32_t m = order[b];
-      TrevcArgs one = t;
-      one.T = dT + off[m];
-      one.Z = dZ + off[m];
-      one.ldt = one.ldz = one.ldv = n[m];
-      for (int left = 0; left < 2; ++left) {
-        one.left = left;
-        one.V = static_cast<double*>(left ? bVL.p : bVR.p) + 2 * off[m];
-        if ((e = launch_dtrevc_big(one, n[m], ws.p, s)) != hipSuccess)
-          return handle_fail_hip(h, e, "eigenvector launch");
-      }
-    }
-  }
-  if (nbigv < count) {
-    t.order = d_order + nbigv;
-    t.count = (int)(count - nbigv);
-    const int nsmall = n[order[nbigv]];
-    t.V = static_cast<double*>(bVR.p);
-    t.left = 0;
-    if ((e = launch_dtrevc(t, nsmall, s)) != hipSuccess) return handle_fail_hip(h, e, "eigenvector launch");
-    t.V = static_cast<double*>(bVL.p);
-    t.left = 1;
-    if ((e = launch_dtrevc(t, nsmall, s)) != hipSuccess) return handle_fail_hip(h, e, "eigenvector launch");
+  t.wsn = d_off + 2 * count;
+  t.wsnn = d_off + 3 * count;
+  // right and left eigenvectors, the second side reusing the workspace
+  DevBuf& ws = handle_buf(h, 13);
+  if ((e = ws.ensure(plan.bytes)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
+  for (int left = 0; left < 2; ++left) {
+    t.left = left;
+    t.V = static_cast<double*>(left ? bVL.p : bVR.p);
+    if ((e = launch_trevc(false, t, plan, ws.p, s)) != hipSuccess)
+      return handle_fail_hip(h, e, "eigenvector launch");
   }
   // orders whose two factors fit LDS: one workgroup per matrix; larger
   // ones (first in the descending order) two launches for each run of

@@ -1,8 +1,10 @@
 // A vector of up to 64*R entries distributed over one wavefront: lane l
 // holds entries l, l+64, ... (0-based) in registers.  Entry access by a
-// uniform index broadcasts through a cross-lane shuffle, so back- and
+// uniform index broadcasts by v_readlane, so back- and
 // forward-substitutions keep the solution vector out of LDS.
 #pragma once
+#include <type_traits>
+
 #include "dev_common.h"
 
 template <int R> struct WaveVecZ {
@@ -15,10 +17,8 @@ template <int R> struct WaveVecZ {
 #pragma unroll
     for (int k = 1; k < R; ++k)
       if (q == k) s = v[k];
-    zd r;
-    r.x = __shfl(s.x, l, 64);
-    r.y = __shfl(s.y, l, 64);
-    return r;
+    const int lu = __builtin_amdgcn_readfirstlane(l);
+    return zmk(rdlane(s.x, lu), rdlane(s.y, lu));
   }
   // set entry i (0-based, uniform) to a uniform value
   GS_DEV void set(int i, zd val) {
@@ -54,6 +54,13 @@ template <int R> struct WaveVecL {
     for (int k = 0; k < R; ++k) v[k] = v[k] * s;
   }
 };
+
+// Registers up to R = 4 (256 entries), LDS above: a register vector's entry
+// access selects among its R slots.
+template <int R> using WaveVec = typename std::conditional<(R <= 4), WaveVecZ<R>, WaveVecL<R>>::type;
+template <int R> constexpr size_t wavevec_lds_bytes() { return R <= 4 ? 0 : 64 * R * sizeof(zd); }
+GS_DEV void wavevec_bind(LdsLaneRef& v, void* lds) { v.p = static_cast<zd*>(lds); }
+template <int R> GS_DEV void wavevec_bind(zd (&)[R], void*) {}
 
 // wave-wide maximum over lanes (all lanes receive it)
 GS_DEV double wmax(double x) { return wave_max(x); }

@@ -4,38 +4,15 @@
 //   left    vectors.jl:372-460  with _cusolve! util.jl:301-461
 //   unit 2-norm, largest entry real: _enormalize! util.jl:572-592
 //
-// One workgroup per matrix, NT/64 wavefronts.  T is held in LDS in compact
-// upper-triangular storage.  Each wavefront solves whole eigenvectors: the
-// right-hand side / solution lives in registers across its 64 lanes
-// (WaveVecZ), the substitution walks T's columns (right) or rows (left) in
-// LDS, and the scalar control of the scaled solver runs uniformly in every
-// lane.  The solutions are parked in the output V, then each column is
-// back-transformed by Z (V[:, k] = Z x) and normalised.
-#include <type_traits>
-
+// The launches over a list of matrices are described in trevc_grid.h; here
+// one wavefront per eigenvector, the scalar control of the scaled solver
+// running uniformly in every lane.
 #include "dev_common.h"
 #include "internal.h"
-#include "trevc_big.h"
+#include "trevc_grid.h"
 #include "wavevec.h"
 
 namespace gs {
-
-
-// compact upper triangle: column j (0-based) holds rows 0..j at j(j+1)/2
-GS_DEV int tri(int i, int j) { return (j * (j + 1)) / 2 + i; }
-
-// Entry (i, j), i <= j, of T: from the compact copy in LDS (orders whose
-// triangle fits a CU's LDS) or from T itself in global memory (larger
-// orders; the reads stay in L2 across the substitutions).
-struct TriLdsZ {
-  const zd* p;
-  GS_DEV zd operator()(int i, int j) const { return p[tri(i, j)]; }
-};
-struct GlobZ {
-  const zd* p;
-  int64_t ld;
-  GS_DEV zd operator()(int i, int j) const { return p[i + (int64_t)j * ld]; }
-};
 
 // ------------------------------------------------------------------------
 // Shifted, clamped diagonal of the solve: T(j,j) - lam, replaced by smin
@@ -46,9 +23,65 @@ template <class TA> GS_DEV zd shifted_diag(const TA& Tc, int j, zd lam, double s
   return d;
 }
 
+// The substitutions without scaling divide by the shifted diagonal with
+// Smith's algorithm, whose ratio and denominator depend on the diagonal only:
+// ZFac holds them for the 64 rows of a chunk, one row per lane (LDS), and a
+// step reads its row's as a broadcast.
+struct ZFac {
+  double r, d, sw, pad;
+};
+GS_DEV ZFac zfac(zd b) {
+  const bool sw = fabs(b.y) > fabs(b.x);
+  const double r = sw ? b.x / b.y : b.y / b.x;
+  return ZFac{r, sw ? b.x * r + b.y : b.x + b.y * r, sw ? 1.0 : 0.0, 0.0};
+}
+GS_DEV zd zfac_div(zd a, ZFac f) {
+  const bool sw = __builtin_amdgcn_readfirstlane((int)f.sw) != 0;
+  const double p = sw ? a.y : a.x, q = sw ? a.x : a.y;
+  const double x = (p + q * f.r) / f.d, y = (q - p * f.r) / f.d;
+  return zmk(x, sw ? -y : y);
+}
+
+// Whether the growth estimate of zlatrs is certain to allow the substitution
+// without scaling: with every |t_jj| >= smallnum the estimate is at least
+// grow0 times the product of min(1, t_jj) / 1 at its smallest and of
+// t_jj / (t_jj + cnorm_j) (left: min(1, t_jj / (1 + cnorm_j)) and 1 / (1 +
+// cnorm_j)), here bounded from below by powers of two summed over the lanes.
+// The estimate itself is a chain of n divisions; it runs where this bound
+// does not decide.
+template <bool LEFT, class TA> GS_DEV bool grow_certain(const TA& Tc, const double* cnorm, int o, int m, zd lam,
+                                                        double smin, double grow0) {
+  const int lane = threadIdx.x & 63;
+  const double smallnum = GS_FMIN / GS_EPS;
+  int e = 0, emin = 0;
+  bool ok = true;
+  for (int j = lane; j < m; j += 64) {
+    zd d = Tc(o + j, o + j) - lam;
+    if (zabs1(d) < smin) d = zr(smin);
+    const double t = zabs1(d);
+    ok = ok && t >= smallnum && t < 0x1p1000 && cnorm[j] < 0x1p1000;
+    const int et = ilogb(t);
+    if (LEFT) {
+      const int ec = ilogb(1.0 + cnorm[j]) + 1;  // 1 + cnorm < 2^ec
+      e += min(0, et - ec);
+      emin = min(emin, -ec);
+    } else {
+      e += et - (ilogb(t + cnorm[j]) + 1);  // t / (t + c) > 2^(et - ec)
+      emin = min(emin, et);
+    }
+  }
+  // 64 lanes: sums of exponents by lane exchange
+  for (int s = 32; s > 0; s >>= 1) {
+    e += __shfl_xor(e, s, 64);
+    emin = min(emin, __shfl_xor(emin, s, 64));
+  }
+  if (__builtin_amdgcn_ballot_w64(!ok) != 0) return false;
+  return grow0 >= 0x1p-1000 && ilogb(grow0) + e + emin > ilogb(smallnum) + 2;
+}
+
 // _usolve! on entries 0..m-1 of x (A = T shifted by lam, leading m x m).
 template <int R, class TA, class VEC> GS_DEV double usolve_w(const TA& Tc, const double* cnorm, int m, zd lam,
-                                                             double smin, VEC& x) {
+                                                             double smin, VEC& x, ZFac* fac) {
   const int lane = threadIdx.x & 63;
   const double half = 0.5;
   const double smallnum = GS_FMIN / GS_EPS;
@@ -75,6 +108,7 @@ template <int R, class TA, class VEC> GS_DEV double usolve_w(const TA& Tc, const
     grow = half / fmax(xbound, smallnum);
     xbound = grow;
     bool toosmall = false;
+    if (!grow_certain<false>(Tc, cnorm, 0, m, lam, smin, grow))
     for (int j = m - 1; j >= 0; --j) {
       toosmall = (grow <= smallnum);
       if (toosmall) break;
@@ -88,13 +122,40 @@ template <int R, class TA, class VEC> GS_DEV double usolve_w(const TA& Tc, const
     if (!toosmall) grow = xbound;
   }
   if (grow * tscale > smallnum) {
+    // columns of T one step ahead up to R = 4 entries per lane
+    constexpr bool PF = R <= 4;
+    zd c[PF ? R : 1];
+    auto load = [&](int j) {
+      if constexpr (PF) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) c[q] = Tc(min(lane + 64 * q, m - 1), max(j, 0));
+      }
+    };
+    load(m - 1);
+    int chunk = -1;
     for (int j = m - 1; j >= 0; --j) {
-      const zd xj = x.get(j) / shifted_diag(Tc, j, lam, smin);
+      if ((j >> 6) != chunk) {
+        chunk = j >> 6;
+        wsync();
+        fac[lane] = zfac(shifted_diag(Tc, min(64 * chunk + lane, m - 1), lam, smin));
+        wsync();
+      }
+      zd k[PF ? R : 1];
+      if constexpr (PF) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) k[q] = c[q];
+      }
+      load(j - 1);
+      const zd xj = zfac_div(x.get(j), fac[j & 63]);
       x.set(j, xj);
 #pragma unroll
       for (int q = 0; q < R; ++q) {
         const int i = lane + 64 * q;
-        if (i < j) x.v[q] = x.v[q] - Tc(i, j) * xj;
+        if constexpr (PF) {
+          if (i < j) x.v[q] = x.v[q] - k[q] * xj;
+        } else {
+          if (i < j) x.v[q] = x.v[q] - Tc(i, j) * xj;
+        }
       }
     }
     return xscale;
@@ -177,7 +238,7 @@ template <int R, class TA, class VEC> GS_DEV double usolve_w(const TA& Tc, const
 // A(i, j) = T(o+i, o+j) for i < j and the shifted, clamped diagonal; cnorm
 // is indexed from 0 (the reference passes the full tnorms, vectors.jl:417-420).
 template <int R, class TA, class VEC> GS_DEV double cusolve_w(const TA& Tc, const double* cnorm, int o, int m, zd lam,
-                                                              double smin, VEC& x) {
+                                                              double smin, VEC& x, ZFac* fac) {
   const int lane = threadIdx.x & 63;
   const double half = 0.5;
   const double smallnum = GS_FMIN / GS_EPS;
@@ -207,6 +268,7 @@ template <int R, class TA, class VEC> GS_DEV double cusolve_w(const TA& Tc, cons
     grow = half / fmax(xbound, smallnum);
     xbound = grow;
     bool toosmall = false;
+    if (!grow_certain<true>(Tc, cnorm, o, m, lam, smin, grow))
     for (int j = 0; j < m; ++j) {
       toosmall = (grow <= smallnum);
       if (toosmall) break;
@@ -224,13 +286,39 @@ template <int R, class TA, class VEC> GS_DEV double cusolve_w(const TA& Tc, cons
   if (grow * tscale > smallnum) {
     // forward substitution in axpy form: after x[j] is final, remove its
     // contribution from the later right-hand sides
+    constexpr bool PF = R <= 4;
+    zd c[PF ? R : 1];
+    auto load = [&](int j) {
+      if constexpr (PF) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) c[q] = Tc(o + min(j, m - 1), min(lane + 64 * q, o + m - 1));
+      }
+    };
+    load(0);
+    int chunk = -1;
     for (int j = 0; j < m; ++j) {
-      const zd xj = x.get(o + j) / zconj(shifted_diag(Tc, o + j, lam, smin));
+      if (((o + j) >> 6) != chunk) {
+        chunk = (o + j) >> 6;
+        wsync();
+        fac[lane] = zfac(zconj(shifted_diag(Tc, min(max(64 * chunk + lane, o), o + m - 1), lam, smin)));
+        wsync();
+      }
+      zd k[PF ? R : 1];
+      if constexpr (PF) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) k[q] = c[q];
+      }
+      load(j + 1);
+      const zd xj = zfac_div(x.get(o + j), fac[(o + j) & 63]);
       x.set(o + j, xj);
 #pragma unroll
       for (int q = 0; q < R; ++q) {
         const int i = lane + 64 * q;  // absolute entry index
-        if (i > o + j && i < o + m) x.v[q] = x.v[q] - zconj(Tc(o + j, i)) * xj;
+        if constexpr (PF) {
+          if (i > o + j && i < o + m) x.v[q] = x.v[q] - zconj(k[q]) * xj;
+        } else {
+          if (i > o + j && i < o + m) x.v[q] = x.v[q] - zconj(Tc(o + j, i)) * xj;
+        }
       }
     }
     return xscale;
@@ -368,294 +456,105 @@ template <int R, class VEC> GS_DEV void normalize_col(VEC& v, int n, bool enorm)
   v.set(bi, zr(r0.x));
 }
 
-template <int NT, int R, bool GLOB> __global__ void __launch_bounds__(NT) ztrevc_kernel(TrevcArgs a) {
+// strictly-upper column norms: abs for right (vectors.jl:70-75), abs1 for
+// left (vectors.jl:395-400); one wavefront per column
+__global__ void __launch_bounds__(256) ztrevc_norms_kernel(TrevcArgs a) {
+  const TrevcMat<zd> t = trevc_mat<zd>(a, blockIdx.y);
+  const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (j >= t.n) return;
+  double s = 0.0;
+  for (int i = lane; i < j; i += 64) s += tmag(t.T[i + (int64_t)j * t.ldt], a.left != 0);
+  s = wave_sum(s);
+  if (lane == 0) t.cn[j] = s;
+}
+
+// workgroup (t, matrix) solves column n-1-t (right) or t (left), the longest
+// first; the scale goes to the diagonal slot
+template <int R, bool LEFT> __global__ void __launch_bounds__(64) ztrevc_solve_kernel(TrevcArgs a) {
   extern __shared__ double smem[];
-  const int b = blockIdx.x;
-  if (b >= a.count) return;
-  const int m = a.order ? a.order[b] : b;
-  const int n = a.n[m];
-  if (n <= 0) return;
-  const int64_t o = a.off[m];
-  const int64_t ldt = a.ldt > 0 ? a.ldt : n;
-  const int64_t ldz = a.ldz > 0 ? a.ldz : n;
-  const int64_t ldv = a.ldv > 0 ? a.ldv : n;
-  const zd* Tg = reinterpret_cast<const zd*>(a.T) + o;
-  const zd* Zg = a.Z ? reinterpret_cast<const zd*>(a.Z) + o : nullptr;
-  zd* Vg = reinterpret_cast<zd*>(a.V) + o;
-  zd* Tl = reinterpret_cast<zd*>(smem);
-  double* tnorms = GLOB ? smem : reinterpret_cast<double*>(Tl + (n * (n + 1)) / 2);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  constexpr int NW = NT / 64;
-  const bool left = a.left != 0;
-  if (!GLOB) {
-    for (int j = 0; j < n; ++j)
-      for (int i = tid; i <= j; i += NT) Tl[tri(i, j)] = Tg[i + j * ldt];
-    __syncthreads();
-  }
-  typedef typename std::conditional<GLOB, GlobZ, TriLdsZ>::type TA;
-  TA Tc;
-  if constexpr (GLOB) Tc = GlobZ{Tg, ldt};
-  else Tc = TriLdsZ{Tl};
-  // strictly-upper column norms: abs for right (vectors.jl:70-75), abs1 for
-  // left (vectors.jl:395-400)
-  for (int j = tid; j < n; j += NT) {
-    double s = 0.0;
-    for (int i = 0; i < j; ++i) s += left ? zabs1(Tc(i, j)) : zabs(Tc(i, j));
-    tnorms[j] = s;
-  }
-  __syncthreads();
-  const double ulp = GS_EPS;
-  const double smallnum = GS_FMIN * (double)n;  // safemin * n (vectors.jl:61,386)
-  // solves, one eigenvector per wavefront at a time; the solution (with the
-  // scale at the diagonal slot) is parked in V's column
-  for (int kk = (left ? w : n - 1 - w); left ? (kk < n) : (kk >= 0); kk += (left ? NW : -NW)) {
-    const zd lam = Tc(kk, kk);
-    const double smin = fmax(ulp * zabs1(lam), smallnum);
-    WaveVecZ<R> x;
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int i = lane + 64 * q;
-      zd v = zr(0.0);
-      if (!left) {
-        if (i < kk) v = -Tc(i, kk);
-      } else {
-        if (i > kk && i < n) v = -zconj(Tc(kk, i));
-      }
-      x.v[q] = v;
-    }
-    double vscale;
-    if (!left) {
-      vscale = (kk > 0) ? usolve_w<R>(Tc, tnorms, kk, lam, smin, x) : 1.0;
-    } else {
-      vscale = (kk < n - 1) ? cusolve_w<R>(Tc, tnorms, kk + 1, n - 1 - kk, lam, smin, x) : 1.0;
-    }
-    x.set(kk, zr(vscale));
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int i = lane + 64 * q;
-      if (i < n) Vg[i + kk * ldv] = (left ? (i >= kk) : (i <= kk)) ? x.v[q] : zr(0.0);
-    }
-  }
-  __syncthreads();
-  // back-transform by Z and normalise, one column per wavefront
-  for (int kk = w; kk < n; kk += NW) {
-    WaveVecZ<R> x;
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int i = lane + 64 * q;
-      x.v[q] = (i < n) ? Vg[i + kk * ldv] : zr(0.0);
-    }
-    WaveVecZ<R> y;
-    if (Zg) {
-      const zd vs = x.get(kk);
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = lane + 64 * q;
-        y.v[q] = (r < n) ? vs * Zg[r + kk * ldz] : zr(0.0);
-      }
-      const int i0 = left ? kk + 1 : 0, i1 = left ? n : kk;
-      for (int i = i0; i < i1; ++i) {
-        const zd xi = x.get(i);
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-          const int r = lane + 64 * q;
-          if (r < n) y.v[q] = y.v[q] + Zg[r + (int64_t)i * ldz] * xi;
-        }
-      }
-    } else {
-      y = x;
-    }
-    normalize_col<R>(y, n, a.normalize != 0);
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int r = lane + 64 * q;
-      if (r < n) Vg[r + kk * ldv] = y.v[q];
-    }
-  }
-}
-
-size_t ztrevc_lds_bytes(int n) { return 16 * ((size_t)n * (n + 1) / 2) + 8 * (size_t)n + 64; }
-
-template <int NT, int R, bool GLOB> static void launch_ztrevc_t(const TrevcArgs& a, size_t lds, hipStream_t s) {
-  (void)hipFuncSetAttribute((const void*)ztrevc_kernel<NT, R, GLOB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds);
-  hipLaunchKernelGGL((ztrevc_kernel<NT, R, GLOB>), dim3(a.count), dim3(NT), lds, s, a);
-}
-
-// Orders up to 128 keep T's triangle in LDS; above, T is read from global
-// memory (only the column norms in LDS), up to ztrevc_max_n().
-hipError_t launch_ztrevc(const TrevcArgs& a, int nmax, hipStream_t s) {
-  if (a.count <= 0) return hipSuccess;
-  if (nmax <= 64) launch_ztrevc_t<256, 1, false>(a, ztrevc_lds_bytes(nmax), s);
-  else if (nmax <= 128) launch_ztrevc_t<256, 2, false>(a, ztrevc_lds_bytes(nmax), s);
-  else if (nmax <= 256) launch_ztrevc_t<512, 4, true>(a, 8 * (size_t)nmax + 64, s);
-  else if (nmax <= 512) launch_ztrevc_t<256, 8, true>(a, 8 * (size_t)nmax + 64, s);
-  else if (nmax <= 1024) launch_ztrevc_t<256, 16, true>(a, 8 * (size_t)nmax + 64, s);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-int ztrevc_max_n() { return 1024; }
-
-// ------------------------------------------------------- larger orders
-// One matrix of order 1024 < n <= trevc_big_max_n() over the whole GPU:
-// column norms in global memory, one solve per workgroup (a single
-// wavefront, solution vector in LDS), solutions in planar X = [Re | Im]
-// (n x 2n), the back-transform Z X as three FP64 MFMA GEMMs on Z's planar
-// copy, then one wavefront per column normalises and writes V.  The
-// per-column steps are those of ztrevc_kernel.
-struct ZBig {
-  int n, left, normalize;
-  const zd* T;
-  int64_t ldt;
-  const zd* Tt;  // T's transpose (left solves), ld n
-  const zd* Z;   // may be null
-  int64_t ldz;
-  zd* V;
-  int64_t ldv;
-  double* tnorms;
-  double* Zp;  // [Re Z | Im Z], n x 2n, ld n
-  double* X;   // n x 2n, ld n
-  double* Y;   // n x 2n, ld n
-};
-
-// workgroup t solves column n-1-t (right) or t (left), longest first
-template <int R, class TA> __global__ void __launch_bounds__(64) ztrevc_big_solve(ZBig a, TA Tc) {
-  extern __shared__ double smem[];
-  const int n = a.n, lane = threadIdx.x & 63, t = blockIdx.x;
-  const bool left = a.left != 0;
-  const int kk = left ? t : n - 1 - t;
+  const TrevcMat<zd> t = trevc_mat<zd>(a, blockIdx.y);
+  const int n = t.n, lane = threadIdx.x & 63, b = blockIdx.x;
+  if (b >= n) return;
+  const int kk = LEFT ? b : n - 1 - b;
+  typedef typename std::conditional<LEFT, TransG<zd>, ColG<zd>>::type TA;
+  const TA Tc = LEFT ? TA{t.Tt, n} : TA{t.T, t.ldt};
   const zd lam = Tc(kk, kk);
   const double smin = fmax(GS_EPS * zabs1(lam), GS_FMIN * (double)n);  // vectors.jl:61,386
-  WaveVecL<R> x{{reinterpret_cast<zd*>(smem)}};
+  WaveVec<R> x;
+  wavevec_bind(x.v, smem);
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int i = lane + 64 * q;
     zd v = zr(0.0);
-    if (!left) {
+    if (!LEFT) {
       if (i < kk) v = -Tc(i, kk);
     } else {
       if (i > kk && i < n) v = -zconj(Tc(kk, i));
     }
     x.v[q] = v;
   }
+  __shared__ ZFac fac[64];
   double vscale;
-  if (!left) vscale = (kk > 0) ? usolve_w<R>(Tc, a.tnorms, kk, lam, smin, x) : 1.0;
-  else vscale = (kk < n - 1) ? cusolve_w<R>(Tc, a.tnorms, kk + 1, n - 1 - kk, lam, smin, x) : 1.0;
+  if (!LEFT) vscale = (kk > 0) ? usolve_w<R>(Tc, t.cn, kk, lam, smin, x, fac) : 1.0;
+  else vscale = (kk < n - 1) ? cusolve_w<R>(Tc, t.cn, kk + 1, n - 1 - kk, lam, smin, x, fac) : 1.0;
   x.set(kk, zr(vscale));
-  double* xr = a.X + (int64_t)kk * n;
-  double* xi = xr + (int64_t)n * n;
+  zd* xo = t.X + (int64_t)kk * n;
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int i = lane + 64 * q;
-    if (i < n) {
-      const zd z = (left ? (i >= kk) : (i <= kk)) ? x.v[q] : zr(0.0);
-      xr[i] = z.x;
-      xi[i] = z.y;
-    }
+    if (i < n) xo[i] = (LEFT ? (i >= kk) : (i <= kk)) ? x.v[q] : zr(0.0);
   }
 }
 
-// Zp = [Re Z | Im Z]
-__global__ void __launch_bounds__(256) ztrevc_big_planar(int n, const zd* Z, int64_t ldz, double* Zp) {
-  const int64_t nn = (int64_t)n * n;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < nn; e += (int64_t)gridDim.x * 256) {
-    const int64_t c = e / n, r = e - c * n;
-    const zd z = Z[r + c * ldz];
-    Zp[e] = z.x;
-    Zp[e + nn] = z.y;
-  }
-}
-
-template <int R> __global__ void __launch_bounds__(64) ztrevc_big_finish(ZBig a) {
+template <int R> __global__ void __launch_bounds__(64) ztrevc_finish_kernel(TrevcArgs a) {
   extern __shared__ double smem[];
-  const int n = a.n, lane = threadIdx.x & 63, kk = blockIdx.x;
-  WaveVecL<R> y{{reinterpret_cast<zd*>(smem)}};
-  const double* src = a.Z ? a.Y : a.X;
-  const double* yr = src + (int64_t)kk * n;
-  const double* yi = yr + (int64_t)n * n;
+  const TrevcMat<zd> t = trevc_mat<zd>(a, blockIdx.y);
+  const int n = t.n, lane = threadIdx.x & 63, kk = blockIdx.x;
+  if (kk >= n) return;
+  WaveVec<R> y;
+  wavevec_bind(y.v, smem);
+  zd* vo = t.V + (int64_t)kk * t.ldv;
+  const zd* src = t.Z ? vo : t.X + (int64_t)kk * n;
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int r = lane + 64 * q;
-    y.v[q] = (r < n) ? zmk(yr[r], yi[r]) : zr(0.0);
+    y.v[q] = (r < n) ? src[r] : zr(0.0);
   }
   normalize_col<R>(y, n, a.normalize != 0);
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int r = lane + 64 * q;
-    if (r < n) a.V[r + (int64_t)kk * a.ldv] = y.v[q];
+    if (r < n) vo[r] = y.v[q];
   }
 }
 
-size_t ztrevc_big_ws_bytes(int n) {
-  const size_t nn = (size_t)n * n;
-  return trevc_seg(8 * (size_t)n) + 4 * trevc_seg(16 * nn);
-}
-
-template <int R> static hipError_t launch_zbig_r(const ZBig& b, hipStream_t s) {
-  const int n = b.n;
-  const size_t lds = 64 * R * sizeof(zd);
-  if (b.left) {
-    auto k = ztrevc_big_solve<R, TransG<zd>>;
-    (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(k, dim3(n), dim3(64), lds, s, b, TransG<zd>{b.Tt, n});
+template <int R> static hipError_t launch_ztrevc_r(const TrevcArgs& a, int nmax, hipStream_t s) {
+  const size_t lds = wavevec_lds_bytes<R>();
+  const int nt = (nmax + 63) / 64;
+  hipLaunchKernelGGL(ztrevc_norms_kernel, dim3((nmax + 3) / 4, a.count), dim3(256), 0, s, a);
+  if (a.left) {
+    hipLaunchKernelGGL(trevc_transpose_kernel<zd>, dim3((nmax + 31) / 32, (nmax + 31) / 32, a.count), dim3(256), 0, s,
+                       a);
+    hipLaunchKernelGGL((ztrevc_solve_kernel<R, true>), dim3(nmax, a.count), dim3(64), lds, s, a);
   } else {
-    auto k = ztrevc_big_solve<R, GlobZ>;
-    (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(k, dim3(n), dim3(64), lds, s, b, GlobZ{b.T, b.ldt});
+    hipLaunchKernelGGL((ztrevc_solve_kernel<R, false>), dim3(nmax, a.count), dim3(64), lds, s, a);
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (b.Z) {
-    // [Yr | Yi] = Re Z [Xr | Xi]; Yr -= Im Z Xi; Yi += Im Z Xr
-    const int64_t nn = (int64_t)n * n;
-    const double *Zr = b.Zp, *Zi = b.Zp + nn, *Xr = b.X, *Xi = b.X + nn;
-    double *Yr = b.Y, *Yi = b.Y + nn;
-    if ((e = launch_dgemm(false, false, n, 2 * n, n, 1.0, Zr, n, Xr, n, 0.0, Yr, n, s)) != hipSuccess) return e;
-    if ((e = launch_dgemm(false, false, n, n, n, -1.0, Zi, n, Xi, n, 1.0, Yr, n, s)) != hipSuccess) return e;
-    if ((e = launch_dgemm(false, false, n, n, n, 1.0, Zi, n, Xr, n, 1.0, Yi, n, s)) != hipSuccess) return e;
-  }
-  (void)hipFuncSetAttribute((const void*)ztrevc_big_finish<R>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(ztrevc_big_finish<R>, dim3(n), dim3(64), lds, s, b);
+  if (a.Z) hipLaunchKernelGGL(trevc_back_kernel<zd>, dim3(nt, nt, a.count), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(ztrevc_finish_kernel<R>, dim3(nmax, a.count), dim3(64), lds, s, a);
   return hipGetLastError();
 }
 
-// a.T, a.Z, a.V point at the matrix (complex interleaved), ld from
-// a.ldt/ldz/ldv; ws holds ztrevc_big_ws_bytes(n)
-hipError_t launch_ztrevc_big(const TrevcArgs& a, int n, void* ws, hipStream_t s) {
-  if (n <= ztrevc_max_n() || n > trevc_big_max_n() || !ws) return hipErrorInvalidValue;
-  const size_t nn = (size_t)n * n;
-  char* p = static_cast<char*>(ws);
-  ZBig b;
-  b.n = n;
-  b.left = a.left;
-  b.normalize = a.normalize;
-  b.T = reinterpret_cast<const zd*>(a.T);
-  b.ldt = a.ldt > 0 ? a.ldt : n;
-  b.Z = reinterpret_cast<const zd*>(a.Z);
-  b.ldz = a.ldz > 0 ? a.ldz : n;
-  b.V = reinterpret_cast<zd*>(a.V);
-  b.ldv = a.ldv > 0 ? a.ldv : n;
-  b.tnorms = reinterpret_cast<double*>(p);
-  p += trevc_seg(8 * (size_t)n);
-  zd* tt = reinterpret_cast<zd*>(p);
-  b.Tt = tt;
-  p += trevc_seg(16 * nn);
-  b.Zp = reinterpret_cast<double*>(p);
-  p += trevc_seg(16 * nn);
-  b.X = reinterpret_cast<double*>(p);
-  p += trevc_seg(16 * nn);
-  b.Y = reinterpret_cast<double*>(p);
-  // strictly-upper column norms: abs for right (vectors.jl:70-75), abs1 for
-  // left (vectors.jl:395-400)
-  hipLaunchKernelGGL(trevc_colnorm_kernel<zd>, dim3((n + 3) / 4), dim3(256), 0, s, n, b.T, b.ldt, b.left != 0,
-                     b.tnorms);
-  if (b.left)
-    hipLaunchKernelGGL(trevc_transpose_kernel<zd>, dim3((n + 31) / 32, (n + 31) / 32), dim3(256), 0, s, n, b.T,
-                       b.ldt, tt);
-  if (b.Z) hipLaunchKernelGGL(ztrevc_big_planar, dim3(2048), dim3(256), 0, s, n, b.Z, b.ldz, b.Zp);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return n <= 2048 ? launch_zbig_r<32>(b, s) : launch_zbig_r<64>(b, s);
+hipError_t launch_ztrevc(const TrevcArgs& a, int nmax, hipStream_t s) {
+  switch (trevc_class(nmax)) {
+    case 1: return launch_ztrevc_r<1>(a, nmax, s);
+    case 2: return launch_ztrevc_r<2>(a, nmax, s);
+    case 4: return launch_ztrevc_r<4>(a, nmax, s);
+    case 8: return launch_ztrevc_r<8>(a, nmax, s);
+    case 16: return launch_ztrevc_r<16>(a, nmax, s);
+    case 32: return launch_ztrevc_r<32>(a, nmax, s);
+    case 64: return launch_ztrevc_r<64>(a, nmax, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace gs

@@ -232,3 +232,39 @@ def test_vectors_unnormalized(gs, oracle, n, cplx):
         Vg = gs.geigvecs(S(T, Z, w), left=left, normalize=False)
         Vo = oracle.eigvecs(T, Z, left=left, normalize=False)
         assert np.abs(Vg - Vo).max() <= (1e-9 if n <= 64 else 1e-7), left
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("left", [False, True])
+def test_class_edges_batched(gs, cplx, left):
+    """Orders at the edges of the launch classes (entries per lane), the back
+    transform's tiles and the 64-row factor chunks, in one batch with an empty
+    matrix: the batch gives the single calls' bits, and every vector satisfies
+    its eigenvalue equation (residual at most 50 n eps ||A||_F, unit vectors)."""
+    import ctypes
+    from genericschur import _lib
+    orders = (1, 2, 3, 15, 63, 64, 65, 0, 127, 128, 129, 130, 200, 256, 257, 300)
+    mats = []
+    for n in orders:
+        rng = gen.stream(41, 100, n)
+        mats.append(gen.ginibre_complex(n, rng) if cplx else gen.ginibre_real(n, rng))
+    Ss = [gs.gschur(A) for A in mats]
+    dt = np.complex128 if cplx else np.float64
+    ns, off, T = gs.pack([S.T for S in Ss], dt)
+    _, _, Z = gs.pack([S.Z for S in Ss], dt)
+    V = np.zeros(T.shape, dtype=np.complex128)
+    h = _lib.handle()
+    p = lambda a: ctypes.c_void_p(a.ctypes.data)
+    f = _lib.lib().gs_trevc_batched_z if cplx else _lib.lib().gs_trevc_batched_d
+    _lib.check(f(h, len(ns), p(ns), p(off), p(T), p(Z), p(V), int(left), 1, 0), h, "gs_trevc_batched")
+    eps = np.finfo(np.float64).eps
+    for A, S, X in zip(mats, Ss, gs.unpack(ns, off, V)):
+        n = A.shape[0]
+        print(f"case vectors n={n} cplx={cplx} left={left}", flush=True)
+        if n == 0:
+            continue
+        assert np.array_equal(X, gs.geigvecs(S, left=left))
+        M, w = (A.conj().T, S.values.conj()) if left else (A, S.values)
+        res = np.linalg.norm(M @ X - X * w, axis=0)
+        assert res.max() <= 50 * n * eps * np.linalg.norm(A)
+        assert np.abs(np.linalg.norm(X, axis=0) - 1).max() <= 50 * eps
