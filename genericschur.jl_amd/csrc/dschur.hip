@@ -498,7 +498,7 @@ constexpr int DWL = DW + 1;  // odd LDS pitch of a window column (bank spread)
 
 // Z log of the windowed real QR kernel (records: chains.h::dlog_row).  Z is
 // not read while the sweeps run, so the kernel records them (and the 2 x 2
-// blocks' rotations) and dlog_kernel applies the records to Z, held in LDS,
+// blocks' rotations) and dlog_kernel applies the records to Z, held in registers,
 // afterwards.  A record that would not fit makes the kernel apply the log so
 // far to Z in HBM itself and start it again.
 struct DLog {
@@ -979,113 +979,107 @@ hipError_t launch_dqrw(const BatchArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// After a bin's QR launch (orders 65 .. 128): each matrix's Z log applied to
-// Z by one workgroup of ceil(n / 64) wavefronts, all of Z in LDS (row r,
-// column c at zs[(c - 1) n + r]), each thread replaying the log on one row
-// (dlog_row's operations).  Each wavefront stages a record in its own LDS
-// buffer and loads the next one into registers while it replays the
-// current one.
-constexpr int DLREC = 384;  // >= 2 + 3 (n - 1) for n <= 128
-__global__ void __launch_bounds__(128) dlog_kernel(BatchArgs a) {
-  extern __shared__ double dzs[];
-  __shared__ double rbuf[2][DLREC];  // a separate array: its reads do not wait on the row writes
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int b = blockIdx.x;
-  if (b >= a.count) return;
-  const int m = a.order[a.first + b];
+// After a bin's QR launch: each matrix's Z log applied to Z, one wavefront per
+// 64 rows and one row per lane with its NC entries in registers (zlog_kernel's
+// form, dlog_row's operations; a sweep's last, two-element step is logged with
+// v3 = 0 and runs as a three-element one).  1208 matrices n = 97..128 take 4.5
+// ms and 1094 n = 65..96 1.2 ms, against 8.7 ms together with Z in LDS.
+template <int NC> __global__ void __launch_bounds__(64) dlog_kernel(BatchArgs a) {
+  constexpr int NT = (2 + 3 * NC + 63) / 64;  // a record has at most 2 + 3 (n - 1) doubles
+  constexpr int NE = (4 * NC + 63) / 64;      // lane registers of a sweep's steps
+  constexpr int NG = NC / 8;
+  __shared__ double ev[64 * NE];
+  const int lane = threadIdx.x;
+  const int m = a.order[a.first + blockIdx.x];
   const int n = a.n[m];
-  if (n <= 0 || wave * 64 >= n) return;
+  if (n > NC || (int)blockIdx.y * 64 >= n) return;
   const int64_t len = a.llen[m];
   if (len <= 0) return;
   double* Z = a.Z + a.off[m];
   const double* lg = a.zlog + a.loff[m];
-  const int r = min(tid, n - 1);  // threads past the last row repeat it, unstored
-  const bool live = tid < n;
-  double t[DLREC / 64];
+  const int row = blockIdx.y * 64 + lane;
+  const int r = min(row, n - 1);  // lanes past the last row repeat it, unstored
+  double t[NT];
   auto fetch = [&](int64_t p) {
 #pragma unroll
-    for (int j = 0; j < DLREC / 64; ++j) t[j] = lg[min(p + lane + 64 * j, len - 1)];
+    for (int j = 0; j < NT; ++j) t[j] = lg[min(p + lane + 64 * j, len - 1)];
   };
-  fetch(0);
-  for (int c0 = 0; c0 < n; c0 += 8) {
-    double v[8];
+  double x[NC];
+  const double* zc = Z;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = Z[r + (int64_t)min(c0 + i, n - 1) * n];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (c0 + i < n && live) dzs[(c0 + i) * n + r] = v[i];
+  for (int c = 0; c < NC; ++c) {
+    x[c] = zc[(unsigned)r];
+    zc += c + 1 < n ? n : 0;
+    asm volatile("" : "+s"(zc));
   }
-  double* row = dzs + r;
-  const int st = n;
-  double* rec = rbuf[wave];
+  fetch(0);
   for (int64_t pos = 0; pos < len;) {
+    const int h0 = __builtin_amdgcn_readfirstlane((int)t[0]);
+    if (h0 < 0) {  // Givens rotation of columns -h0, -h0 + 1 (1-based)
+      const int c0 = -h0 - 1;
+      const double cs = rdlane(t[0], 1), sn = rdlane(t[0], 2);
+      pos += 3;
+      fetch(pos);
 #pragma unroll
-    for (int j = 0; j < DLREC / 64; ++j) rec[lane + 64 * j] = t[j];
+      for (int g = 0; g < NG; ++g)
+        if ((c0 >> 3) == g) {
+#pragma unroll
+          for (int c = 8 * g; c < 8 * g + 8; ++c)
+            if (c + 1 < NC) drot_fixed(x[c], x[c + 1], c == c0 ? cs : 1.0, c == c0 ? sn : 0.0);
+        }
+      continue;
+    }
+    // 0-based: steps s0 .. s1, the last one (two elements) logged with v3 = 0
+    const int s0 = h0 - 1, s1 = (int)rdlane(t[0], 1) - 2;
+    const int rl = 2 + 3 * (s1 + 1 - s0);
+    const int g0 = s0 >> 3, g1 = s1 >> 3;
+    wsync();  // the previous record's reads
+    ev[32 * (lane < 32 ? g0 : g1) + (lane & 31)] = 0.0;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int e = lane + 64 * j - 2, st = e / 3;
+      if (e >= 0 && e < rl - 2) ev[4 * (s0 + st) + e - 3 * st] = t[j];
+    }
     wsync();
-    const double h0 = rec[0];
-    const bool rotation = h0 < 0.0;
-    const int i1 = __builtin_amdgcn_readfirstlane(rotation ? (int)(-h0) : (int)h0);
-    const int ie = __builtin_amdgcn_readfirstlane(rotation ? 0 : (int)rec[1]);
-    const int64_t rl = rotation ? 3 : 2 + 3 * (int64_t)(ie - i1);
-    if (pos + rl < len) fetch(pos + rl);
-    if (live) {
-      if (rotation) {
-        double a1 = row[(i1 - 1) * st], a2 = row[i1 * st];
-        drot_fixed(a1, a2, rec[1], rec[2]);
-        row[(i1 - 1) * st] = a1;
-        row[i1 * st] = a2;
-      } else {
-        const double* e = rec + 2;
-        double c0 = row[(i1 - 1) * st], c1 = row[i1 * st];
-        // groups of eight steps: the group's row entries (which its own steps
-        // do not write first) are read before any of its writes
-        int k = i1;
-        for (; k + 7 < ie - 1; k += 8) {
-          double bb[8];
+    pos += rl;
+    fetch(pos);
+    double ex[NE];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) bb[j] = row[(k + j + 1) * st];
+    for (int j = 0; j < NE; ++j) ex[j] = ev[lane + 64 * j];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            drefl3_fixed(c0, c1, bb[j], e[3 * (k + j - i1)], e[3 * (k + j - i1) + 1], e[3 * (k + j - i1) + 2]);
-            row[(k + j - 1) * st] = c0;
-            c0 = c1;
-            c1 = bb[j];
-          }
+    for (int g = 0; g < NG; ++g) {
+      if (g >= g0 && g <= g1) {
+#pragma unroll
+        for (int k = 8 * g; k < 8 * g + 8; ++k) {
+          const int j = (4 * k) >> 6, l = (4 * k) & 63;
+          const double t1 = rdlane(ex[j], l), v2 = rdlane(ex[j], l + 1), v3 = rdlane(ex[j], l + 2);
+          if (k + 2 < NC) drefl3_fixed(x[k], x[k + 1], x[k + 2], t1, v2, v3);
+          else if (k + 1 < NC) drefl2_fixed(x[k], x[k + 1], t1, v2);
+          if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
-        for (; k < ie - 1; ++k) {
-          double bb = row[(k + 1) * st];
-          drefl3_fixed(c0, c1, bb, e[3 * (k - i1)], e[3 * (k - i1) + 1], e[3 * (k - i1) + 2]);
-          row[(k - 1) * st] = c0;
-          c0 = c1;
-          c1 = bb;
-        }
-        drefl2_fixed(c0, c1, e[3 * (ie - 1 - i1)], e[3 * (ie - 1 - i1) + 1]);
-        row[(ie - 2) * st] = c0;
-        row[(ie - 1) * st] = c1;
       }
     }
-    wsync();  // the record buffer is rewritten for the next record
-    pos += rl;
   }
-  if (live) {
-    for (int c0 = 0; c0 < n; c0 += 8) {
-      double v[8];
+  if (row < n) {
+    double* zs = Z;
+    asm volatile("" : "+s"(zs));
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = dzs[min(c0 + i, n - 1) * n + r];
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (c0 + i < n) Z[r + (int64_t)(c0 + i) * n] = v[i];
+    for (int c = 0; c < NC; ++c) {
+      if (c < n) zs[(unsigned)row] = x[c];
+      zs += n;
+      asm volatile("" : "+s"(zs));
     }
   }
 }
 
 hipError_t launch_dlog(const BatchArgs& a, int nmax, hipStream_t s) {
   if (a.count <= 0 || !a.zlog) return hipSuccess;
-  if (2 + 3 * (nmax - 1) > DLREC || nmax > 128) return hipErrorInvalidValue;
-  const int waves = (nmax + 63) / 64;
-  const size_t lds = (size_t)nmax * nmax * sizeof(double);
-  (void)hipFuncSetAttribute((const void*)dlog_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(dlog_kernel, dim3(a.count), dim3(64 * waves), lds, s, a);
+  const dim3 g(a.count, (nmax + 63) / 64);
+  if (nmax <= 32) hipLaunchKernelGGL(dlog_kernel<32>, g, dim3(64), 0, s, a);
+  else if (nmax <= 64) hipLaunchKernelGGL(dlog_kernel<64>, g, dim3(64), 0, s, a);
+  else if (nmax <= 96) hipLaunchKernelGGL(dlog_kernel<96>, g, dim3(64), 0, s, a);
+  else if (nmax <= 128) hipLaunchKernelGGL(dlog_kernel<128>, g, dim3(64), 0, s, a);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

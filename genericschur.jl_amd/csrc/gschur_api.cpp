@@ -488,13 +488,15 @@ static int build_plan(gs_handle* h, bool cplx, int64_t count, const int32_t* n, 
   return GS_OK;
 }
 
-// Bin orders whose QR launch logs its Z updates.  The smallest: measured on
-// MI355X with each launch alone, a bin's QR + replay against in-place
-// updates: n = 81..96 (1470 matrices) 25.1 ms vs 32.4 ms, n = 65..80 (1479)
-// 16.7 ms vs 15.0 ms.  The largest real one: the replay holds all of Z in
-// LDS with its record buffers (128^2 doubles + 6 KB).
-constexpr int kZlogMinN = 81;
-constexpr int kDlogMinN = 33;
+// Bin orders whose QR launch logs its Z updates (the bin's largest order is
+// at least the minimum).  Measured with each launch alone, QR + replay against
+// in place: complex n = 4..24 (1000 matrices) 1.29 against 1.25 ms, and with
+// every larger order of 8192 matrices n ~ U{8..96} in place up to 72 the batch
+// takes 56.3 ms, with the log from 25 up 50.9 ms; real n = 4..24 0.72 against
+// 0.79 ms, n = 16..32 1.14 against 1.23 ms, n = 129..141 (1000 matrices, the
+// replay's row no longer fits the registers) 30.6 against 30.2 ms.
+constexpr int kZlogMinN = 25;
+constexpr int kDlogMinN = 2;
 constexpr int kDlogMaxN = 128;
 
 // Whether the batched QR launches of this call log their Z updates
@@ -674,8 +676,7 @@ static hipError_t launch_plan(gs_handle* h, const PlanDev& pd, const double* A, 
     }
     a.first = b.first;
     a.count = b.count;
-    // the Z log pays off where Z's rows are long (its replay holds all of Z
-    // in LDS); GS_ZLOG_TINY exercises it on every bin
+    // GS_ZLOG_TINY exercises the Z log on every bin
     a.zlog = (zl && bin_zlog(p->is_complex, b, flags)) ? zlog : nullptr;
     if (timed && (e = hipEventRecord(h->tev[6 * bi + 2], s)) != hipSuccess) return e;
     if (flags & GS_QR_BAND)

@@ -13,8 +13,8 @@
 // in LDS (one workgroup per matrix); zqrw2_kernel runs the QR iterations
 // with H and Z in HBM, two wavefronts per matrix (the bulge chase in a
 // 32 x 32 LDS window, and the chunk's reflectors applied to the rest of H
-// and Z as chains); for bins above n = 80 it logs the Z updates instead and
-// zlog_kernel applies the log with Z in LDS.  zqr_kernel (GS_QR_BAND) keeps
+// and Z as chains); for most bins it logs the Z updates instead and
+// zlog_kernel applies the log with Z's rows in registers.  zqr_kernel (GS_QR_BAND) keeps
 // H's band j >= i-2 in LDS instead.  The single-matrix kernel keeps H in
 // HBM.
 //
@@ -700,7 +700,7 @@ template <int G> GS_DEV void zchain_full_row(zd* p, int64_t st, const zd* lg, in
 
 // Z log of the windowed QR kernel.  Z is not read while the sweeps run, so
 // instead of updating Z in HBM after every chunk the kernel records each
-// sweep and zlog_kernel applies the records to Z, held in LDS, afterwards:
+// sweep and zlog_kernel applies the records to Z, held in registers, afterwards:
 // the same operations on every element of Z in the same order.  Record of a
 // sweep, in complex entries: (istart1, iend); ctt of the phase scaling after
 // the first step, or 0; (tau1, v2) per step; t of the tail scaling, or 0.
@@ -1770,118 +1770,154 @@ hipError_t launch_zqrw_single(const BatchArgs& a, int nt, hipStream_t s) {
   return hipGetLastError();
 }
 
-// After a bin's QR launch: each matrix's Z log applied to Z by one
-// workgroup of ceil(n / 64) wavefronts, all of Z held in LDS (row r, column
-// c at zs[(c - 1) n + r]), each thread replaying the log on one row with
-// zlog_row's operations.  Each wavefront stages a sweep's record in its own
-// LDS buffer and loads the next record into registers while it replays the
-// current one, so the wavefronts never wait for each other.
-constexpr int ZLREC = 200;  // >= 3 + 2 (n - 1) for every batched complex order
-__global__ void __launch_bounds__(128) zlog_kernel(BatchArgs a) {
-  extern __shared__ zd zs[];
-  __shared__ zd rbuf[2][ZLREC];  // a separate array: its reads do not wait on the row writes
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int b = blockIdx.x;
-  if (b >= a.count) return;
-  const int m = a.order[a.first + b];
+// After the QR launch: each matrix's Z log applied to Z, one wavefront per 64
+// rows and one row per lane, the row's NC entries in registers (n <= NC), with
+// zlog_row's operations.  A sweep runs over the row in groups of eight steps
+// whose indices are compile-time constants; uniform branches skip the groups
+// outside the sweep, and its two end groups are filled with zero reflectors
+// (x -= 0: the entries keep their values).  The scalings work the same way,
+// with factor 1.  A sweep's record goes through LDS to its absolute step index
+// and from there into the lanes (entry l + 64 j in lane l), so that a step
+// reads its reflector by v_readlane with constant lanes (as LDS broadcasts 5.2
+// against 5.1 ms for 2230 matrices n = 73..96; by scalar loads four steps
+// ahead, which still waited for L2, 8.2 ms).  The next record is loaded
+// meanwhile.  About 28 instructions per step, bound by their issue from the
+// one wavefront per SIMD that a row of 384 registers leaves.  Rows never meet,
+// so nothing is gained by holding all of Z in LDS, which allowed one workgroup
+// of two wavefronts per CU above order 72: those 2230 matrices took 9.6 ms,
+// and the smaller orders' updates stayed in the QR launch (8192 matrices n ~
+// U{8..96}: QR launch 36.5 -> 32.9 ms, the batch 56.3 -> 50.9 ms).
+template <int NC> __global__ void __launch_bounds__(64) zlog_kernel(BatchArgs a) {
+  constexpr int NT = (2 * NC + 1 + 63) / 64;  // a record has at most 3 + 2 (n - 1) entries
+  constexpr int NE = (2 * NC + 63) / 64;      // lane registers of a sweep's steps
+  constexpr int NG = NC / 8;
+  __shared__ zd ev[64 * NE];
+  __shared__ zd tl;
+  const int lane = threadIdx.x;
+  const int m = a.order[a.first + blockIdx.x];
   const int n = a.n[m];
-  if (n <= 0 || wave * 64 >= n) return;
+  if (n > NC || (int)blockIdx.y * 64 >= n) return;
   const int64_t len = a.llen[m];
   if (len <= 0) return;
   zd* Z = reinterpret_cast<zd*>(a.Z) + a.off[m];
   const zd* lg = reinterpret_cast<const zd*>(a.zlog) + a.loff[m];
-  const int r = min(tid, n - 1);  // threads past the last row repeat it, unstored
-  const bool live = tid < n;
-  zd t[4];
+  const int row = blockIdx.y * 64 + lane;
+  const int r = min(row, n - 1);  // lanes past the last row repeat it, unstored
+  double tx[NT], ty[NT];
   auto fetch = [&](int64_t p) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) t[j] = lg[min(p + lane + 64 * j, len - 1)];
-  };
-  fetch(0);
-  for (int c0 = 0; c0 < n; c0 += 8) {
-    zd v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = Z[r + (int64_t)min(c0 + i, n - 1) * n];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (c0 + i < n && live) zs[(c0 + i) * n + r] = v[i];
-  }
-  zd* row = zs + r;
-  const int st = n;
-  zd* rec = rbuf[wave];
-  for (int64_t pos = 0; pos < len;) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (lane + 64 * j < ZLREC) rec[lane + 64 * j] = t[j];
-    wsync();
-    const zd h0 = rec[0];
-    const int i1 = __builtin_amdgcn_readfirstlane((int)h0.x), ie = __builtin_amdgcn_readfirstlane((int)h0.y);
-    const int64_t rl = 3 + 2 * (int64_t)(ie - i1);
-    if (pos + rl < len) fetch(pos + rl);
-    if (live) {
-      const zd ctt = rec[1];
-      const zd* e = rec + 2;
-      zd c0 = row[(i1 - 1) * st];
-      {  // first step, then the phase scaling when logged
-        zd x1 = row[i1 * st];
-        zrot_right_fixed(c0, x1, e[0], e[1]);
-        row[(i1 - 1) * st] = c0;
-        c0 = x1;
-        if (!(ctt.x == 0.0 && ctt.y == 0.0)) {
-          row[(i1 - 1) * st] = zmul_fixed(row[(i1 - 1) * st], ctt);
-#pragma unroll 4
-          for (int c = i1 + 2; c <= ie; ++c) row[(c - 1) * st] = zmul_fixed(row[(c - 1) * st], ctt);
-        }
-      }
-      // groups of eight steps: the group's row entries (which its own steps
-      // do not write first) are read before any of its writes, so a group
-      // waits for LDS once
-      int k = i1 + 1;
-      for (; k + 7 < ie; k += 8) {
-        zd xa[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) xa[j] = row[(k + j) * st];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          zrot_right_fixed(c0, xa[j], e[2 * (k + j - i1)], e[2 * (k + j - i1) + 1]);
-          row[(k + j - 1) * st] = c0;
-          c0 = xa[j];
-        }
-      }
-      for (; k < ie; ++k) {
-        zd x1 = row[k * st];
-        zrot_right_fixed(c0, x1, e[2 * (k - i1)], e[2 * (k - i1) + 1]);
-        row[(k - 1) * st] = c0;
-        c0 = x1;
-      }
-      row[(ie - 1) * st] = c0;
-      const zd tt = e[2 * (ie - i1)];
-      if (!(tt.x == 0.0 && tt.y == 0.0)) row[(ie - 1) * st] = zmul_fixed(row[(ie - 1) * st], tt);
+    for (int j = 0; j < NT; ++j) {
+      const zd v = lg[min(p + lane + 64 * j, len - 1)];
+      tx[j] = v.x;
+      ty[j] = v.y;
     }
-    wsync();  // the record buffer is rewritten for the next sweep
-    pos += rl;
+  };
+  // Z's columns through a scalar base and one lane offset (an address pair per
+  // column would cost as many registers as the row)
+  zd x[NC];
+  const zd* zc = Z;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    x[c] = zc[(unsigned)r];
+    zc += c + 1 < n ? n : 0;
+    asm volatile("" : "+s"(zc));
   }
-  if (live) {
-    for (int c0 = 0; c0 < n; c0 += 8) {
-      zd v[8];
+  fetch(0);
+  for (int64_t pos = 0; pos < len;) {
+    // 0-based: the sweep's steps are s0 .. s1 - 1, its columns s0 .. s1
+    const int s0 = __builtin_amdgcn_readfirstlane((int)tx[0]) - 1;
+    const int s1 = __builtin_amdgcn_readfirstlane((int)ty[0]) - 1;
+    const zd ctt = zmk(rdlane(tx[0], 1), rdlane(ty[0], 1));
+    const int rl = 3 + 2 * (s1 - s0);
+    const int g0 = s0 >> 3, g1 = (s1 - 1) >> 3;
+    wsync();  // the previous sweep's reads
+    if (lane < 32) ev[16 * (lane < 16 ? g0 : g1) + (lane & 15)] = zr(0.0);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = zs[min(c0 + i, n - 1) * n + r];
+    for (int j = 0; j < NT; ++j) {
+      const int e = lane + 64 * j;
+      if (e >= 2 && e < rl - 1) ev[2 * s0 + e - 2] = zmk(tx[j], ty[j]);
+      if (e == rl - 1) tl = zmk(tx[j], ty[j]);
+    }
+    wsync();
+    pos += rl;
+    fetch(pos);
+    if (!(ctt.x == 0.0 && ctt.y == 0.0)) {
+      // the first step, then the logged phase scaling of columns s0 and
+      // s0 + 2 .. s1
+      const zd ta = ev[2 * s0], va = ev[2 * s0 + 1];
+      wsync();
+      if (lane < 2) ev[2 * s0 + lane] = zr(0.0);
+      wsync();
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (c0 + i < n) Z[r + (int64_t)(c0 + i) * n] = v[i];
+      for (int g = 0; g < NG; ++g)
+        if (g == g0) {
+#pragma unroll
+          for (int k = 8 * g; k < 8 * g + 8; ++k)
+            if (k + 1 < NC) zrot_right_fixed(x[k], x[k + 1], zmk(k == s0 ? ta.x : 0.0, k == s0 ? ta.y : 0.0), va);
+        }
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+        if (g >= g0 && g <= (s1 >> 3)) {
+#pragma unroll
+          for (int c = 8 * g; c < 8 * g + 8; ++c) {
+            const bool on = c == s0 || (c >= s0 + 2 && c <= s1);
+            x[c] = zmul_fixed(x[c], zmk(on ? ctt.x : 1.0, on ? ctt.y : 0.0));
+          }
+        }
+    }
+    double ex[NE], ey[NE];
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+      const zd v = ev[lane + 64 * j];
+      ex[j] = v.x;
+      ey[j] = v.y;
+    }
+    const zd tt = tl;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g >= g0 && g <= g1) {
+#pragma unroll
+        for (int k = 8 * g; k < 8 * g + 8; ++k) {
+          const int j = (2 * k) >> 6, l = (2 * k) & 63;
+          if (k + 1 < NC)
+            zrot_right_fixed(x[k], x[k + 1], zmk(rdlane(ex[j], l), rdlane(ey[j], l)),
+                             zmk(rdlane(ex[j], l + 1), rdlane(ey[j], l + 1)));
+          if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    if (!(tt.x == 0.0 && tt.y == 0.0)) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+        if ((s1 >> 3) == g) {
+#pragma unroll
+          for (int c = 8 * g; c < 8 * g + 8; ++c)
+            x[c] = zmul_fixed(x[c], zmk(c == s1 ? tt.x : 1.0, c == s1 ? tt.y : 0.0));
+        }
+    }
+  }
+  if (row < n) {
+    zd* zs = Z;
+    asm volatile("" : "+s"(zs));
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      if (c < n) zs[(unsigned)row] = x[c];
+      zs += n;
+      asm volatile("" : "+s"(zs));
     }
   }
 }
 
-static size_t zlog_lds_bytes(int nmax) { return (size_t)nmax * nmax * sizeof(zd); }
-
 hipError_t launch_zlog(const BatchArgs& a, int nmax, hipStream_t s) {
   if (a.count <= 0 || !a.zlog) return hipSuccess;
-  if (3 + 2 * (nmax - 1) > ZLREC || nmax > 128) return hipErrorInvalidValue;
-  const int waves = (nmax + 63) / 64;
-  const size_t lds = zlog_lds_bytes(nmax);
-  (void)hipFuncSetAttribute((const void*)zlog_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(zlog_kernel, dim3(a.count), dim3(64 * waves), lds, s, a);
+  const dim3 g(a.count, (nmax + 63) / 64);
+  if (nmax <= 32) hipLaunchKernelGGL(zlog_kernel<32>, g, dim3(64), 0, s, a);
+  else if (nmax <= 48) hipLaunchKernelGGL(zlog_kernel<48>, g, dim3(64), 0, s, a);
+  else if (nmax <= 64) hipLaunchKernelGGL(zlog_kernel<64>, g, dim3(64), 0, s, a);
+  else if (nmax <= 80) hipLaunchKernelGGL(zlog_kernel<80>, g, dim3(64), 0, s, a);
+  else if (nmax <= 96) hipLaunchKernelGGL(zlog_kernel<96>, g, dim3(64), 0, s, a);
+  else if (nmax <= 104) hipLaunchKernelGGL(zlog_kernel<104>, g, dim3(64), 0, s, a);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

@@ -183,3 +183,22 @@ def test_windowed_matches_band_qr(gs):
                 assert np.linalg.norm(a.Z - b.Z @ D) <= 1e-6 * n
                 nphase += 1
         print(f"{kind}: bitwise equal {nbit}, equal up to diagonal phases {nphase}, of {len(mats)}", flush=True)
+
+
+@pytest.mark.parametrize("cplx,n", [(True, n) for n in (25, 31, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 99)] +
+                         [(False, n) for n in (2, 3, 4, 8, 9, 10, 32, 33, 64, 65, 96, 97, 128, 129)])
+def test_log_replay_order_edges(gs, cplx, n):
+    """The Z log's replay at the edges of its register classes, groups of
+    eight steps and blocks of 64 rows: T, Z and the values bitwise those of
+    the updates in place.  The matrices deflate in the middle (sweeps that
+    start late) and, real, leave 2 x 2 blocks to rotate."""
+    rng = gen.stream(33, 100, n)
+    mats = [gen.ginibre_complex(n, rng) if cplx else gen.ginibre_real(n, rng) for _ in range(3)]
+    B = mats[0].copy()
+    B[n // 2:, :n // 2] *= 1e-13
+    mats += [B, gen.cyclic_shift(n, cplx) if n > 2 else mats[1]]
+    Sl, il = gs.gschur_batched(mats)
+    Sd, _ = gs.gschur_batched(mats, zdirect=True)
+    assert np.all(il == 0)
+    for a, d in zip(Sl, Sd):
+        assert np.array_equal(a.T, d.T) and np.array_equal(a.Z, d.Z) and np.array_equal(a.values, d.values)
