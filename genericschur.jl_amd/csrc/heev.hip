@@ -295,7 +295,7 @@ GS_DEV void st_solve(StState& S, double* d, double* e, bool wantz, int nrows, ZA
   const int tid = threadIdx.x;
   const StVec dv{d, 1}, ev{e, 1};
   if (!wantz) {
-    if (tid == 0) st_produce<StLog>(S, dv, ev, nullptr);
+    if (tid == 0) st_produce<false, StLog>(S, dv, ev, nullptr);
     __syncthreads();
     return;
   }
@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(64) steqr_lanes_kernel(HeevArgs a) {
     st_produce(S, d, e, &L);
     a.logpos[b] = L.pos;
   } else {
-    st_produce<StLogG>(S, d, e, nullptr);
+    st_produce<false, StLogG>(S, d, e, nullptr);
   }
   for (int i = 0; i < n; ++i) a.W[(int64_t)b * a.sW + i] = d[i];
   for (int i = 0; i < n - 1; ++i) a.E[(int64_t)b * a.sE + i] = e[i];
@@ -694,42 +694,54 @@ template <class T> __global__ void __launch_bounds__(256) hb_out_kernel(HbArgs<T
   }
 }
 
-// The QL/QR recurrence of one large matrix by one thread (d, e staged in
-// LDS), from the start or (resume) from the state record; with rec its
-// rotations go to a record stream in HBM, and a full stream stops it at a
-// step boundary with its state left for the next round.
-__global__ void __launch_bounds__(64) hb_produce_kernel(int n, int maxsweeps, double* d, double* e, double2* rec,
-                                                       int cap, int* npos, StState* state, int resume) {
+// One round of a large matrix's QL/QR iteration.  Workgroup 0: the recurrence
+// (d, e staged in LDS), every lane of one wavefront running the same scalar
+// chain and sharing its searches, from the start or (resume) from the state
+// record; its rotations go to the record stream rec in HBM, and a full stream
+// stops it at a step boundary with its state left for the next round.
+// Workgroups 1 ..: the previous round's stream replayed onto rows 0 .. nrows-1
+// of Z (ld ldz), one row per lane.  Bound by the recurrence's chain, about 400
+// cycles per rotation (950 as one lane's rotation at a time, with a branch
+// for each scaling case and full square root and divisions); the replay, which
+// took another 100 ms in a launch of its own, runs beside it.  Order 1000
+// complex with vectors: 585 -> 239 ms.
+template <class T> __global__ void __launch_bounds__(64) hb_round_kernel(int n, int maxsweeps, double* d, double* e,
+                                                                        double2* rec, int cap, int* npos,
+                                                                        StState* state, int resume, int nrows,
+                                                                        int64_t ldz, const double2* prec,
+                                                                        const int* pnpos, T* Z) {
   extern __shared__ double smem[];
+  if (blockIdx.x > 0) {
+    const int r = (blockIdx.x - 1) * 64 + threadIdx.x;
+    if (r < nrows) st_replay_row<T>(prec, *pnpos, [&](int k) -> T& { return Z[r + (int64_t)(k - 1) * ldz]; });
+    return;
+  }
   double* dl = smem;
   double* el = smem + n;
   for (int i = threadIdx.x; i < n; i += 64) dl[i] = d[i];
   for (int i = threadIdx.x; i < n - 1; i += 64) el[i] = e[i];
   __syncthreads();
-  if (threadIdx.x == 0) {
-    StState S;
-    if (resume) S = *state;
-    else st_init(S, n, maxsweeps);
-    if (rec) {
-      StLogG L;
-      L.rec = rec;
-      L.pos = 0;
-      L.cap = cap;
-      st_produce(S, StVec{dl, 1}, StVec{el, 1}, &L);
-      *npos = L.pos;
-    } else {
-      st_produce<StLogG>(S, StVec{dl, 1}, StVec{el, 1}, nullptr);
-      *npos = 0;
-    }
-    *state = S;
+  StState S;
+  if (resume) S = *state;
+  else st_init(S, n, maxsweeps);
+  if (rec) {
+    StLogG L;
+    L.rec = rec;
+    L.pos = 0;
+    L.cap = cap;
+    st_produce<true>(S, StVec{dl, 1}, StVec{el, 1}, &L);
+    if (threadIdx.x == 0) *npos = L.pos;
+  } else {
+    st_produce<true, StLogG>(S, StVec{dl, 1}, StVec{el, 1}, nullptr);
+    if (threadIdx.x == 0) *npos = 0;
   }
+  if (threadIdx.x == 0) *state = S;
   __syncthreads();
   for (int i = threadIdx.x; i < n; i += 64) d[i] = dl[i];
   for (int i = threadIdx.x; i < n - 1; i += 64) e[i] = el[i];
 }
 
-// the record stream replayed onto rows 0 .. nrows-1 of Z (ld ldz), one row
-// per thread
+// a stream replayed onto rows 0 .. nrows-1 of Z (ld ldz), one row per lane
 template <class T> __global__ void __launch_bounds__(64) hb_replay_kernel(int nrows, int64_t ldz, const double2* rec,
                                                                          const int* npos, T* Z) {
   const int r = blockIdx.x * 64 + threadIdx.x;
@@ -822,30 +834,41 @@ size_t heev_big_ws_bytes(int n, bool cplx) {
   const size_t es = cplx ? 16 : 8, nn = (size_t)n * n;
   auto seg = [](size_t b) { return (b + 255) / 256 * 256; };
   return 3 * seg(nn * es) + 4 * seg((size_t)n * es) + seg(16 * (size_t)n * es) + 4 * seg(8 * (size_t)n) +
-         seg(4 * (size_t)n) + seg(16 * heev_log_records(n)) + seg(4) + seg(sizeof(StState));
+         seg(4 * (size_t)n) + seg(16 * heev_log_records(n)) + seg(8) + seg(sizeof(StState));
 }
 
 // The QL/QR iteration of one matrix (d, e in device memory, n <= 4096)
 // with its rotations replayed onto rows 0 .. zrows-1 of Z (ld ldz; null:
-// values only) in rounds of at most cap records: the producer thread, then
-// the replay over the whole GPU, until the recurrence is done (the host
-// reads the state record after each round; one round unless a stream
-// fills).  The element operations are those of steqr_kernel.
+// values only).  A round is one launch of hb_round_kernel: the recurrence
+// fills one half of the record buffer (at most n^2 / 8 records, a tenth of a
+// typical stream, so that little of the replay is left after it) while the
+// other half's records are replayed; the host reads the state record after
+// each, and the last stream is replayed by a launch without the recurrence.
+// The element operations are those of steqr_kernel.  npos: two ints.
 template <class T> static hipError_t st_rounds(int n, int maxsweeps, double* d, double* e, T* Z, int zrows,
                                                int64_t ldz, double2* rec, int cap, int* npos, StState* state,
                                                int* info, int* sweeps, hipStream_t s) {
   const bool wantz = Z != nullptr && zrows > 0;
-  cap = std::max(cap, n + 2);  // room for any one step: every round progresses
+  // every round has room for any one step, so that it progresses
+  const int half = std::max(std::min(cap / 2, n * n / 8), n + 2);
+  const int nb = (zrows + 63) / 64;
+  const size_t lds = 16 * (size_t)n;
+  (void)hipFuncSetAttribute((const void*)hb_round_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   for (int round = 0;; ++round) {
-    hipLaunchKernelGGL(hb_produce_kernel, dim3(1), dim3(64), 16 * (size_t)n, s, n, maxsweeps, d, e,
-                       wantz ? rec : nullptr, cap, npos, state, round > 0 ? 1 : 0);
+    const int cur = round & 1;
+    double2* mine = wantz ? rec + (size_t)cur * half : nullptr;
+    const double2* prev = rec + (size_t)(cur ^ 1) * half;
+    hipLaunchKernelGGL(hb_round_kernel<T>, dim3(round > 0 ? 1 + nb : 1), dim3(64), lds, s, n, maxsweeps, d, e, mine,
+                       half, npos + cur, state, round > 0 ? 1 : 0, zrows, ldz, prev, npos + (cur ^ 1), Z);
     if (!wantz) break;
-    hipLaunchKernelGGL(hb_replay_kernel<T>, dim3((zrows + 63) / 64), dim3(64), 0, s, zrows, ldz, rec, npos, Z);
     StState hs;
     hipError_t e2 = hipMemcpyAsync(&hs, state, sizeof hs, hipMemcpyDeviceToHost, s);
     if (e2 == hipSuccess) e2 = hipStreamSynchronize(s);
     if (e2 != hipSuccess) return e2;
-    if (hs.done) break;
+    if (hs.done) {
+      hipLaunchKernelGGL(hb_replay_kernel<T>, dim3(nb), dim3(64), 0, s, zrows, ldz, mine, npos + cur, Z);
+      break;
+    }
   }
   hipLaunchKernelGGL(hb_info_kernel, dim3(1), dim3(64), 0, s, state, info, sweeps);
   return hipGetLastError();
@@ -909,7 +932,7 @@ template <class T> static hipError_t launch_heev_big_t(const HeevArgs& a, bool c
   const int cap = (a.logcap > 0 && (size_t)a.logcap <= heev_log_records(n)) ? a.logcap : (int)heev_log_records(n);
   p += seg(16 * heev_log_records(n));
   int* npos = reinterpret_cast<int*>(p);
-  p += seg(4);
+  p += seg(8);
   StState* state = reinterpret_cast<StState*>(p);
   const bool wantz = a.Z != nullptr;
   for (int b = 0; b < a.count; ++b) {

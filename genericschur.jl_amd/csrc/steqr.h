@@ -85,6 +85,41 @@ GS_DEV void givens_re(double f, double g, double& cs, double& sn, double& r) {
   }
 }
 
+// givens_re for the recurrence's rotations, whose chain of a square root and
+// a division is what bounds it, for |f| and |g| in [2^-480, 2^480], where no
+// scaling applies: the square root and the quotients from one reciprocal
+// square root estimate y (to 2^-24), one coupled Newton step (s, h) ->
+// sqrt(x), 1 / (2 sqrt(x)) to 2^-47, then for the root and for each quotient
+// one correction by its exact residual (P. Markstein, IBM J. Res. Dev. 34(1),
+// 1990): s + h (x - s^2), q + 2h (f - r q).  The corrected values are within
+// 2^-94 before they are rounded, so they are the correctly rounded ones but
+// for about one operand in 2^40 (none of 2.1e9 random pairs differed from
+// sqrt and / in any of the three).
+GS_DEV void givens_mid(double f, double g, double& cs, double& sn, double& r) {
+#pragma clang fp contract(off)
+  // the sign fix when |f| > |g| and cs = f / r < 0
+  const bool flip = (fabs(f) > fabs(g)) & (f < 0.0);
+  const double f1 = flip ? -f : f, g1 = flip ? -g : g;
+  const double x = f * f + g * g;
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double e = __builtin_fma(-s, h, 0.5);
+  s = __builtin_fma(s, e, s);
+  h = __builtin_fma(h, e, h);
+  const double yy = h + h;
+  const double q = f1 * yy, p = g1 * yy;
+  const double rt = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+  cs = __builtin_fma(__builtin_fma(-rt, q, f1), yy, q);
+  sn = __builtin_fma(__builtin_fma(-rt, p, g1), yy, p);
+  r = flip ? -rt : rt;
+}
+GS_DEV bool givens_mid_range(double lo, double hi) { return (lo >= 0x1p-480) & (hi <= 0x1p480); }
+// either, by the operands
+GS_DEV void givens_any(double f, double g, double& cs, double& sn, double& r) {
+  if (givens_mid_range(fmin(fabs(f), fabs(g)), fmax(fabs(f), fabs(g)))) givens_mid(f, g, cs, sn, r);
+  else givens_re(f, g, cs, sn, r);
+}
+
 // _dgz_sym2x2(a, b, c, wantvec) (symtridiag.jl:375-427; LAPACK xLAEV2)
 GS_DEV void sym2x2(double a, double b, double c, bool wantvec, double& rt1, double& rt2, double& cs1, double& sn1) {
 #pragma clang fp contract(off)
@@ -251,8 +286,10 @@ GS_DEV int st_next_bound(const StState& S) { return S.inblk ? abs(S.lend - S.l) 
 
 // One step of the producer: the set-up of the next unreduced block, one QL
 // or QR iteration, or the end of a block.  d, e: 0-based; D(i) = d[i-1] is
-// the reference's 1-based d[i].  Rotations go to lg when non-null.
-template <class Log> GS_DEV void st_step(StState& S, StVec d, StVec e, Log* lg) {
+// the reference's 1-based d[i].  Rotations go to lg when non-null.  COOP: the
+// 64 lanes of a wavefront call together with the same state (each does every
+// step, storing the same values to the same places) and share the searches.
+template <bool COOP, class Log> GS_DEV void st_step(StState& S, StVec d, StVec e, Log* lg) {
 #pragma clang fp contract(off)
   const int n = S.n;
   const double eps = GS_EPS, eps2 = GS_EPS * GS_EPS, safmin = GS_FMIN;
@@ -339,8 +376,10 @@ template <class Log> GS_DEV void st_step(StState& S, StVec d, StVec e, Log* lg) 
   // end) and _st_QRIter! (dir = -1) loop bodies as one: the two are mirror
   // images, with the same operations on mirrored indices, so lanes of a
   // wavefront in either iteration share the path.
-  const int l = S.l, lend = S.lend;
-  const int dir = S.ql ? 1 : -1;
+  // (COOP: the indices as scalars)
+  auto uni = [](int v) { return COOP ? __builtin_amdgcn_readfirstlane(v) : v; };
+  const int l = uni(S.l), lend = uni(S.lend);
+  const int dir = uni(S.ql ? 1 : -1);
   const bool wantz = lg != nullptr;
   // search for a small off-diagonal entry: pairs (m, m + dir), e index
   // m (QL) or m - 1 (QR)
@@ -351,7 +390,18 @@ template <class Log> GS_DEV void st_step(StState& S, StVec d, StVec e, Log* lg) 
     return E(em) * E(em) <= (eps2 * fabs(D(m))) * fabs(D(m + dir)) + safmin;
   };
   int msplit = lend;
-  {
+  if constexpr (COOP) {
+    const int lane = threadIdx.x & 63;
+    const int len = dir > 0 ? lend - l : l - lend;
+    for (int t = 0; t < len; t += 64) {
+      const bool hit = t + lane < len && small(l + dir * (t + lane));
+      const unsigned long long b = __builtin_amdgcn_ballot_w64(hit);
+      if (b) {
+        msplit = l + dir * (t + __builtin_ctzll(b));
+        break;
+      }
+    }
+  } else {
     const int len = dir > 0 ? lend - l : l - lend;
     int t = 0;
     for (; t + 4 <= len; t += 4) {
@@ -401,18 +451,107 @@ template <class Log> GS_DEV void st_step(StState& S, StVec d, StVec e, Log* lg) 
     p = 0.0;
     // rotations j = j0, j0 - dir, ..., j1 on pairs (j, j + 1): QL updates
     // d[j + 1] against d[j], QR d[j] against d[j + 1]
-    const int j0 = dir > 0 ? msplit - 1 : msplit;
-    const int cnt = dir > 0 ? msplit - l : l - msplit;
+    const int j0 = uni(dir > 0 ? msplit - 1 : msplit);
+    const int cnt = uni(dir > 0 ? msplit - l : l - msplit);
     const int r0 = wantz ? lg->begin() : 0;
+    const int u0 = dir > 0 ? j0 + 1 : j0;  // rotation k: e[j0 - dir k], d[u0 - dir k], d[u0 - dir (k + 1)]
+    int k = 0;
+    if constexpr (COOP) {
+      // Four rotations at a time as straight-line code, the next four's
+      // entries loaded meanwhile; one branch per group where some operand
+      // left givens_mid's range, which redoes the group with givens_any.
+      constexpr int G = 4;
+      const int lane = threadIdx.x & 63;
+      double en[G], dn[G], dc = D(u0);
+      auto load = [&](int k1) {
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+          const int kk = min(k1 + i, cnt - 1);
+          en[i] = E(j0 - dir * kk);
+          dn[i] = D(u0 - dir * (kk + 1));
+        }
+      };
+      if (cnt >= G) load(0);
+      for (; k + G <= cnt; k += G) {
+        double ek[G], dk[G + 1], er[G], dd[G], cc[G], ss[G];
+        dk[0] = dc;
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+          ek[i] = en[i];
+          dk[i + 1] = dn[i];
+        }
+        dc = dn[G - 1];
+        load(k + G);
+        const double gs = g, ps = p, cs0 = c, ss0 = s;
+        double lo = 1.0, hi = 1.0;
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+          const double f = s * ek[i];
+          const double b = c * ek[i];
+          lo = fmin(lo, fmin(fabs(f), fabs(g)));
+          hi = fmax(hi, fmax(fabs(f), fabs(g)));
+          givens_mid(g, f, c, s, er[i]);
+          g = dk[i] - p;
+          r = (dk[i + 1] - g) * s + 2.0 * c * b;
+          p = s * r;
+          dd[i] = g + p;
+          g = c * r - b;
+          cc[i] = c;
+          ss[i] = s;
+        }
+        if (!wave_any(givens_mid_range(lo, hi))) {
+          g = gs;
+          p = ps;
+          c = cs0;
+          s = ss0;
+#pragma unroll 1
+          for (int i = 0; i < G; ++i) {
+            double e1 = ek[0], d0 = dk[0], d1 = dk[1], r1, d2;
+#pragma unroll
+            for (int q = 1; q < G; ++q) {
+              e1 = i == q ? ek[q] : e1;
+              d0 = i == q ? dk[q] : d0;
+              d1 = i == q ? dk[q + 1] : d1;
+            }
+            const double f = s * e1;
+            const double b = c * e1;
+            givens_any(g, f, c, s, r1);
+            g = d0 - p;
+            r = (d1 - g) * s + 2.0 * c * b;
+            p = s * r;
+            d2 = g + p;
+            g = c * r - b;
+#pragma unroll
+            for (int q = 0; q < G; ++q)
+              if (i == q) {
+                er[q] = r1;
+                dd[q] = d2;
+                cc[q] = c;
+                ss[q] = s;
+              }
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+          const int jj = j0 - dir * (k + i);
+          if (i > 0 || k > 0) E(jj + dir) = er[i];
+          D(u0 - dir * (k + i)) = dd[i];
+        }
+        if (wantz && lane == 0) {
+#pragma unroll
+          for (int i = 0; i < G; ++i) lg->put(r0, k + i, cc[i], dir > 0 ? -ss[i] : ss[i]);
+        }
+      }
+    }
     // the entries of rotation k + 1 (e[jj - dir], d[up - dir], d[far - dir])
     // are loaded during rotation k, which writes only e[jj + dir], d[up]
     double ej = 0.0, dup = 0.0, dfar = 0.0;
-    if (cnt > 0) {
-      ej = E(j0);
-      dup = D(dir > 0 ? j0 + 1 : j0);
-      dfar = D(dir > 0 ? j0 : j0 + 1);
+    if (k < cnt) {
+      ej = E(j0 - dir * k);
+      dup = D(u0 - dir * k);
+      dfar = D(u0 - dir * (k + 1));
     }
-    for (int k = 0; k < cnt; ++k) {
+    for (; k < cnt; ++k) {
       const int jj = j0 - dir * k;
       const int up = dir > 0 ? jj + 1 : jj, far = dir > 0 ? jj : jj + 1;
       const double ek = ej, dupk = dup, dfark = dfar;
@@ -423,7 +562,7 @@ template <class Log> GS_DEV void st_step(StState& S, StVec d, StVec e, Log* lg) 
       }
       const double f = s * ek;
       const double b = c * ek;
-      givens_re(g, f, c, s, r);
+      givens_any(g, f, c, s, r);
       if (k > 0) E(jj + dir) = r;
       g = dupk - p;
       r = (dfark - g) * s + 2.0 * c * b;
@@ -445,10 +584,10 @@ template <class Log> GS_DEV void st_step(StState& S, StVec d, StVec e, Log* lg) 
 
 // Runs the producer until the log cannot take another step's rotations or
 // the recurrence is done.
-template <class Log> GS_DEV void st_produce(StState& S, StVec d, StVec e, Log* lg) {
+template <bool COOP = false, class Log> GS_DEV void st_produce(StState& S, StVec d, StVec e, Log* lg) {
   while (!S.done) {
     if (lg && !lg->room(st_next_bound(S))) break;
-    st_step(S, d, e, lg);
+    st_step<COOP>(S, d, e, lg);
   }
 }
 

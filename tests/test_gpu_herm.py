@@ -369,3 +369,30 @@ def test_wrappers_sortby(gs, kind):
         p = np.vdot(a, b)
         assert abs(abs(p) - np.linalg.norm(a) * np.linalg.norm(b)) <= 1e-8, j
     assert np.abs(A @ V - V * w).max() <= 1e3 * n * EPS * np.abs(A).max() * max(1.0, np.abs(V).max())
+
+
+@pytest.mark.parametrize("kind", ["zeros", "wide", "laplace"])
+@pytest.mark.parametrize("n", [2049, 2054])
+def test_steqr_groups_bitwise(gs, oracle, kind, n):
+    """The recurrence of the large orders takes four rotations at a time and
+    redoes a group with the scaled rotations where an operand leaves the
+    middle range: orders that leave remainders, zero and widely varying
+    entries, bit for bit the oracle's d and Z, with and without Z."""
+    r = np.random.default_rng(75)
+    d, e = r.standard_normal(n), r.standard_normal(n - 1)
+    if kind == "zeros":
+        d[r.random(n) < 0.6] = 0.0
+        e[r.random(n - 1) < 0.01] = 0.0
+    elif kind == "wide":
+        d *= 10.0 ** r.uniform(-170, 0, n)
+        e *= 10.0 ** r.uniform(-170, 0, n - 1)
+    else:
+        d, e = np.full(n, 2.0), np.full(n - 1, -1.0)
+    Z = r.standard_normal((3, n))
+    print(f"case steqr {kind} n={n}", flush=True)
+    wo, zo, info_o, _ = oracle.steqr(d, e, Z)
+    wg, zg, _, info_g = gs.steqr_(d, e, Z)
+    assert info_g == info_o == 0
+    assert np.array_equal(wg, wo) and np.array_equal(zg, zo)
+    wv, _, _, _ = gs.steqr_(d, e, None)
+    assert np.array_equal(wv, wo)
