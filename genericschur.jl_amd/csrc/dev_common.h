@@ -572,13 +572,26 @@ template <int NT> GS_DEV void bsync_full() {
 
 // The right update of a pair (x0, x1) by a logged complex reflector,
 // ss = tau1 x0 + tau2 x1, x0 -= ss, x1 -= ss conj(v2) with tau2 = Re(tau1 v2)
-// (GenericSchur.jl:447-460), and a complex product, with a fixed rounding:
-// no contraction beyond the fma calls written here.  Every path that applies
-// a reflector or a scaling to Z (in place during the sweeps, or replayed
-// from the Z log) goes through these, so the paths give the same bits.
+// (GenericSchur.jl:447-460), the left one, ss = conj(tau1) x0 + tau2 x1,
+// x0 -= ss, x1 -= ss v2 (:437-446), and a complex product, with a fixed
+// rounding: no contraction beyond the fma calls written here.  Every path
+// that applies a reflector or a scaling to Z (in place during the sweeps, or
+// replayed from the Z log), and the windowed and LDS-resident sweeps on H, go
+// through these, so the paths give the same bits.
+GS_DEV double ztau2_fixed(zd tau1, zd v2) {
+#pragma clang fp contract(off)
+  return fma(tau1.x, v2.x, -(tau1.y * v2.y));
+}
+GS_DEV void zrot_left_fixed(zd& x0, zd& x1, zd tau1, zd v2, double tau2) {
+#pragma clang fp contract(off)
+  const double sr = fma(tau1.x, x0.x, fma(tau1.y, x0.y, tau2 * x1.x));
+  const double si = fma(tau1.x, x0.y, fma(-tau1.y, x0.x, tau2 * x1.y));
+  x0 = zmk(x0.x - sr, x0.y - si);
+  x1 = zmk(fma(-sr, v2.x, fma(si, v2.y, x1.x)), fma(-sr, v2.y, fma(-si, v2.x, x1.y)));
+}
 GS_DEV void zrot_right_fixed(zd& x0, zd& x1, zd tau1, zd v2) {
 #pragma clang fp contract(off)
-  const double tau2 = fma(tau1.x, v2.x, -(tau1.y * v2.y));
+  const double tau2 = ztau2_fixed(tau1, v2);
   const double sr = fma(tau1.x, x0.x, fma(-tau1.y, x0.y, tau2 * x1.x));
   const double si = fma(tau1.x, x0.y, fma(tau1.y, x0.x, tau2 * x1.y));
   x0 = zmk(x0.x - sr, x0.y - si);

@@ -520,7 +520,10 @@ GS_DEV void dlog_reserve(DLog& zl, int64_t need, double* Zg, int64_t ldz, int n)
   }
 }
 
-template <bool FAST> GS_DEV void d_sweep_win(double* H, int64_t ld, int n, double* Zg, int64_t ldz, bool wantz,
+// RP > 0: H is the whole matrix in LDS with pitch RP (n < RP, n <= 62): the
+// chase's window is the matrix, a sweep one chunk without window copies and
+// chains; lg then holds the whole sweep after two header entries.
+template <bool FAST, int RP = 0> GS_DEV void d_sweep_win(double* H, int64_t ld, int n, double* Zg, int64_t ldz, bool wantz,
                                             double* win, double* lg, int* redi, zd shift1, zd shift2, int istart,
                                             int iend, int64_t& nstep, DLog* zl) {
   const int lane = threadIdx.x;
@@ -566,6 +569,22 @@ template <bool FAST> GS_DEV void d_sweep_win(double* H, int64_t ld, int n, doubl
     }
   }
   for (int k0 = mx; k0 <= iend - 1;) {
+    if constexpr (RP > 0) {
+      dchase_chunk<RP, FAST>(H, 1, n, mx, iend - 1, mx, istart, iend, v0, v1, v2s, lg + 2);
+      wsync();
+      if (zlg) {
+        for (int i = lane; i < 3 * (iend - mx); i += 64) rec[2 + i] = lg[2 + i];
+      } else if (wantz) {
+        if (lane == 0) {
+          lg[0] = (double)mx;
+          lg[1] = (double)iend;
+        }
+        wsync();
+        for (int row = 1 + lane; row <= n; row += 64) dlog_row(Zg + (row - 1), ldz, lg, need);
+      }
+      wsync();
+      break;
+    }
     const int kend = min(k0 + DKC - 1, iend - 1);
     const int wb = max(k0 - 1, 1), we = min(kend + 3, iend);
     const int W = we - wb + 1;
@@ -600,7 +619,9 @@ template <bool FAST> GS_DEV void d_sweep_win(double* H, int64_t ld, int n, doubl
 
 // ------------------------------------------------------------------------
 // gschur!(H::Hessenberg{<:AbstractFloat}, Z) (GenericSchur.jl:513-699)
-template <int NT, class L, bool FAST, bool WIN = false> GS_DEV int64_t d_qr(double* H, L lay, int n, double* Zg, int64_t ldz, bool wantz,
+// WIN: 0 d_sweep, 1 d_sweep_win, otherwise d_sweep_win resident with pitch
+// WIN (rot: the sweep's log).
+template <int NT, class L, bool FAST, int WIN = 0> GS_DEV int64_t d_qr(double* H, L lay, int n, double* Zg, int64_t ldz, bool wantz,
                                                double* rot, int* redi, zd* Wg, int64_t maxiter, int64_t& nsweep,
                                                int64_t& nstep, DLog* zl = nullptr) {
   const int tid = threadIdx.x;
@@ -708,7 +729,10 @@ template <int NT, class L, bool FAST, bool WIN = false> GS_DEV int64_t d_qr(doub
         }
       }
       nsweep += 1;
-      if constexpr (WIN)
+      if constexpr (WIN > 1)
+        d_sweep_win<FAST, WIN>(H, WIN, n, Zg, ldz, wantz, nullptr, rot, redi, zmk(r1r, r1i), zmk(r2r, r2i), istart,
+                               iend, nstep, zl);
+      else if constexpr (WIN == 1)
         d_sweep_win<FAST>(H, lay.ld, n, Zg, ldz, wantz, rot, rot + DWL * DW, redi, zmk(r1r, r1i), zmk(r2r, r2i),
                           istart, iend, nstep, zl);
       else
@@ -933,12 +957,8 @@ template <int NT> __global__ void __launch_bounds__(NT) dschur_global_kernel(Sin
 
 // Batched kernel 2, windowed form: one wavefront per matrix, H (the T
 // buffer) and Z in HBM, LDS holds the chase window and the chunk's log.
-template <bool FAST> __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) dqrw_kernel(BatchArgs a) {
-  __shared__ double win[DWL * DW + 3 * DKC];
-  __shared__ int redi[2];
-  const int b = blockIdx.x;
-  if (b >= a.count) return;
-  const int m = a.order[a.first + b];
+// RP > 0: H resident in LDS at hs with pitch RP.
+template <bool FAST, int RP> GS_DEV void dqrw_matrix(const BatchArgs& a, int m, double* win, int* redi, double* hs) {
   const int n = a.n[m];
   if (a.zlog && threadIdx.x == 0) a.llen[m] = 0;
   if (n <= 0) return;
@@ -956,8 +976,18 @@ template <bool FAST> __global__ void __launch_bounds__(64) __attribute__((amdgpu
     zl.g = a.zlog + a.loff[m];
     zl.cap = a.loff[m + 1] - a.loff[m];
   }
-  const int64_t st = d_qr<64, FullLayout, FAST, true>(T, lay, n, Z, (int64_t)n, wantz, win, redi, W, maxiter, nsweep,
-                                                      nstep, &zl);
+  int64_t st;
+  const FullLayout rlay{RP};
+  if constexpr (RP > 0) {
+    for (int e = threadIdx.x; e < n * n; e += 64) {
+      const int c = e / n, r = e - c * n;
+      hs[r + c * RP] = T[e];
+    }
+    __syncthreads();
+    st = d_qr<64, FullLayout, FAST, RP>(hs, rlay, n, Z, (int64_t)n, wantz, win, redi, W, maxiter, nsweep, nstep, &zl);
+  } else {
+    st = d_qr<64, FullLayout, FAST, 1>(T, lay, n, Z, (int64_t)n, wantz, win, redi, W, maxiter, nsweep, nstep, &zl);
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
     if (zl.g) a.llen[m] = zl.pos;
@@ -967,11 +997,61 @@ template <bool FAST> __global__ void __launch_bounds__(64) __attribute__((amdgpu
     }
     a.info[m] = (int32_t)(st > 0x7fffffff ? 0x7fffffff : st);
   }
-  if (st != 0) return;
-  d_finish<64>(T, lay, n, T, (int64_t)n, W, a.scl[2 * m], a.scl[2 * m + 1]);
+  if (st != 0) {  // not converged: T is what the sweeps have made of it
+    if constexpr (RP > 0)
+      for (int e = threadIdx.x; e < n * n; e += 64) {
+        const int c = e / n, r = e - c * n;
+        T[e] = hs[r + c * RP];
+      }
+    return;
+  }
+  if constexpr (RP > 0) d_finish<64>(hs, rlay, n, T, (int64_t)n, W, a.scl[2 * m], a.scl[2 * m + 1]);
+  else d_finish<64>(T, lay, n, T, (int64_t)n, W, a.scl[2 * m], a.scl[2 * m + 1]);
 }
 
-hipError_t launch_dqrw(const BatchArgs& a, hipStream_t s) {
+template <bool FAST> __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) dqrw_kernel(BatchArgs a) {
+  __shared__ double win[DWL * DW + 3 * DKC];
+  __shared__ int redi[2];
+  dqrw_matrix<FAST, 0>(a, a.order[a.first + blockIdx.x], win, redi, nullptr);
+}
+
+// Orders below RP with H whole in LDS: a sweep is one chase over the matrix,
+// with no window copies and no chains through memory.  Bound by the chase's
+// chain of dependent double operations.  Measured against the windowed
+// kernel: one matrix n = 13 0.29 / 0.38 ms per call, n = 24 0.62 / 0.87,
+// n = 60 2.29 / 3.49; 1000 matrices n = 4..24 0.64 / 0.88 ms, 16384 n = 4..32
+// 2.98 / 4.05, 2000 n = 49..62 4.6 / 5.1.
+template <bool FAST, int RP> __global__ void __launch_bounds__(64) dqrr_kernel(BatchArgs a) {
+  __shared__ double hs[RP * (RP - 1)];
+  __shared__ double lg[3 * RP + 2];
+  __shared__ int redi[2];
+  dqrw_matrix<FAST, RP>(a, a.order[a.first + blockIdx.x], lg, redi, hs);
+}
+
+template <bool FAST> static void launch_dqrr(const BatchArgs& a, int nmax, hipStream_t s) {
+  if (nmax <= 16) hipLaunchKernelGGL((dqrr_kernel<FAST, 17>), dim3(a.count), dim3(64), 0, s, a);
+  else if (nmax <= 32) hipLaunchKernelGGL((dqrr_kernel<FAST, 33>), dim3(a.count), dim3(64), 0, s, a);
+  else if (nmax <= 48) hipLaunchKernelGGL((dqrr_kernel<FAST, 49>), dim3(a.count), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL((dqrr_kernel<FAST, 63>), dim3(a.count), dim3(64), 0, s, a);
+}
+
+// The chase has one lane per row and column of the matrix and two to spare.
+int dqr_res_max_n() { return 62; }
+// Largest launch of the widest resident class: its LDS holds five matrices to
+// a CU where the windowed kernel holds more, so a large enough batch runs
+// faster windowed (n = 49..62, QR alone: 4000 matrices 6.4 resident against
+// 6.8 ms, 8000 12.7 against 11.4; n = 33..62: 3000 3.75 either way, 6500 8.3
+// against 7.4).  The narrower classes stay ahead (8000 n = 33..48 4.5 against
+// 6.1 ms).
+constexpr int kResWideCount = 4096;
+
+hipError_t launch_dqrw(const BatchArgs& a, int nmax, hipStream_t s) {
+  if (a.count <= 0) return hipSuccess;
+  if (nmax <= 48 || (nmax <= dqr_res_max_n() && a.count <= kResWideCount)) {
+    if (a.flags & 0x1000) launch_dqrr<false>(a, nmax, s);
+    else launch_dqrr<true>(a, nmax, s);
+    return hipGetLastError();
+  }
   if (a.flags & 0x1000)
     hipLaunchKernelGGL((dqrw_kernel<false>), dim3(a.count), dim3(64), 0, s, a);
   else

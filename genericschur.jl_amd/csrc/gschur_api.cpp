@@ -389,10 +389,12 @@ static void plan_bins(const Tuning& tn, bool cplx, int64_t count, const int32_t*
     w += n[i];
   }
   const int bw = bin_width(tn, cplx);
-  const int nb = (nmax_lds + bw - 1) / bw + 1;
+  // no bin holds orders on both sides of the LDS-resident QR kernels' limit
+  const int nres = cplx ? zqr_res_max_n() : dqr_res_max_n();
+  const int nb = (nmax_lds + bw - 1) / bw + 2;
   std::vector<std::vector<int32_t>> byb(nb);
   for (int64_t i = 0; i < count; ++i) {
-    const int b = n[i] <= 0 ? 0 : (n[i] - 1) / bw;
+    const int b = n[i] <= 0 ? 0 : (n[i] - 1) / bw + (n[i] > nres ? 1 : 0);
     byb[b].push_back((int32_t)i);
   }
   for (int b = nb - 1; b >= 0; --b) {
@@ -488,15 +490,13 @@ static int build_plan(gs_handle* h, bool cplx, int64_t count, const int32_t* n, 
   return GS_OK;
 }
 
-// Bin orders whose QR launch logs its Z updates (the bin's largest order is
-// at least the minimum).  Measured with each launch alone, QR + replay against
-// in place: complex n = 4..24 (1000 matrices) 1.29 against 1.25 ms, and with
+// The largest real order whose QR launch logs its Z updates; complex bins log
+// at every order.  Measured with each launch alone, QR + replay against in
+// place: complex n = 4..24 (1000 matrices) 0.83 against 0.90 ms, and with
 // every larger order of 8192 matrices n ~ U{8..96} in place up to 72 the batch
-// takes 56.3 ms, with the log from 25 up 50.9 ms; real n = 4..24 0.72 against
-// 0.79 ms, n = 16..32 1.14 against 1.23 ms, n = 129..141 (1000 matrices, the
-// replay's row no longer fits the registers) 30.6 against 30.2 ms.
-constexpr int kZlogMinN = 25;
-constexpr int kDlogMinN = 2;
+// takes 56.3 ms, with the log 50.4 ms; real n = 4..24 0.72 against 0.79 ms,
+// n = 16..32 1.14 against 1.23 ms, n = 129..141 (1000 matrices, the replay's
+// row no longer fits the registers) 30.6 against 30.2 ms.
 constexpr int kDlogMaxN = 128;
 
 // Whether the batched QR launches of this call log their Z updates
@@ -508,7 +508,17 @@ static bool bin_zlog(bool cplx, const Bin& b, int kflags) {
   if (!cplx && b.nmax > kDlogMaxN) return false;
   if (kflags & GS_ZLOG_TINY) return true;
   if (b.zlog >= 0) return b.zlog == 1;
-  return b.nmax >= (cplx ? kZlogMinN : kDlogMinN);
+  return b.nmax >= 2;
+}
+
+// Whether a complex plan's QR iterations run as one work-queue launch: not
+// where every order fits the LDS-resident kernels (one QR launch per bin;
+// 16384 matrices n = 4..24 3.8 against 6.9 ms, n = 33..48 34.3 against 39.7).
+// A plan with larger orders queues the small ones too: they fill the queue's
+// tail (2500 matrices n = 24..60 8.5 ms; those up to 48 in resident launches
+// beside the queue 11.2, the 8192 of n = 8..96 50.4 against 53.6).
+static bool plan_queue(const Tuning& t, bool cplx, const std::vector<Bin>& bins) {
+  return qr_queue(t, cplx) && !bins.empty() && bins[0].nmax > zqr_res_max_n();
 }
 
 // Work-queue form of a complex batch (tuning queue = 1): the bins'
@@ -633,7 +643,7 @@ static hipError_t launch_plan(gs_handle* h, const PlanDev& pd, const double* A, 
   // kBranches streams, so the LDS left free by a large bin's workgroups is
   // filled by the smaller bins' workgroups
   const Tuning& tn = h->tune[p->is_complex ? 1 : 0];
-  if (pd.qctr && !(flags & GS_QR_BAND) && qr_queue(tn, p->is_complex))
+  if (pd.qctr && !(flags & GS_QR_BAND) && plan_queue(tn, p->is_complex, *pd.bins))
     return launch_plan_queue(h, pd, a, flags, zl ? zlog : nullptr, timed, tn);
   hipError_t e = hipEventRecord(h->evfork, h->stream);
   if (e != hipSuccess) return e;
@@ -682,7 +692,7 @@ static hipError_t launch_plan(gs_handle* h, const PlanDev& pd, const double* A, 
     if (flags & GS_QR_BAND)
       e = p->is_complex ? launch_zqr(a, b.nmax, b.nt_qr, s) : launch_dqr(a, b.nmax, b.nt_qr, s);
     else
-      e = p->is_complex ? launch_zqrw(a, s) : launch_dqrw(a, s);
+      e = p->is_complex ? launch_zqrw(a, b.nmax, s) : launch_dqrw(a, b.nmax, s);
     if (e != hipSuccess) return e;
     if (timed && (e = hipEventRecord(h->tev[6 * bi + 3], s)) != hipSuccess) return e;
     if (timed && (e = hipEventRecord(h->tev[6 * bi + 4], s)) != hipSuccess) return e;
@@ -716,7 +726,7 @@ static int run_timed(gs_handle* h, Plan* p, const double* A, double* T, double* 
   // the work-queue form: one QR record for the whole batch, and the Z-log
   // replays of the bins at or above the smallest logging order
   const Tuning& tn = h->tune[p->is_complex ? 1 : 0];
-  const bool queue = !(kflags & GS_QR_BAND) && qr_queue(tn, p->is_complex);
+  const bool queue = !(kflags & GS_QR_BAND) && plan_queue(tn, p->is_complex, p->bins);
   const int zmin = queue ? queue_zmin(p->bins, zlog && uses_zlog(kflags), p->is_complex, kflags) : (1 << 30);
   auto put = [&](int kind, int nmin, int nmax, int64_t cnt, double work, hipEvent_t e0, hipEvent_t e1) -> int {
     float ms = 0.f;
@@ -1081,12 +1091,19 @@ static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda
     if (le != hipSuccess)
       return fail_hip(h, le, h->large_where.empty() ? "large path" : ("large path: " + h->large_where).c_str());
   } else if (use_lds) {
-    HIPCHK(h, h->bMeta.ensure(64));
-    // metadata for a batch of one: order = 0, n, off = 0, woff = 0
+    HIPCHK(h, h->bMeta.ensure(128));
+    // the LDS-resident QR kernels log Z's updates (in place they would wait
+    // for memory at every sweep); above, Z is updated in place
+    const bool zlg = uses_zlog(kflags) && n <= (cplx ? zqr_res_max_n() : dqr_res_max_n());
+    const bool tiny = (kflags & GS_ZLOG_TINY) != 0;
+    const int64_t lcap = !zlg ? 0 : cplx ? zlog_capacity((int)n, tiny) : dlog_capacity((int)n, tiny);
+    if (zlg) HIPCHK(h, h->bLog.ensure(es * (size_t)lcap));
+    // metadata for a batch of one: order = 0, n, off = 0, woff = 0, the log
     struct Meta {
       int32_t order, n;
       int64_t off, woff;
-    } meta = {0, (int32_t)n, 0, 0};
+      int64_t loff[2], llen;
+    } meta = {0, (int32_t)n, 0, 0, {0, lcap}, 0};
     HIPCHK(h, hipMemcpyAsync(h->bMeta.p, &meta, sizeof meta, hipMemcpyHostToDevice, h->stream));
     char* mp = static_cast<char*>(h->bMeta.p);
     BatchArgs a;
@@ -1106,16 +1123,17 @@ static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda
     a.flags = kflags;
     a.maxiter = maxiter;
     a.maxinner = maxinner;
-    a.zlog = nullptr;  // one matrix: Z updated in place
-    a.loff = nullptr;
-    a.llen = nullptr;
+    a.zlog = zlg ? static_cast<double*>(h->bLog.p) : nullptr;
+    a.loff = reinterpret_cast<const int64_t*>(mp + offsetof(Meta, loff));
+    a.llen = reinterpret_cast<int64_t*>(mp + offsetof(Meta, llen));
     const int nthq = bin_nt_hq(h->tune[cplx ? 1 : 0], cplx, (int)n), ntqr = default_nt_qr(cplx, (int)n);
     le = cplx ? launch_zhq(a, (int)n, nthq, h->stream) : launch_dhq(a, (int)n, nthq, h->stream);
     if (le == hipSuccess) {
       if (kflags & GS_QR_BAND)
         le = cplx ? launch_zqr(a, (int)n, ntqr, h->stream) : launch_dqr(a, (int)n, ntqr, h->stream);
       else
-        le = cplx ? launch_zqrw(a, h->stream) : launch_dqrw(a, h->stream);
+        le = cplx ? launch_zqrw(a, (int)n, h->stream) : launch_dqrw(a, (int)n, h->stream);
+      if (le == hipSuccess && zlg) le = cplx ? launch_zlog(a, (int)n, h->stream) : launch_dlog(a, (int)n, h->stream);
     }
   } else if (use_win) {
     HIPCHK(h, h->bMeta.ensure(128));

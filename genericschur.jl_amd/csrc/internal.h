@@ -72,8 +72,12 @@ int dschur_max_lds_n();
 
 hipError_t launch_zhq(const BatchArgs& a, int nmax, int nt, hipStream_t s);
 hipError_t launch_zqr(const BatchArgs& a, int nmax, int nt, hipStream_t s);
-// windowed QR launch: one wavefront per matrix, H and Z in HBM
-hipError_t launch_zqrw(const BatchArgs& a, hipStream_t s);
+// QR launch of matrices of order at most nmax: up to z/dqr_res_max_n() one
+// wavefront per matrix with H in LDS, above windowed with H and Z in HBM (a
+// launch's matrices all on one side of that order)
+int zqr_res_max_n();
+int dqr_res_max_n();
+hipError_t launch_zqrw(const BatchArgs& a, int nmax, hipStream_t s);
 // The persistent form of launch_zqrw: `slots` workgroups take the matrices
 // order[first .. first + count) from the work queue a.qctr, in order.
 hipError_t launch_zqrw_queue(const BatchArgs& a, int slots, hipStream_t s);
@@ -86,7 +90,7 @@ inline int64_t zlog_capacity(int n, bool tiny) {
   const int64_t one_sweep = 3 + 2 * (int64_t)n;
   return tiny ? one_sweep : 6 * (int64_t)n * n + 16 * (int64_t)n + 64;
 }
-hipError_t launch_dqrw(const BatchArgs& a, hipStream_t s);
+hipError_t launch_dqrw(const BatchArgs& a, int nmax, hipStream_t s);
 hipError_t launch_dlog(const BatchArgs& a, int nmax, hipStream_t s);
 // Real Z-log capacity of one matrix of order n, in doubles (tiny: one sweep
 // and one rotation, the least the kernel accepts)

@@ -588,18 +588,11 @@ template <bool LEFT> GS_DEV void zchain(zd* p, int64_t st, const zd* lg, int ka,
       const int q = g * ZCG + i;
       if (q < s) {
         const zd tau1 = lgq[2 * q], v2 = lgq[2 * q + 1];
-        const double tau2 = (tau1 * v2).x;
-        const zd a = x[q], b = x[q + 1];
-        if (LEFT) {
-          const zd ss = zconj(tau1) * a + tau2 * b;
-          x[q] = a - ss;
-          x[q + 1] = b - ss * v2;
-        } else {
-          zd x0 = a, x1 = b;
-          zrot_right_fixed(x0, x1, tau1, v2);
-          x[q] = x0;
-          x[q + 1] = x1;
-        }
+        zd x0 = x[q], x1 = x[q + 1];
+        if (LEFT) zrot_left_fixed(x0, x1, tau1, v2, ztau2_fixed(tau1, v2));
+        else zrot_right_fixed(x0, x1, tau1, v2);
+        x[q] = x0;
+        x[q + 1] = x1;
       }
     }
 #pragma unroll
@@ -640,11 +633,7 @@ template <bool TAIL = true> GS_DEV void zchain_full(zd* p, const zd* lg, int ka,
       const int q = g * ZCG + i;
       if (q < S) {
         const zd tau1 = lgq[2 * q], v2 = lgq[2 * q + 1];
-        const double tau2 = (tau1 * v2).x;
-        const zd a = x[q], b = x[q + 1];
-        const zd ss = zconj(tau1) * a + tau2 * b;
-        x[q] = a - ss;
-        x[q + 1] = b - ss * v2;
+        zrot_left_fixed(x[q], x[q + 1], tau1, v2, ztau2_fixed(tau1, v2));
       }
     }
 #pragma unroll
@@ -741,16 +730,13 @@ GS_DEV void zlog_row(zd* row, int64_t st, const zd* __restrict__ lg, int64_t len
   }
 }
 
-template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, int n, zd* Zg, int64_t ldz, bool wantz, zd* win,
-                                             zd* lgbuf, int* redi, zd shift, int istart, int iend, int64_t& nstep,
-                                             ZLog& zl) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int CS = NT - 64;  // threads of the chain wavefronts
-  const int cw = tid - 64;
+// Start row of a sweep (GenericSchur.jl:391-423: two consecutive small
+// subdiagonal entries) and its first reflector's input.
+template <int NT, class L> GS_DEV int z_sweep_start(zd* H, L lay, int* redi, zd shift, int istart, int iend, zd& v0,
+                                                    zd& v1) {
   const double ulp = GS_EPS;
-  const FullLayout lay{ld};
   int found = -1;
-  for (int mm = iend - 1 - tid; mm >= istart + 1; mm -= NT) {
+  for (int mm = iend - 1 - (int)threadIdx.x; mm >= istart + 1; mm -= NT) {
     const zd h11 = HH(mm, mm);
     const zd h22 = HH(mm + 1, mm + 1);
     zd h11s = h11 - shift;
@@ -766,17 +752,187 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
   }
   found = block_max_int<NT>(found, redi);
   const int istart1 = (found > 0) ? found : istart;
-  zd v0, v1;
-  {
-    const zd h11 = HH(istart1, istart1);
-    zd h11s = h11 - shift;
-    double h21 = HH(istart1 + 1, istart1).x;
-    const double s = zabs1(h11s) + fabs(h21);
-    h11s = h11s / s;
-    h21 = h21 / s;
-    v0 = h11s;
-    v1 = zr(h21);
+  const zd h11 = HH(istart1, istart1);
+  zd h11s = h11 - shift;
+  double h21 = HH(istart1 + 1, istart1).x;
+  const double s = zabs1(h11s) + fabs(h21);
+  v0 = h11s / s;
+  v1 = zr(h21 / s);
+  return istart1;
+}
+
+// The bulge chase of steps k0 .. kend of a sweep (GenericSchur.jl:437-460)
+// on a window of H in LDS (rows and columns wb .. we, entry (r, c) at
+// win[(r - wb) + (c - wb) WP]) by one wavefront; step k's (tau1, v2) go to
+// lg[2 (k - k0)].  v0, v1: the sweep's first reflector input, used when k0 ==
+// istart1.  dmy: WP + 1 entries that idle lanes store to.
+template <bool FAST, int WP> GS_DEV void z_chase_chunk(zd* win, int wb, int we, int k0, int kend, int istart1, int iend,
+                                                       zd v0, zd v1, zd* lg, zd* dmy) {
+  const int lane = threadIdx.x & 63;
+  auto WIN = [&](int r, int cc) -> zd& { return win[(r - wb) + (cc - wb) * WP]; };
+  // Step k in lanes: the row pass (rows k, k + 1) on column k + lane;
+  // the column pass (columns k, k + 1) on row k + lane for lanes 0..2
+  // and on row wb + lane - 3 (rows above k) for lanes 3 and up.  All
+  // operands but the column pass's rows k and k + 1 are final before
+  // the step's reflector, so they are loaded first (the wavefront's
+  // LDS accesses complete in order); rows k and k + 1 come from the
+  // row pass's lanes 0 and 1 by a quad permutation, and the next
+  // reflector's inputs from the column pass's lanes 1 and 2, so no LDS
+  // round trip lies between one reflector and the next.  Lanes with
+  // nothing to do load in-window entries and store to a dummy area.
+  const bool hi3 = lane >= 3;
+  const int cidx = hi3 ? lane - 3 : lane;
+  const int laneZ = lane * WP;
+  if (k0 > istart1) {
+    v0 = WIN(k0, k0 - 1);
+    v1 = WIN(k0 + 1, k0 - 1);
   }
+  // the reflector's inputs, the same in every lane: kept in scalar
+  // registers from one step to the next
+  zd nv0 = zmk(rdfirst(v0.x), rdfirst(v0.y)), nv1 = zmk(rdfirst(v1.x), rdfirst(v1.y));
+  zd* wk = &WIN(k0, k0);
+  zd* lgk = lg;
+  double betal = 0.0;  // lane s: beta of step k0 + s
+  for (int k = k0; k <= kend; ++k, wk += WP + 1, lgk += 2) {
+    const int kw = k - wb;
+    const bool rv = lane <= we - k;
+    zd* const rp = wk + (rv ? laneZ : 0);
+    zd ra = rp[0], rb = rp[1];
+    // column pass rows relative to k: lane (lanes 0..2), lane - 3 - kw (3 and up)
+    const bool cv = cidx < (hi3 ? kw : (k + 2 <= iend ? 3 : 2));
+    zd* const cp = wk + (cv ? (hi3 ? cidx - kw : lane) : 0);
+    zd ca = cp[0], cb = cp[WP];
+    v0 = nv0;
+    v1 = nv1;
+    const zd tau1 = FAST ? zreflector2_wave(v0, v1) : zreflector2(v0, v1);
+    const zd v2 = v1;
+    zrot_left_fixed(ra, rb, tau1, v2, ztau2_fixed(tau1, v2));
+    {
+      // lane 0 takes lane 1's (k, k + 1), lane 1 takes lane 0's (k + 1, k)
+      const zd x10 = zmk(qperm<0xF5>(ra.x), qperm<0xF5>(ra.y));
+      const zd x01 = zmk(qperm<0xA0>(rb.x), qperm<0xA0>(rb.y));
+      const bool l0 = lane == 0, l1 = lane == 1;
+      ca = zmk(l0 ? ra.x : (l1 ? x01.x : ca.x), l0 ? ra.y : (l1 ? x01.y : ca.y));
+      cb = zmk(l0 ? x10.x : (l1 ? rb.x : cb.x), l0 ? x10.y : (l1 ? rb.y : cb.y));
+    }
+    zrot_right_fixed(ca, cb, tau1, v2);
+    nv0 = zmk(rdlane(ca.x, 1), rdlane(ca.y, 1));
+    nv1 = zmk(rdlane(ca.x, 2), rdlane(ca.y, 2));
+    zd* const rq = (rv && lane >= 2) ? rp : dmy;
+    rq[0] = ra;
+    rq[1] = rb;
+    zd* const cq = cv ? cp : dmy;
+    cq[0] = ca;
+    cq[WP] = cb;
+    betal = lane == k - k0 ? v0.x : betal;
+    // lane 0: the step's log entry; the other lanes store to the dummy area
+    zd* const lq = lane == 0 ? lgk : dmy;
+    lq[0] = tau1;
+    lq[1] = v2;
+    wsync();
+  }
+  // the annihilated columns: (k, k - 1) = beta, (k + 1, k - 1) = 0 (no
+  // later step of the chunk reads them)
+  {
+    const int k = k0 + lane;
+    if (k <= kend && k > istart1) {
+      WIN(k, k - 1) = zr(betal);
+      WIN(k + 1, k - 1) = zr(0.0);
+    }
+    wsync();
+  }
+}
+
+// singleShiftQR! (GenericSchur.jl:374-504) of a matrix held whole in LDS
+// (H(r, c) at H[(r - 1) + (c - 1) WP], n < WP) by one wavefront: the chase's
+// window is the matrix, so a sweep has no chunks, no window copies and no
+// chains.  rec: 2 WP + 4 entries of LDS for the sweep's Z log record, which
+// is copied to the log, or (zl.g null) applied to Z at once.
+template <bool FAST, int WP> GS_DEV void z_sweep_res(zd* H, int n, zd* Zg, int64_t ldz, bool wantz, zd* rec, zd* dmy,
+                                                     int* redi, zd shift, int istart, int iend, int64_t& nstep,
+                                                     ZLog& zl) {
+  const int lane = threadIdx.x;
+  const FullLayout lay{WP};
+  zd v0, v1;
+  const int istart1 = z_sweep_start<64>(H, lay, redi, shift, istart, iend, v0, v1);
+  const int need = 3 + 2 * (iend - istart1);
+  zd* lg = rec + 2;
+  zd ctt = zr(0.0);
+  int k0 = istart1;
+  if (istart1 > istart) {
+    // the first step, then the phase scaling (GenericSchur.jl:461-482)
+    z_chase_chunk<FAST, WP>(H, 1, n, k0, k0, istart1, iend, v0, v1, lg, dmy);
+    zd t = zr(1.0) - lg[0];
+    t = t / zabs(t);
+    ctt = zconj(t);
+    wsync();
+    if (lane == 0) {
+      HH(istart1 + 1, istart1) = zmul_fixed(HH(istart1 + 1, istart1), ctt);
+      if (istart1 + 2 <= iend) HH(istart1 + 2, istart1 + 1) = zmul_fixed(HH(istart1 + 2, istart1 + 1), t);
+    }
+    wsync();
+    for (int cc = 1; cc <= n; ++cc) {
+      const bool cin = (cc >= istart1 && cc <= iend && cc != istart1 + 1);
+      const int r = 1 + lane;
+      const bool rin = (r >= istart1 && r != istart1 + 1);
+      if (r <= min(cc - 1, iend) && (rin || cin)) {
+        zd x = HH(r, cc);
+        if (rin) x = zmul_fixed(x, t);
+        if (cin) x = zmul_fixed(x, ctt);
+        HH(r, cc) = x;
+      }
+    }
+    wsync();
+    ++k0;
+  }
+  if (k0 <= iend - 1)
+    z_chase_chunk<FAST, WP>(H, 1, n, k0, iend - 1, istart1, iend, v0, v1, lg + 2 * (k0 - istart1), dmy);
+  nstep += iend - istart1;
+  // tail realness (GenericSchur.jl:486-500)
+  zd t = HH(iend, iend - 1);
+  const bool tail = t.y != 0.0;
+  if (tail) {
+    const double rtv = zabs(t);
+    t = t / rtv;
+    const zd ct = zconj(t);
+    wsync();
+    if (lane == 0) HH(iend, iend - 1) = zr(rtv);
+    const int cc = iend + 1 + lane, r = 1 + lane;
+    if (cc <= n) HH(iend, cc) = zmul_fixed(HH(iend, cc), ct);
+    if (r <= iend - 1) HH(r, iend) = zmul_fixed(HH(r, iend), t);
+  }
+  wsync();
+  if (!wantz) return;
+  if (lane == 0) {
+    rec[0] = zmk((double)istart1, (double)iend);
+    rec[1] = ctt;
+    rec[need - 1] = tail ? t : zr(0.0);
+  }
+  wsync();
+  if (!zl.g) {
+    for (int row = 1 + lane; row <= n; row += 64) zlog_row(Zg + (row - 1), ldz, rec, need);
+  } else {
+    if (zl.pos + need > zl.cap) {
+      __syncthreads();
+      for (int row = 1 + lane; row <= n; row += 64) zlog_row(Zg + (row - 1), ldz, zl.g, zl.pos);
+      __syncthreads();
+      zl.pos = 0;
+    }
+    for (int e = lane; e < need; e += 64) zl.g[zl.pos + e] = rec[e];
+    zl.pos += need;
+  }
+  wsync();
+}
+
+template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, int n, zd* Zg, int64_t ldz, bool wantz, zd* win,
+                                             zd* lgbuf, int* redi, zd shift, int istart, int iend, int64_t& nstep,
+                                             ZLog& zl) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int CS = NT - 64;  // threads of the chain wavefronts
+  const int cw = tid - 64;
+  const FullLayout lay{ld};
+  zd v0, v1;
+  const int istart1 = z_sweep_start<NT>(H, lay, redi, shift, istart, iend, v0, v1);
   bool phase_pending = istart1 > istart;
   // Z log: room for this sweep's record, then its header
   const bool zlg = wantz && zl.g;
@@ -831,92 +987,7 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
           __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the window is in LDS
         }
         wsync();
-        auto WIN = [&](int r, int cc) -> zd& { return win[(r - wb) + (cc - wb) * ZWL]; };
-        // Step k in lanes: the row pass (rows k, k + 1) on column k + lane;
-        // the column pass (columns k, k + 1) on row k + lane for lanes 0..2
-        // and on row wb + lane - 3 (rows above k) for lanes 3 and up.  All
-        // operands but the column pass's rows k and k + 1 are final before
-        // the step's reflector, so they are loaded first (the wavefront's
-        // LDS accesses complete in order); rows k and k + 1 come from the
-        // row pass's lanes 0 and 1 by a quad permutation, and the next
-        // reflector's inputs from the column pass's lanes 1 and 2, so no LDS
-        // round trip lies between one reflector and the next.  Lanes with
-        // nothing to do load in-window entries and store to a dummy area.
-        zd* const dmy = lgbuf + 4 * ZKC;
-        const bool hi3 = lane >= 3;
-        const int cidx = hi3 ? lane - 3 : lane;
-        const int laneZ = lane * ZWL;
-        if (k0 > istart1) {
-          v0 = WIN(k0, k0 - 1);
-          v1 = WIN(k0 + 1, k0 - 1);
-        }
-        // the reflector's inputs, the same in every lane: kept in scalar
-        // registers from one step to the next
-        zd nv0 = zmk(rdfirst(v0.x), rdfirst(v0.y)), nv1 = zmk(rdfirst(v1.x), rdfirst(v1.y));
-        zd* wk = &WIN(k0, k0);
-        zd* lgk = lg;
-        double betal = 0.0;  // lane s: beta of step k0 + s
-        for (int k = k0; k <= kend; ++k, wk += ZWL + 1, lgk += 2) {
-          const int kw = k - wb;
-          const bool rv = lane <= we - k;
-          zd* const rp = wk + (rv ? laneZ : 0);
-          zd ra = rp[0], rb = rp[1];
-          // column pass rows relative to k: lane (lanes 0..2), lane - 3 - kw (3 and up)
-          const bool cv = cidx < (hi3 ? kw : (k + 2 <= iend ? 3 : 2));
-          zd* const cp = wk + (cv ? (hi3 ? cidx - kw : lane) : 0);
-          zd ca = cp[0], cb = cp[ZWL];
-          v0 = nv0;
-          v1 = nv1;
-          const zd tau1 = FAST ? zreflector2_wave(v0, v1) : zreflector2(v0, v1);
-          const zd v2 = v1;
-          const double tau2 = tau1.x * v2.x - tau1.y * v2.y;
-          {
-            // ss = conj(tau1) ra + tau2 rb; ra -= ss; rb -= ss v2
-            const double sx = fma(tau1.x, ra.x, fma(tau1.y, ra.y, tau2 * rb.x));
-            const double sy = fma(tau1.x, ra.y, fma(-tau1.y, ra.x, tau2 * rb.y));
-            ra = zmk(ra.x - sx, ra.y - sy);
-            rb = zmk(fma(-sx, v2.x, fma(sy, v2.y, rb.x)), fma(-sx, v2.y, fma(-sy, v2.x, rb.y)));
-          }
-          {
-            // lane 0 takes lane 1's (k, k + 1), lane 1 takes lane 0's (k + 1, k)
-            const zd x10 = zmk(qperm<0xF5>(ra.x), qperm<0xF5>(ra.y));
-            const zd x01 = zmk(qperm<0xA0>(rb.x), qperm<0xA0>(rb.y));
-            const bool l0 = lane == 0, l1 = lane == 1;
-            ca = zmk(l0 ? ra.x : (l1 ? x01.x : ca.x), l0 ? ra.y : (l1 ? x01.y : ca.y));
-            cb = zmk(l0 ? x10.x : (l1 ? rb.x : cb.x), l0 ? x10.y : (l1 ? rb.y : cb.y));
-          }
-          {
-            // ss = tau1 ca + tau2 cb; ca -= ss; cb -= ss conj(v2)
-            const double sx = fma(tau1.x, ca.x, fma(-tau1.y, ca.y, tau2 * cb.x));
-            const double sy = fma(tau1.x, ca.y, fma(tau1.y, ca.x, tau2 * cb.y));
-            ca = zmk(ca.x - sx, ca.y - sy);
-            cb = zmk(fma(-sx, v2.x, fma(-sy, v2.y, cb.x)), fma(-sy, v2.x, fma(sx, v2.y, cb.y)));
-          }
-          nv0 = zmk(rdlane(ca.x, 1), rdlane(ca.y, 1));
-          nv1 = zmk(rdlane(ca.x, 2), rdlane(ca.y, 2));
-          zd* const rq = (rv && lane >= 2) ? rp : dmy;
-          rq[0] = ra;
-          rq[1] = rb;
-          zd* const cq = cv ? cp : dmy;
-          cq[0] = ca;
-          cq[ZWL] = cb;
-          betal = lane == k - k0 ? v0.x : betal;
-          // lane 0: the step's log entry; the other lanes store to the dummy area
-          zd* const lq = lane == 0 ? lgk : dmy;
-          lq[0] = tau1;
-          lq[1] = v2;
-          wsync();
-        }
-        // the annihilated columns: (k, k - 1) = beta, (k + 1, k - 1) = 0 (no
-        // later step of the chunk reads them)
-        {
-          const int k = k0 + lane;
-          if (k <= kend && k > istart1) {
-            WIN(k, k - 1) = zr(betal);
-            WIN(k + 1, k - 1) = zr(0.0);
-          }
-          wsync();
-        }
+        z_chase_chunk<FAST, ZWL>(win, wb, we, k0, kend, istart1, iend, v0, v1, lg, lgbuf + 4 * ZKC);
         win_store<zd, ZW, ZWL>(H + (wb - 1) + (int64_t)(wb - 1) * ld, ld, W, win, lane);
         if (zlg && lane < 2 * (kend - k0 + 1)) rec[2 + 2 * (k0 - istart1) + lane] = lg[lane];
       }
@@ -959,8 +1030,8 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
       t = t / zabs(t);
       const zd ctt = zconj(t);
       if (tid == 0) {
-        HH(istart1 + 1, istart1) = HH(istart1 + 1, istart1) * ctt;
-        if (istart1 + 2 <= iend) HH(istart1 + 2, istart1 + 1) = HH(istart1 + 2, istart1 + 1) * t;
+        HH(istart1 + 1, istart1) = zmul_fixed(HH(istart1 + 1, istart1), ctt);
+        if (istart1 + 2 <= iend) HH(istart1 + 2, istart1 + 1) = zmul_fixed(HH(istart1 + 2, istart1 + 1), t);
       }
       __syncthreads();
       for (int cc = 1; cc <= n; ++cc) {
@@ -970,8 +1041,8 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
           const bool rin = (r >= istart1 && r != istart1 + 1);
           if (!rin && !cin) continue;
           zd x = HH(r, cc);
-          if (rin) x = x * t;
-          if (cin) x = x * ctt;
+          if (rin) x = zmul_fixed(x, t);
+          if (cin) x = zmul_fixed(x, ctt);
           HH(r, cc) = x;
         }
       }
@@ -1003,8 +1074,8 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
     __syncthreads();
     if (tid == 0) HH(iend, iend - 1) = zr(rtv);
     const zd ctt = zconj(t);
-    for (int cc = iend + 1 + tid; cc <= n; cc += NT) HH(iend, cc) = HH(iend, cc) * ctt;
-    for (int r = 1 + tid; r <= iend - 1; r += NT) HH(r, iend) = HH(r, iend) * t;
+    for (int cc = iend + 1 + tid; cc <= n; cc += NT) HH(iend, cc) = zmul_fixed(HH(iend, cc), ctt);
+    for (int r = 1 + tid; r <= iend - 1; r += NT) HH(r, iend) = zmul_fixed(HH(r, iend), t);
     if (wantz && !zlg)
       for (int r = 1 + tid; r <= n; r += NT) ZZ(r, iend) = zmul_fixed(ZZ(r, iend), t);
   }
@@ -1018,6 +1089,8 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
 // ------------------------------------------------------------------------
 // gschur!(H::Hessenberg{Complex}, Z) (GenericSchur.jl:194-335).
 // Returns 0, or the positive iteration count when maxiter was exceeded.
+// WIN: 0 z_sweep, 2 z_sweep_win2, otherwise z_sweep_res of pitch WIN (rot:
+// its record and dummy areas).
 template <int NT, class L, bool FAST, int WIN = 0> GS_DEV int64_t z_qr(zd* H, L lay, int n, zd* Zg, int64_t ldz, bool wantz, zd* rot,
                                                int* redi, int64_t maxiter, int64_t maxinner, int64_t& nsweep,
                                                int64_t& nstep, ZLog* zl = nullptr) {
@@ -1095,6 +1168,8 @@ template <int NT, class L, bool FAST, int WIN = 0> GS_DEV int64_t z_qr(zd* H, L 
       nsweep += 1;
       if constexpr (WIN == 2)
         z_sweep_win2<FAST, NT>(H, lay.ld, n, Zg, ldz, wantz, rot, rot + ZWL * ZW, redi, t, istart, iend, nstep, *zl);
+      else if constexpr (WIN > 2)
+        z_sweep_res<FAST, WIN>(H, n, Zg, ldz, wantz, rot, rot + 2 * WIN + 4, redi, t, istart, iend, nstep, *zl);
       else
         z_sweep<NT, L, FAST>(H, lay, n, Zg, ldz, wantz, rot, redi, t, istart, iend, nstep);
     }
@@ -1212,8 +1287,9 @@ template <int NT, bool FAST> __global__ void __launch_bounds__(NT) zqr_kernel(Ba
 // of chunk c-1 (z_sweep_win2); the control logic runs on both wavefronts.
 // QR iterations of matrix m of a batch (the body of zqrw2_kernel and of its
 // work-queue form); every thread of the workgroup calls it.
-template <bool FAST, int NT>
-GS_DEV void zqrw2_matrix(const BatchArgs& a, int m, zd* win, int* redi) {
+// RP > 0: the matrix resident in LDS at hs with pitch RP (z_sweep_res).
+template <bool FAST, int NT, int RP = 0>
+GS_DEV void zqrw2_matrix(const BatchArgs& a, int m, zd* win, int* redi, zd* hs = nullptr) {
   const int n = a.n[m];
   if (a.zlog && threadIdx.x == 0) a.llen[m] = 0;
   if (n <= 0) return;
@@ -1232,8 +1308,20 @@ GS_DEV void zqrw2_matrix(const BatchArgs& a, int m, zd* win, int* redi) {
     zl.g = reinterpret_cast<zd*>(a.zlog) + a.loff[m];
     zl.cap = a.loff[m + 1] - a.loff[m];
   }
-  const int64_t st = z_qr<NT, FullLayout, FAST, 2>(T, lay, n, Z, (int64_t)n, wantz, win, redi, maxiter, maxinner,
-                                                    nsweep, nstep, &zl);
+  int64_t st;
+  const FullLayout rlay{RP};
+  if constexpr (RP > 0) {
+    for (int e = threadIdx.x; e < n * n; e += NT) {
+      const int c = e / n, r = e - c * n;
+      hs[r + c * RP] = T[e];
+    }
+    __syncthreads();
+    st = z_qr<NT, FullLayout, FAST, RP>(hs, rlay, n, Z, (int64_t)n, wantz, win, redi, maxiter, maxinner, nsweep,
+                                        nstep, &zl);
+  } else {
+    st = z_qr<NT, FullLayout, FAST, 2>(T, lay, n, Z, (int64_t)n, wantz, win, redi, maxiter, maxinner, nsweep, nstep,
+                                       &zl);
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
     if (zl.g) a.llen[m] = zl.pos;
@@ -1243,8 +1331,31 @@ GS_DEV void zqrw2_matrix(const BatchArgs& a, int m, zd* win, int* redi) {
     }
     a.info[m] = (int32_t)(st > 0x7fffffff ? 0x7fffffff : st);
   }
-  if (st != 0) return;
-  z_finish<NT>(T, lay, n, T, (int64_t)n, W, a.scl[2 * m], a.scl[2 * m + 1]);
+  if (st != 0) {  // not converged: T is what the sweeps have made of it
+    if constexpr (RP > 0)
+      for (int e = threadIdx.x; e < n * n; e += NT) {
+        const int c = e / n, r = e - c * n;
+        T[e] = hs[r + c * RP];
+      }
+    return;
+  }
+  if constexpr (RP > 0) z_finish<NT>(hs, rlay, n, T, (int64_t)n, W, a.scl[2 * m], a.scl[2 * m + 1]);
+  else z_finish<NT>(T, lay, n, T, (int64_t)n, W, a.scl[2 * m], a.scl[2 * m + 1]);
+}
+
+// Orders below RP with H whole in LDS, one wavefront per matrix: a sweep is
+// one chase over the matrix instead of a window copied in and out per chunk
+// of 29 steps with chains through memory beside it.  Bound by the chase's
+// chain of dependent double operations (about 0.35 us a step).  Measured, QR +
+// Z log of one matrix, against the windowed kernel: n = 13 0.45 / 0.56 ms per
+// call, n = 24 0.97 / 1.27, n = 48 2.59 / 3.63; 2000 matrices n = 33..48 4.5 /
+// 6.9 ms, 16384 34.3 / 39.7.  Classes of RP: the LDS decides how many
+// matrices share a CU (RP = 49: four, 33: nine, below by registers).
+template <bool FAST, int RP> __global__ void __launch_bounds__(64) zqrr_kernel(BatchArgs a) {
+  __shared__ zd hs[RP * (RP - 1)];
+  __shared__ zd wk[2 * RP + 4 + RP + 1];
+  __shared__ int redi[4];
+  zqrw2_matrix<FAST, 64, RP>(a, a.order[a.first + blockIdx.x], wk, redi, hs);
 }
 
 template <bool FAST, int NT = 128>
@@ -1676,6 +1787,10 @@ size_t zqr_lds_bytes(int n, int nt) {
   return 16 * ((size_t)BandLayout<2>::size(n) + 2 * (size_t)(n > 0 ? n : 1)) + 4 * (size_t)(nt / 64 + 1);
 }
 
+// The chase takes orders to 63 (one lane per row and column), the LDS four
+// matrices of order 48 per CU; a class up to 63 would hold two.
+int zqr_res_max_n() { return 48; }
+
 int zschur_max_lds_n() {
   // largest n whose Hessenberg-phase footprint fits the 160 KiB of LDS of a
   // gfx950 CU
@@ -1725,8 +1840,20 @@ hipError_t launch_zqr(const BatchArgs& a, int nmax, int nt, hipStream_t s) {
   }
 }
 
-hipError_t launch_zqrw(const BatchArgs& a, hipStream_t s) {
+template <bool FAST> static void launch_zqrr(const BatchArgs& a, int nmax, hipStream_t s) {
+  if (nmax <= 16) hipLaunchKernelGGL((zqrr_kernel<FAST, 17>), dim3(a.count), dim3(64), 0, s, a);
+  else if (nmax <= 24) hipLaunchKernelGGL((zqrr_kernel<FAST, 25>), dim3(a.count), dim3(64), 0, s, a);
+  else if (nmax <= 32) hipLaunchKernelGGL((zqrr_kernel<FAST, 33>), dim3(a.count), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL((zqrr_kernel<FAST, 49>), dim3(a.count), dim3(64), 0, s, a);
+}
+
+hipError_t launch_zqrw(const BatchArgs& a, int nmax, hipStream_t s) {
   if (a.count <= 0) return hipSuccess;
+  if (nmax <= zqr_res_max_n()) {
+    if (a.flags & 0x1000) launch_zqrr<false>(a, nmax, s);
+    else launch_zqrr<true>(a, nmax, s);
+    return hipGetLastError();
+  }
   if (a.flags & 0x1000)
     hipLaunchKernelGGL((zqrw2_kernel<false>), dim3(a.count), dim3(128), 0, s, a);
   else

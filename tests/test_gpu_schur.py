@@ -202,3 +202,37 @@ def test_log_replay_order_edges(gs, cplx, n):
     assert np.all(il == 0)
     for a, d in zip(Sl, Sd):
         assert np.array_equal(a.T, d.T) and np.array_equal(a.Z, d.Z) and np.array_equal(a.values, d.values)
+
+
+@pytest.mark.parametrize("cplx,n", [(True, n) for n in (2, 3, 15, 16, 17, 24, 25, 31, 32, 33, 47, 48, 49)] +
+                         [(False, n) for n in (2, 3, 15, 16, 17, 32, 33, 48, 49, 61, 62, 63, 64)])
+def test_resident_qr_order_edges(gs, oracle, cplx, n):
+    """QR with the matrix held in LDS, at the edges of its pitch classes and of
+    its range: the checks against the oracle for a matrix alone, the same bits
+    in a batch that takes the windowed kernels (complex: beside larger orders;
+    real: above the widest class's launch size), with Z updated in place, with
+    a one-sweep log, and T without Z.  The matrices deflate in the middle,
+    are scaled to near underflow, and cycle (exceptional shifts)."""
+    rng = gen.stream(34, 100, n)
+    A = gen.ginibre_complex(n, rng) if cplx else gen.ginibre_real(n, rng)
+    B = A.copy()
+    B[n // 2:, :n // 2] *= 1e-13
+    mats = [A, B, A * 1e-300, gen.cyclic_shift(n, cplx) if n > 2 else A.T.copy()]
+    S1 = [gs.gschur(M) for M in mats]
+    for M, S in zip(mats[:2], S1):
+        _check(oracle, M, S)
+    if cplx:
+        rest = [gen.ginibre_complex(60, rng)]
+    else:
+        rest = [A] * 4097 if n in (49, 62) else []
+    for kw in ({}, {"zdirect": True}, {"zlog_tiny": True}):
+        Sb, ib = gs.gschur_batched(mats + rest, **kw)
+        assert np.all(ib == 0)
+        for a, b in zip(S1, Sb):
+            assert np.array_equal(a.T, b.T) and np.array_equal(a.Z, b.Z) and np.array_equal(a.values, b.values)
+        rest = rest[:1]
+    Sb, _ = gs.gschur_batched(mats)
+    for a, M, b in zip(S1, mats, Sb):
+        N = gs.gschur(M, wantZ=False)
+        assert np.array_equal(a.T, N.T) and np.array_equal(a.values, N.values)
+        assert np.array_equal(a.T, b.T) and np.array_equal(a.Z, b.Z)
