@@ -12,7 +12,10 @@
 //      (hessenberg.jl:150-195 hands this to LAPACK's orgqr).
 //   4. Francis double-shift QR (GenericSchur.jl:513-699, 837-952).  One
 //      workgroup runs the control logic (deflation, shifts, 2x2 standard
-//      form, start row) between sweeps.  A sweep's bulge chase runs in
+//      form, start row) between sweeps.  From order MSMINN up, active blocks
+//      of MSMIN rows and more take multishift sweeps (multishift.h), MNB
+//      double shifts at a time; the others a double-shift sweep, whose bulge
+//      chase runs in
 //      chunks of up to LKC steps: the chunk's window of H (rows and columns
 //      k0-1 .. kend+3) sits in LDS of one wavefront that chases the bulge
 //      and logs the reflectors, while the other workgroups of the same
@@ -30,6 +33,7 @@
 #include "dchase.h"
 #include "gs2x2.h"
 #include "internal.h"
+#include "multishift.h"
 
 namespace gs {
 
@@ -355,12 +359,6 @@ template <int NT> __global__ void __launch_bounds__(NT) lzero_lower_kernel(doubl
 }
 
 // ------------------------------------------------------------- QR phase
-struct LState {
-  int64_t iter, nsweep, nstep;
-  int iend, istart, iterqr, iwcur, phase, status, mx, pad;
-  double v0, v1, v2;
-};
-
 struct LQArgs {
   double* H;
   int64_t ld;
@@ -370,8 +368,9 @@ struct LQArgs {
   int wantz;
   zd* W;
   LState* st;
-  double* lg;  // 3 per bulge step of the current sweep
+  double* lg;  // 3 per bulge step of the current sweep; multishift: two chunks' logs
   int64_t maxiter;
+  int msmin;  // smallest active block with multishift sweeps, 0: none
 };
 
 // Control logic of gschur!(H::Hessenberg{<:AbstractFloat}) (GenericSchur.jl:
@@ -409,9 +408,11 @@ template <int NT> __global__ void __launch_bounds__(NT) lctrl_kernel(LQArgs a) {
       break;
     }
     const int iend = s.iend;
-    int istart = s.istart;
     int found = -1;
-    for (int k = iend - tid; k >= istart + 1; k -= NT) {
+    // with multishift sweeps, down to the known split, where they have to start
+    // (a double-shift sweep's start row finds it by itself)
+    const int klo = a.msmin > 0 ? 2 : s.istart + 1;
+    for (int k = iend - tid; k >= klo; k -= NT) {
       bool split = fabs(H(k, k - 1)) < smallnum;
       if (!split) {
         const double Hkk = H(k, k);
@@ -438,7 +439,7 @@ template <int NT> __global__ void __launch_bounds__(NT) lctrl_kernel(LQArgs a) {
       }
     }
     found = block_max_int<NT>(found, redi);
-    istart = (found > 0) ? found : 1;
+    const int istart = (found > 0) ? found : 1;
     s.istart = istart;
     if (istart > 1) {
       __syncthreads();
@@ -495,8 +496,20 @@ template <int NT> __global__ void __launch_bounds__(NT) lctrl_kernel(LQArgs a) {
       s.phase = 0;
       continue;
     }
-    // shifts (GenericSchur.jl:613-665)
+    // a multishift sweep (its shifts come from dshift_kernel); it counts as MNB
+    // iterations, and an iteration that stalls takes the exceptional shifts
     s.iterqr += 1;
+    s.nb = 0;
+    if (a.msmin > 0 && iend - istart + 1 >= a.msmin && s.iterqr != 10 && s.iterqr != 20) {
+      s.nb = MNB;
+      s.iter += MNB - 1;
+      s.nsweep += MNB;
+      s.nstep += MNB * (int64_t)(iend - istart);
+      s.mx = istart;
+      s.status = 0;
+      break;
+    }
+    // shifts (GenericSchur.jl:613-665)
     const double threeq = 0.75, m7_16 = -7.0 / 16.0;
     double H11, H12, H21, H22;
     if (s.iterqr == 10) {
@@ -709,6 +722,110 @@ __global__ void __launch_bounds__(64) lchunk_kernel(LQArgs a, int c) {
   (void)plast;
 }
 
+// One chunk of a multishift sweep (multishift.h).  Bound by workgroup 0: the
+// chase (64 times, about 0.8 us each: two barriers, two LDS round trips and a
+// reflector in a chain, two wavefronts to a SIMD), then the new columns' left
+// update, the window's loads and stores (about 20 us a chunk together).  The
+// other workgroups' lines fit behind it.  A chunk moves eight bulges 64 rows in
+// about 70 us, lchunk_kernel one bulge 60 rows in about 30.
+__global__ void __launch_bounds__(64 * MNB) lms_kernel(LQArgs a, int c) {
+  extern __shared__ double lds[];
+  double* const win = lds;                      // MNW columns of pitch MWP
+  double* const buf = win + MWP * MNW;          // 64 lines of up to MNW elements and two of padding
+  double* const plg = buf + MLP * (MNW + 2);    // the previous chunk's log
+  if (a.st->status != 0 || a.st->nb == 0) return;
+  const int I = a.st->istart, E = a.st->iend;
+  MChunk ck;
+  if (!ms_chunk_of(I, E, c, ck)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = a.n;
+  const int64_t ld = a.ld;
+  double* const H = a.H;
+  const bool chase = ck.t0 <= ck.t1, prev = ck.pt0 <= ck.pt1;
+  const int wb = chase ? ms_wb(I, ck.t0) : 0, we = chase ? ms_we(I, E, ck.t1) : 0;
+  const int pwb = prev ? ms_wb(I, ck.pt0) : 1, pwe = prev ? ms_we(I, E, ck.pt1) : 0;
+  const int pn = pwe - pwb + 1;  // elements of a line
+  if (prev) {
+    const double* g = a.lg + MLG * ((c - 1) & 1);
+    for (int e = tid; e < 3 * MNB * (ck.pt1 - ck.pt0 + 1); e += 64 * MNB) plg[e] = g[e];
+    // the padding of the lines
+    if (tid < 2 * 64) buf[(pn + wave) * MLP + lane] = 0.0;
+  }
+  if (blockIdx.x == 0) {
+    if (!chase) return;
+    const int W = we - wb + 1;
+    // the window, without the rows of its new columns that the previous
+    // chunk's left update comes to first
+    for (int col = wb + wave; col <= we; col += MNB) {
+      const double* src = H + (int64_t)(col - 1) * ld;
+      double* dst = win + (col - wb) * MWP;
+      const int r0 = prev && col > pwe ? pwe + 1 : wb;
+      for (int r = r0 + lane; r <= we; r += 64) dst[r - wb] = src[r - 1];
+    }
+    if (prev && we > pwe) {
+      const int nc = we - pwe;  // at most MST
+      for (int l = wave; l < 64; l += MNB) {
+        const double* src = H + (int64_t)(pwe + l) * ld + (pwb - 1);
+        for (int e = lane; e < pn; e += 64) buf[e * MLP + l] = l < nc ? src[e] : 0.0;
+      }
+      __syncthreads();
+      ms_lines(buf, plg, ck.pt0, ck.pt1, I, E, pwb);
+      for (int l = wave; l < nc; l += MNB) {
+        double* dst = H + (int64_t)(pwe + l) * ld + (pwb - 1);
+        double* wc = win + (pwe + 1 + l - wb) * MWP;
+        for (int e = lane; e < pn; e += 64) {
+          const double v = buf[e * MLP + l];
+          if (pwb + e < wb) dst[e] = v;
+          else wc[pwb + e - wb] = v;
+        }
+      }
+    }
+    __syncthreads();
+    ms_chase(win, a.lg + MLG * (c & 1), a.st->sh, ck.t0, ck.t1, I, E, wb, we);
+    for (int col = wave; col < W; col += MNB) {
+      double* dst = H + (wb - 1) + (int64_t)(wb - 1 + col) * ld;
+      for (int r = lane; r < W; r += 64) dst[r] = win[r + col * MWP];
+    }
+    return;
+  }
+  if (!prev) return;
+  // the previous chunk's updates outside both windows, 64 lines at a time
+  const int lcol0 = (chase ? we : pwe) + 1;
+  const int nL = n >= lcol0 ? (n - lcol0 + 64) / 64 : 0;
+  const int nR = (pwb - 1 + 63) / 64;
+  const int nZ = a.wantz ? (n + 63) / 64 : 0;
+  for (int t = blockIdx.x - 1; t < nL + nR + nZ; t += gridDim.x - 1) {
+    __syncthreads();
+    if (t < nL) {
+      const int col0 = lcol0 + 64 * t;
+      for (int l = wave; l < 64; l += MNB) {
+        const double* src = H + (int64_t)(min(col0 + l, n) - 1) * ld + (pwb - 1);
+        for (int e = lane; e < pn; e += 64) buf[e * MLP + l] = src[e];
+      }
+      __syncthreads();
+      ms_lines(buf, plg, ck.pt0, ck.pt1, I, E, pwb);
+      for (int l = wave; l < 64 && col0 + l <= n; l += MNB) {
+        double* dst = H + (int64_t)(col0 + l - 1) * ld + (pwb - 1);
+        for (int e = lane; e < pn; e += 64) dst[e] = buf[e * MLP + l];
+      }
+    } else {
+      const bool isz = t >= nL + nR;
+      double* const M = isz ? a.Z : H;
+      const int64_t lm = isz ? a.ldz : ld;
+      const int nrow = isz ? n : pwb - 1;
+      const int row = 64 * (t - (isz ? nL + nR : nL)) + lane;  // 0-based
+      const double* src = M + min(row, nrow - 1) + (int64_t)(pwb - 1) * lm;
+      for (int e = wave; e < pn; e += MNB) buf[e * MLP + lane] = src[(int64_t)e * lm];
+      __syncthreads();
+      ms_lines(buf, plg, ck.pt0, ck.pt1, I, E, pwb);
+      if (row < nrow) {
+        double* dst = M + row + (int64_t)(pwb - 1) * lm;
+        for (int e = wave; e < pn; e += MNB) dst[(int64_t)e * lm] = buf[e * MLP + lane];
+      }
+    }
+  }
+}
+
 // T = triu(HH, -1) and safescale! of T and the values (GenericSchur.jl:
 // 697, 830-833)
 template <int NT> __global__ void __launch_bounds__(NT) lfinish_kernel(double* H, int64_t ld, int n, zd* W,
@@ -845,6 +962,7 @@ hipError_t large_schur_d(const LargeArgs& a, LargeWork& w, hipStream_t s, LargeT
   q.st = static_cast<LState*>(w.st);
   q.lg = w.lg;
   q.maxiter = a.maxiter > 0 ? a.maxiter : 100 * (int64_t)n;
+  q.msmin = n >= MSMINN ? MSMIN : 0;
   LState st0;
   std::memset(&st0, 0, sizeof st0);
   st0.iend = n;
@@ -873,7 +991,38 @@ hipError_t large_schur_d(const LargeArgs& a, LargeWork& w, hipStream_t s, LargeT
   int64_t issued = 0, done = 0;  // sweeps issued / whose state was read
   LState last;
   std::memset(&last, 0, sizeof last);
-  while (true) {
+  // Multishift sweeps down to active blocks of MSMIN rows.  Few and long, so
+  // the host waits for each one's state and launches exactly its chunks; a
+  // smaller block that splits off below a larger one takes double-shift sweeps.
+  if ((e = hipFuncSetAttribute((const void*)lms_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, MS_LDS)) !=
+      hipSuccess)
+    return fail(e);
+  while (q.msmin > 0) {
+    hipLaunchKernelGGL(lctrl_kernel<1024>, dim3(1), dim3(1024), 0, s, q);
+    if ((e = hipGetLastError()) != hipSuccess) return fail(e);
+    if ((e = hipMemcpyAsync(hst, q.st, sizeof(LState), hipMemcpyDeviceToHost, s)) != hipSuccess) return fail(e);
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) return fail(e);
+    last = hst[0];
+    status = last.status;
+    seen_iend = last.iend;
+    if (status != 0) break;
+    if (last.nb > 0) {
+      if ((e = launch_dshift(H, ldt, q.st, s)) != hipSuccess) return fail(e);
+      const int nch = ms_chunks(last.istart, last.iend);
+      for (int c = 0; c <= nch; ++c) {
+        hipLaunchKernelGGL(lms_kernel, dim3(1 + std::min(3 * nwork, 255)), dim3(64 * MNB), MS_LDS, s, q, c);
+        if ((e = hipGetLastError()) != hipSuccess) return fail(e);
+      }
+    } else {
+      const int nch = (last.iend - last.mx + LKC - 1) / LKC;
+      for (int c = 0; c <= nch; ++c) {
+        hipLaunchKernelGGL(lchunk_kernel, dim3(grid), dim3(64), 0, s, q, c);
+        if ((e = hipGetLastError()) != hipSuccess) return fail(e);
+      }
+      if (last.iend < q.msmin) break;
+    }
+  }
+  while (status == 0) {
     if (issued - done == kAhead) {
       // read the oldest outstanding state
       const int slot = (int)(done % kAhead);
@@ -926,7 +1075,7 @@ size_t large_work_doubles(int64_t n, LargeWorkSizes* sz) {
   sz->tv = LNB;
   sz->part = std::max<int64_t>((n + 63) / 64 * n, 2048);
   sz->scl = 2;
-  sz->lg = 3 * n + 3;
+  sz->lg = std::max<int64_t>(3 * n + 3, 2 * MLG);
   sz->st = (sizeof(LState) + 7) / 8;
   sz->gk = (int64_t)dgemm_splitk_doubles(LNB, (int)n, (int)n);
   // every segment is carved at a multiple of 32 doubles (256 bytes)
@@ -940,6 +1089,7 @@ size_t large_work_doubles(int64_t n, LargeWorkSizes* sz) {
   return (size_t)total;
 }
 
-size_t large_state_bytes() { return sizeof(LState); }
+// the pinned host record: the state of up to four sweeps
+size_t large_state_bytes() { return 4 * sizeof(LState); }
 
 }  // namespace gs

@@ -22,6 +22,7 @@
 #include "gs2x2.h"
 #include "internal.h"
 #include "layout.h"
+#include "multishift.h"
 
 namespace gs {
 
@@ -1056,6 +1057,58 @@ hipError_t launch_dqrw(const BatchArgs& a, int nmax, hipStream_t s) {
     hipLaunchKernelGGL((dqrw_kernel<false>), dim3(a.count), dim3(64), 0, s, a);
   else
     hipLaunchKernelGGL((dqrw_kernel<true>), dim3(a.count), dim3(64), 0, s, a);
+  return hipGetLastError();
+}
+
+// Shifts of a multishift sweep: the eigenvalues of the trailing 2 MNB x 2 MNB
+// block of the active block, by the resident QR (its diagonal where that does
+// not converge), complex ones in their conjugate pairs, the real ones two by
+// two.  One wavefront.
+__global__ void __launch_bounds__(64) dshift_kernel(const double* H, int64_t ld, LState* st) {
+  constexpr int M = 2 * MNB, RP = M + 1;
+  __shared__ double hs[RP * M];
+  __shared__ double lg[3 * RP + 2];
+  __shared__ zd w[M];
+  __shared__ int redi[2];
+  if (st->status != 0 || st->nb == 0) return;
+  const int i0 = st->iend - M;  // 0-based
+  for (int e = threadIdx.x; e < M * M; e += 64) {
+    const int c = e / M, r = e - c * M;
+    hs[r + c * RP] = r <= c + 1 ? H[(i0 + r) + (int64_t)(i0 + c) * ld] : 0.0;
+  }
+  if (threadIdx.x < M) w[threadIdx.x] = zr(H[(i0 + threadIdx.x) + (int64_t)(i0 + threadIdx.x) * ld]);
+  __syncthreads();
+  const FullLayout lay{RP};
+  int64_t nsweep = 0, nstep = 0;
+  const int64_t rc = d_qr<64, FullLayout, true, RP>(hs, lay, M, nullptr, 0, false, lg, redi, w, 30 * M, nsweep, nstep,
+                                                    nullptr);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  int nc = 0, nr = 0;  // bulges with complex shifts, from the front; real ones, from the back
+  double keep = 0.0;
+  for (int i = 0; i < M; ++i) {
+    const zd x = w[i];
+    if (rc == 0 && x.y != 0.0) {
+      double* sh = st->sh + 4 * nc++;
+      sh[0] = x.x;
+      sh[1] = x.y;
+      sh[2] = x.x;
+      sh[3] = -x.y;
+      ++i;
+    } else if (nr++ & 1) {
+      double* sh = st->sh + 4 * (MNB - nr / 2);
+      sh[0] = keep;
+      sh[1] = 0.0;
+      sh[2] = x.x;
+      sh[3] = 0.0;
+    } else {
+      keep = x.x;
+    }
+  }
+}
+
+hipError_t launch_dshift(const double* H, int64_t ld, LState* st, hipStream_t s) {
+  hipLaunchKernelGGL(dshift_kernel, dim3(1), dim3(64), 0, s, H, ld, st);
   return hipGetLastError();
 }
 

@@ -939,7 +939,7 @@ static hipError_t run_large(gs_handle* h, int64_t n, double* dA, int64_t lda, do
   hipError_t e = h->lwork.ensure(8 * nd);
   if (e != hipSuccess) return e;
   if (!h->lhost) {
-    e = hipHostMalloc(&h->lhost, 1024, hipHostMallocDefault);
+    e = hipHostMalloc(&h->lhost, large_state_bytes(), hipHostMallocDefault);
     if (e != hipSuccess) {
       h->lhost = nullptr;
       return e;

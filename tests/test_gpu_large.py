@@ -184,3 +184,37 @@ def test_large_workload4_full_size(gs):
     # (U makes most eigenvalues ill-conditioned: a small eigenvalue's error
     # disc can hold its neighbours, so the nearest exact value is not unique)
     assert np.all(err <= bound), float(np.max(err / bound))
+
+
+def _multishift_mats(n, rng):
+    """A random matrix; one that splits above its last 64 rows (the smallest
+    block with multishift sweeps) and one above its last 63; a cyclic shift
+    (stalls until the exceptional shifts); a graded one."""
+    A = gen.ginibre_real(n, rng)
+    B, C = A.copy(), A.copy()
+    B[n - 64:, :n - 64] = 0
+    C[n - 63:, :n - 63] = 0
+    d = 10.0 ** np.linspace(4, -4, n)
+    return [A, B, C, gen.cyclic_shift(n, False), d[:, None] * A]
+
+
+@pytest.mark.parametrize("n", [255, 256, 299, 300, 301, 364])
+def test_multishift_orders(gs, n):
+    """Multishift sweeps at orders around a chunk's edges (64 times of the
+    bulge train; n + 20 = 319 .. 321 and 384) and the smallest with them: the Schur invariants, T bitwise the same
+    without Z, the eigenvalues within the eigenvalue bound of the plain
+    double-shift kernel's, and an error at the iteration limit."""
+    eps = np.finfo(np.float64).eps
+    for i, A in enumerate(_multishift_mats(n, gen.stream(26, 100, n))):
+        print(f"case multishift n={n} matrix {i}", flush=True)
+        S = gs.gschur(A)
+        checks.schur_invariants(A, S.T, S.Z, S.values, TOL)
+        assert checks.rel_backward(A, S.T, S.Z) <= 50 * n * eps and checks.rel_orth(S.Z) <= 50 * n * eps
+        N = gs.gschur(A, wantZ=False)
+        assert np.array_equal(S.T, N.T) and np.array_equal(S.values, N.values)
+        if i != 4:  # (a graded matrix's small eigenvalues are as uncertain as its norm)
+            P = gs.gschur(A, plain=True)
+            _, d = checks.match_eigenvalues(S.values, P.values)
+            assert np.max(d) <= 1e4 * n * eps * np.linalg.norm(A, 2)
+    with pytest.raises(gs.UnconvergedException):
+        gs.gschur(gen.ginibre_real(n, gen.stream(26, 101, n)), maxiter=20)
