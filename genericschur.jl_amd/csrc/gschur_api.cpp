@@ -513,12 +513,17 @@ static bool bin_zlog(bool cplx, const Bin& b, int kflags) {
 
 // Whether a complex plan's QR iterations run as one work-queue launch: not
 // where every order fits the LDS-resident kernels (one QR launch per bin;
-// 16384 matrices n = 4..24 3.8 against 6.9 ms, n = 33..48 34.3 against 39.7).
-// A plan with larger orders queues the small ones too: they fill the queue's
-// tail (2500 matrices n = 24..60 8.5 ms; those up to 48 in resident launches
-// beside the queue 11.2, the 8192 of n = 8..96 50.4 against 53.6).
+// 16384 matrices n = 4..24 3.8 against 6.9 ms, n = 33..48 34.3 against 39.7),
+// nor where the matrices are too few for the queue's small workgroups to fill
+// the CUs (200 matrices n = 49..96 12.7 per bin against 14.1 ms).  A larger plan
+// with larger orders queues the small ones too: they fill the queue's tail
+// (2500 matrices n = 24..60 8.5 ms; those up to 48 in resident launches beside
+// the queue 11.2, the 8192 of n = 8..96 50.4 against 53.6).
 static bool plan_queue(const Tuning& t, bool cplx, const std::vector<Bin>& bins) {
-  return qr_queue(t, cplx) && !bins.empty() && bins[0].nmax > zqr_res_max_n();
+  if (!qr_queue(t, cplx) || bins.empty() || bins[0].nmax <= zqr_res_max_n()) return false;
+  int64_t count = 0;
+  for (const Bin& b : bins) count += b.count;
+  return count > kCoopCount;
 }
 
 // Work-queue form of a complex batch (tuning queue = 1): the bins'
@@ -1008,15 +1013,19 @@ static hipError_t run_large(gs_handle* h, int64_t n, double* dA, int64_t lda, do
 }
 
 // Threads of the windowed QR kernel for one matrix above the LDS-resident
-// orders.
+// orders.  Measured, whole call without / with Z, 512 against 1024 threads:
+// n = 130 20.7 / 23.0 against 22.4 / 24.6 ms, n = 400 216 / 248 against 263 /
+// 279, n = 1000 1862 / 2109 against 1864 / 2116, n = 1500 (more chains than
+// seven wavefronts finish behind the chase) 6371 / 7109 against 5798 / 6576.
+// GSCHUR_WIN_NT overrides (512 or 1024).
 static int win_nt(int n) {
   static const int force = [] {
     const char* e = std::getenv("GSCHUR_WIN_NT");
     const int v = e ? std::atoi(e) : 0;
-    return (v == 128 || v == 256 || v == 512 || v == 1024) ? v : 0;
+    return (v == 512 || v == 1024) ? v : 0;
   }();
   if (force) return force;
-  return n <= 128 ? 256 : (n <= 256 ? 512 : 1024);
+  return n <= 1000 ? 512 : 1024;
 }
 
 static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda, double* T, int64_t ldt, double* Z,
@@ -1191,8 +1200,6 @@ static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda
       a.loff = zlg ? reinterpret_cast<const int64_t*>(mp + offsetof(Meta, loff)) : nullptr;
       a.llen = zlg ? reinterpret_cast<int64_t*>(mp + offsetof(Meta, llen)) : nullptr;
       a.zlog_min = 0;
-      // chain wavefronts in proportion to the lines a chunk updates (about
-      // 2n rows and columns): GSCHUR_WIN_NT overrides (128 .. 1024)
       le = launch_zqrw_single(a, win_nt((int)n), h->stream);
       if (le == hipSuccess && zlg)
         le = launch_zlog_rows((int)n, dZ, n, static_cast<const double*>(h->bLog.p),

@@ -75,6 +75,8 @@ hipError_t launch_zqr(const BatchArgs& a, int nmax, int nt, hipStream_t s);
 // QR launch of matrices of order at most nmax: up to z/dqr_res_max_n() one
 // wavefront per matrix with H in LDS, above windowed with H and Z in HBM (a
 // launch's matrices all on one side of that order)
+// complex launches up to this size take the 512-thread windowed form
+constexpr int kCoopCount = 256;
 int zqr_res_max_n();
 int dqr_res_max_n();
 hipError_t launch_zqrw(const BatchArgs& a, int nmax, hipStream_t s);

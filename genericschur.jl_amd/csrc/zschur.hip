@@ -653,6 +653,32 @@ template <bool TAIL = true> GS_DEV void zchain_full(zd* p, const zd* lg, int ka,
   }
 }
 
+// zchain_full in two parts: the column's entries into registers, and the chain.
+GS_DEV void zchain_load(const zd* p, int ka, zd (&x)[ZKC + 1]) {
+  const zd* q0 = p + (__builtin_amdgcn_readfirstlane(ka) - 1);
+#pragma unroll
+  for (int e = 0; e <= ZKC; ++e) x[e] = q0[e];
+}
+GS_DEV void zchain_run(zd* p, const zd* lg, int ka, zd* tail2, zd (&x)[ZKC + 1], bool on) {
+  zd* q0 = p + (__builtin_amdgcn_readfirstlane(ka) - 1);
+#pragma unroll
+  for (int g = 0; g < ZKC; g += ZCG) {
+    int lb = 0;
+    asm volatile("" : "+s"(lb));  // the group's log reads stay here
+#pragma unroll
+    for (int q = g; q < g + ZCG && q < ZKC; ++q) {
+      const zd tau1 = lg[2 * q + lb], v2 = lg[2 * q + 1 + lb];
+      zrot_left_fixed(x[q], x[q + 1], tau1, v2, ztau2_fixed(tau1, v2));
+    }
+  }
+  if (on) {
+#pragma unroll
+    for (int q = 0; q < ZKC - 1; ++q) q0[q] = x[q];
+    tail2[0] = x[ZKC - 1];
+    tail2[1] = x[ZKC];
+  }
+}
+
 // zchain<false> (a row of H or Z, x(t) = p[(t - 1) st]) for a full chunk:
 // fixed shape, as zchain_full.
 template <int G> GS_DEV void zchain_full_row(zd* p, int64_t st, const zd* lg, int ka) {
@@ -931,6 +957,12 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
   constexpr int CS = NT - 64;  // threads of the chain wavefronts
   const int cw = tid - 64;
   const FullLayout lay{ld};
+  // one matrix on the workgroup (registers for the prefetch below up to 512
+  // threads): all its wavefronts take part in the window's loads and stores,
+  // which two window buffers let overlap
+  constexpr bool COOP = NT == 512;
+  constexpr int NWV = NT / 64;
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
   zd v0, v1;
   const int istart1 = z_sweep_start<NT>(H, lay, redi, shift, istart, iend, v0, v1);
   bool phase_pending = istart1 > istart;
@@ -950,6 +982,7 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
   }
   int pk0 = 1, pkend = 0, pwe = 0, pwb = 1;  // chunk whose chains are pending (none)
   int k0 = istart1;
+  zd xn[ZKC + 1];  // COOP, wavefront 1: the next chunk's new columns
   for (int c = 0;; ++c) {
     const bool chase = k0 <= iend - 1;
     const bool prev = pk0 <= pkend;
@@ -958,38 +991,80 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
     const int wb = chase ? max(k0 - 1, 1) : 0, we = chase ? min(kend + 2, iend) : 0;
     zd* lg = lgbuf + (c & 1) * 2 * ZKC;
     const zd* plg = lgbuf + ((c + 1) & 1) * 2 * ZKC;
+    zd* const wcur = COOP ? win + (c & 1) * (ZWL * ZW) : win;
+    if constexpr (COOP) {
+      // the previous window to HBM; the new one takes its last three rows and
+      // columns from there, the other entries from HBM, its new columns (right
+      // of the previous window) after the previous chunk's left update, whose
+      // operands wavefront 1 has loaded behind its own chains on them
+      const zd* const wold = win + ((c + 1) & 1) * (ZWL * ZW);
+      if (prev) {
+        const int pW = pwe - pwb + 1;
+        const int r = lane & 31;
+        for (int col = 2 * wave + (lane >> 5); col < pW; col += 2 * NWV)
+          if (r < pW) HH(pwb + r, pwb + col) = wold[r + col * ZWL];
+        if (zlg && wave == NWV - 1 && lane < 2 * (pkend - pk0 + 1)) rec[2 + 2 * (pk0 - istart1) + lane] = plg[lane];
+      }
+      if (chase) {
+        const int W = we - wb + 1;
+        const int ov = prev ? 3 : 0;  // (a chunk that another follows is a full one: pwe = wb + 2)
+        for (int col = wv; col < W; col += NWV) {
+          const int r0 = col < ov ? ov : (prev ? 2 : 0);
+          if (lane >= r0 && lane < W)
+            __builtin_amdgcn_global_load_lds((const void*)(H + (wb - 1) + (int64_t)(wb - 1 + col) * ld + lane),
+                                             (__attribute__((address_space(3))) void*)(wcur + col * ZWL), 16, 0, 0);
+        }
+        if (prev) {
+          if (wave == 0 && lane < 9) {
+            const int r = lane % 3, col = lane / 3;
+            wcur[r + col * ZWL] = wold[(wb - pwb + r) + (wb - pwb + col) * ZWL];
+          }
+          if (wv == 1) {
+            const int col = min(pwe + 1 + lane, we);
+            zchain_run(H + (int64_t)(col - 1) * ld, plg, pk0, wcur + (pkend - wb) + (col - wb) * ZWL, xn,
+                       pwe + 1 + lane <= we);
+          }
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the window is in LDS
+      }
+      __syncthreads();
+    }
     if (wave == 0) {
       if (chase) {
-        // the window's loads are issued first; while they are in flight the
-        // previous chunk's reflectors are applied to the window's columns
-        // right of the previous window (rows pk0 .. pkend + 1 in HBM), whose
-        // last two rows (the window's rows wb, wb + 1) go to the window
-        const int W = we - wb + 1;
-        {
-          // window columns straight into LDS (lane r: row wb + r), the rows
-          // that the chains below provide left out
-          const int Wu = __builtin_amdgcn_readfirstlane(W);
-          const int cs = prev ? min(max(pwe + 1 - wb, 0), Wu) : Wu;
-          const zd* gp = H + (wb - 1) + (int64_t)(wb - 1) * ld + lane;
-          if (prev) {
-            // the previous chunk is a full one (only a sweep's last chunk is shorter)
-            const int col = pwe + 1 + lane;
-            if (col <= we) zchain_full(H + (int64_t)(col - 1) * ld, plg, pk0, win + (pkend - wb) + (col - wb) * ZWL);
+        if constexpr (!COOP) {
+          // the window's loads are issued first; while they are in flight the
+          // previous chunk's reflectors are applied to the window's columns
+          // right of the previous window (rows pk0 .. pkend + 1 in HBM), whose
+          // last two rows (the window's rows wb, wb + 1) go to the window
+          const int W = we - wb + 1;
+          {
+            // window columns straight into LDS (lane r: row wb + r), the rows
+            // that the chains below provide left out
+            const int Wu = __builtin_amdgcn_readfirstlane(W);
+            const int cs = prev ? min(max(pwe + 1 - wb, 0), Wu) : Wu;
+            const zd* gp = H + (wb - 1) + (int64_t)(wb - 1) * ld + lane;
+            if (prev) {
+              // the previous chunk is a full one (only a sweep's last chunk is shorter)
+              const int col = pwe + 1 + lane;
+              if (col <= we) zchain_full(H + (int64_t)(col - 1) * ld, plg, pk0, win + (pkend - wb) + (col - wb) * ZWL);
+            }
+            if (lane < Wu)
+              for (int c = 0; c < cs; ++c)
+                __builtin_amdgcn_global_load_lds((const void*)(gp + (int64_t)c * ld),
+                                                 (__attribute__((address_space(3))) void*)(win + c * ZWL), 16, 0, 0);
+            if (lane < Wu && lane >= 2)
+              for (int c = cs; c < Wu; ++c)
+                __builtin_amdgcn_global_load_lds((const void*)(gp + (int64_t)c * ld),
+                                                 (__attribute__((address_space(3))) void*)(win + c * ZWL), 16, 0, 0);
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the window is in LDS
           }
-          if (lane < Wu)
-            for (int c = 0; c < cs; ++c)
-              __builtin_amdgcn_global_load_lds((const void*)(gp + (int64_t)c * ld),
-                                               (__attribute__((address_space(3))) void*)(win + c * ZWL), 16, 0, 0);
-          if (lane < Wu && lane >= 2)
-            for (int c = cs; c < Wu; ++c)
-              __builtin_amdgcn_global_load_lds((const void*)(gp + (int64_t)c * ld),
-                                               (__attribute__((address_space(3))) void*)(win + c * ZWL), 16, 0, 0);
-          __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the window is in LDS
+          wsync();
         }
-        wsync();
-        z_chase_chunk<FAST, ZWL>(win, wb, we, k0, kend, istart1, iend, v0, v1, lg, lgbuf + 4 * ZKC);
-        win_store<zd, ZW, ZWL>(H + (wb - 1) + (int64_t)(wb - 1) * ld, ld, W, win, lane);
-        if (zlg && lane < 2 * (kend - k0 + 1)) rec[2 + 2 * (k0 - istart1) + lane] = lg[lane];
+        z_chase_chunk<FAST, ZWL>(wcur, wb, we, k0, kend, istart1, iend, v0, v1, lg, lgbuf + 4 * ZKC);
+        if (!COOP || phase_pending) {
+          win_store<zd, ZW, ZWL>(H + (wb - 1) + (int64_t)(wb - 1) * ld, ld, we - wb + 1, wcur, lane);
+          if (zlg && lane < 2 * (kend - k0 + 1)) rec[2 + 2 * (k0 - istart1) + lane] = lg[lane];
+        }
       }
     } else if (prev) {
       // the chain wavefronts (1 .. NT / 64 - 1) share the lines: thread cw
@@ -1009,6 +1084,14 @@ template <bool FAST, int NT = 128> GS_DEV void z_sweep_win2(zd* H, int64_t ld, i
         for (int row = 1 + cw; row <= pwb - 1; row += CS) zchain<false>(H + (row - 1), ld, plg, pk0, pkend);
         if (wantz && !zlg)
           for (int row = 1 + cw; row <= n; row += CS) zchain<false>(Zg + (row - 1), ldz, plg, pk0, pkend);
+      }
+    }
+    if constexpr (COOP) {
+      // rows k0 .. kend + 1 of the next chunk's new columns; the last writes to
+      // them were this wavefront's
+      if (wv == 1 && chase && !phase_pending && kend + 1 <= iend - 1) {
+        const int col = min(we + 1 + lane, min(kend + ZKC + 2, iend));
+        zchain_load(H + (int64_t)(col - 1) * ld, k0, xn);
       }
     }
     if (wave == 0 && !chase && prev)
@@ -1167,7 +1250,8 @@ template <int NT, class L, bool FAST, int WIN = 0> GS_DEV int64_t z_qr(zd* H, L 
       }
       nsweep += 1;
       if constexpr (WIN == 2)
-        z_sweep_win2<FAST, NT>(H, lay.ld, n, Zg, ldz, wantz, rot, rot + ZWL * ZW, redi, t, istart, iend, nstep, *zl);
+        z_sweep_win2<FAST, NT>(H, lay.ld, n, Zg, ldz, wantz, rot, rot + (NT == 512 ? 2 : 1) * ZWL * ZW, redi, t, istart, iend,
+                               nstep, *zl);
       else if constexpr (WIN > 2)
         z_sweep_res<FAST, WIN>(H, n, Zg, ldz, wantz, rot, rot + 2 * WIN + 4, redi, t, istart, iend, nstep, *zl);
       else
@@ -1359,8 +1443,8 @@ template <bool FAST, int RP> __global__ void __launch_bounds__(64) zqrr_kernel(B
 }
 
 template <bool FAST, int NT = 128>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) zqrw2_kernel(BatchArgs a) {
-  __shared__ zd win[ZWL * ZW + 4 * ZKC + ZWL + 1];
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 512 ? 2 : 4))) zqrw2_kernel(BatchArgs a) {
+  __shared__ zd win[(NT == 512 ? 2 : 1) * ZWL * ZW + 4 * ZKC + ZWL + 1];
   __shared__ int redi[NT / 64 > 4 ? NT / 64 : 4];
   const int b = blockIdx.x;
   if (b >= a.count) return;
@@ -1847,6 +1931,9 @@ template <bool FAST> static void launch_zqrr(const BatchArgs& a, int nmax, hipSt
   else hipLaunchKernelGGL((zqrr_kernel<FAST, 49>), dim3(a.count), dim3(64), 0, s, a);
 }
 
+// Launches of at most one matrix per CU take the 512-thread form (one matrix,
+// whole call with Z: n = 96 11.96 against 12.91 ms, n = 64 5.92 / 5.94; 256
+// matrices n = 73..96 13.84 / 13.97; 400 18.9 against 14.4).
 hipError_t launch_zqrw(const BatchArgs& a, int nmax, hipStream_t s) {
   if (a.count <= 0) return hipSuccess;
   if (nmax <= zqr_res_max_n()) {
@@ -1854,7 +1941,9 @@ hipError_t launch_zqrw(const BatchArgs& a, int nmax, hipStream_t s) {
     else launch_zqrr<true>(a, nmax, s);
     return hipGetLastError();
   }
-  if (a.flags & 0x1000)
+  if (a.count <= kCoopCount && !(a.flags & 0x1000))
+    hipLaunchKernelGGL((zqrw2_kernel<true, 512>), dim3(a.count), dim3(512), 0, s, a);
+  else if (a.flags & 0x1000)
     hipLaunchKernelGGL((zqrw2_kernel<false>), dim3(a.count), dim3(128), 0, s, a);
   else
     hipLaunchKernelGGL((zqrw2_kernel<true>), dim3(a.count), dim3(128), 0, s, a);
@@ -1884,12 +1973,15 @@ hipError_t launch_fill_i32(int* p, int n, hipStream_t s) {
 
 // One matrix above the LDS-resident orders: wavefront 0 chases, the other
 // nt / 64 - 1 wavefronts of the workgroup share the chains (H's rows above
-// and columns right of the window, and Z), whose count grows with n.
+// and columns right of the window, and Z).  With 512 threads wavefront 0 does
+// nothing but chase: the others store the old window, load the new one and
+// run the left update of its new columns from operands prefetched behind
+// their chains (n = 256, per chunk of at most 29 steps: chase 8.2 us of 15.3
+// before; the call 84.0 -> 69.7 ms, n = 130 23.5 -> 20.7).  1024 threads leave
+// too few registers for the prefetch.
 hipError_t launch_zqrw_single(const BatchArgs& a, int nt, hipStream_t s) {
   if (a.count <= 0) return hipSuccess;
   switch (nt) {
-    case 128: hipLaunchKernelGGL((zqrw2_kernel<true, 128>), dim3(a.count), dim3(128), 0, s, a); break;
-    case 256: hipLaunchKernelGGL((zqrw2_kernel<true, 256>), dim3(a.count), dim3(256), 0, s, a); break;
     case 512: hipLaunchKernelGGL((zqrw2_kernel<true, 512>), dim3(a.count), dim3(512), 0, s, a); break;
     case 1024: hipLaunchKernelGGL((zqrw2_kernel<true, 1024>), dim3(a.count), dim3(1024), 0, s, a); break;
     default: return hipErrorInvalidValue;

@@ -236,3 +236,23 @@ def test_resident_qr_order_edges(gs, oracle, cplx, n):
         N = gs.gschur(M, wantZ=False)
         assert np.array_equal(a.T, N.T) and np.array_equal(a.values, N.values)
         assert np.array_equal(a.T, b.T) and np.array_equal(a.Z, b.Z)
+
+
+@pytest.mark.parametrize("n", [49, 58, 59, 60, 87, 88, 89, 99])
+def test_cooperative_window_order_edges(gs, n):
+    """The 512-thread windowed kernel (one matrix, and small batches) at the
+    edges of its chunks of 29 steps: the same bits as the two-wavefront form
+    that larger batches take, with and without Z.  The matrices deflate in the
+    middle (sweeps that start late) and cycle (exceptional shifts)."""
+    A = gen.ginibre_complex(n, gen.stream(35, 100, n))
+    B = A.copy()
+    B[n // 2:, :n // 2] *= 1e-13
+    mats = [A, B, gen.cyclic_shift(n, True)]
+    Sb, ib = gs.gschur_batched(mats + [A] * 254)
+    Sc, ic = gs.gschur_batched(mats)
+    assert np.all(ib == 0) and np.all(ic == 0)
+    for M, b, c in zip(mats, Sb, Sc):
+        for a in (gs.gschur(M), c):
+            assert np.array_equal(a.T, b.T) and np.array_equal(a.Z, b.Z) and np.array_equal(a.values, b.values)
+        N = gs.gschur(M, wantZ=False)
+        assert np.array_equal(N.T, b.T) and np.array_equal(N.values, b.values)
