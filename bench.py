@@ -197,7 +197,7 @@ def main():
     bytes_alg = float((3.0 * n64 ** 2 * 16 + 16 * n64).sum())
     batch_rate = flops / kern_s
     # dominant kernel: the QR phase of each size bin, the QR-sweep launch
-    # plus (the bin above n = 80) the launch applying its Z log
+    # plus the launch applying its Z log
     qr = [r for r in recs if r["kind"] == "qr"]
     zl = [r for r in recs if r["kind"] == "zlog"]
     hq = [r for r in recs if r["kind"] == "hq"]
@@ -257,10 +257,10 @@ def main():
             "traffic": traffic["bytes_per_launch"] if traffic else None,
             "kernel": ("QR phase of the batch: gs::zqrw2_queue_kernel<true> (two-wavefront windowed QR sweeps, "
                        "one work-queue launch over all size bins, largest matrix first) then gs::zlog_kernel "
-                       "(the Z log of the largest matrices applied with Z in LDS, one launch per logging bin)"
+                       "(the sweeps' Z logs applied with Z's rows in registers, one launch per bin)"
                        if queue else
                        "QR phase of a size bin: gs::zqrw2_kernel<true> (two-wavefront windowed QR sweeps) "
-                       "then, for the bin above n = 80, gs::zlog_kernel (the sweeps' Z log applied with Z in LDS)"),
+                       "then gs::zlog_kernel (the sweeps' Z log applied with Z's rows in registers)"),
             "launches": len(qr),
             "avg_launch_us": qr_us / max(len(qr), 1),
             "qr_sweep_avg_launch_us": sum(r["us"] for r in qr) / max(len(qr), 1),

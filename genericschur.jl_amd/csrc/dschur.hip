@@ -9,8 +9,8 @@
 //
 // Same structure as the complex kernel: one workgroup per matrix; batched
 // matrices take a Hessenberg+Z launch with the matrix in LDS, then the QR
-// launch: by default dqrw_kernel, one wavefront per matrix with H and Z in
-// HBM, the bulge chase in a 32 x 32 LDS window and each chunk's 3-element
+// launch: up to order 62 dqrr_kernel, one wavefront per matrix with H whole in
+// LDS, above dqrw_kernel, one wavefront per matrix with H and Z in HBM, the bulge chase in a 32 x 32 LDS window and each chunk's 3-element
 // reflectors applied to the rest of H and to Z as one chain per row or
 // column; with GS_QR_BAND dqr_kernel, the band j >= i-3 of H in LDS (the
 // double-shift bulge reaches the third subdiagonal).  The single-matrix

@@ -29,7 +29,7 @@ struct BatchArgs {
   int flags;
   int64_t maxiter;   // <= 0: 100 n
   int64_t maxinner;  // <= 0: 30 n
-  // Z log of the complex windowed QR kernel (null: Z updated in place):
+  // Z log of the QR kernels (null: Z updated in place):
   // matrix m's records occupy zlog[2 loff[m] .. 2 loff[m+1]) (complex
   // entries as double pairs); the kernel stores the length used in llen[m]
   double* zlog;

@@ -10,10 +10,10 @@
 //
 // Batched matrices take two or three launches per size bin: zhq_kernel
 // reduces A to Hessenberg form and forms Z with the whole matrix resident
-// in LDS (one workgroup per matrix); zqrw2_kernel runs the QR iterations
-// with H and Z in HBM, two wavefronts per matrix (the bulge chase in a
+// in LDS (one workgroup per matrix); zqrr_kernel (orders up to 48) runs the
+// QR iterations with H whole in LDS, zqrw2_kernel with H and Z in HBM, two wavefronts per matrix (the bulge chase in a
 // 32 x 32 LDS window, and the chunk's reflectors applied to the rest of H
-// and Z as chains); for most bins it logs the Z updates instead and
+// and Z as chains); the Z updates of a batch are logged instead and
 // zlog_kernel applies the log with Z's rows in registers.  zqr_kernel (GS_QR_BAND) keeps
 // H's band j >= i-2 in LDS instead.  The single-matrix kernel keeps H in
 // HBM.

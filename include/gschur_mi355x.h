@@ -57,8 +57,8 @@ typedef struct gs_handle gs_handle;
                              /* apply each chunk's reflectors to Z in HBM      */
                              /* during the QR sweeps instead of logging them   */
                              /* and applying the log to Z after the sweeps     */
-                             /* (batched: Z in LDS; single: Z's rows over the  */
-                             /* GPU); same arithmetic and order (comparisons)  */
+                             /* (Z's rows in registers, or over the GPU);      */
+                             /* same arithmetic and order (comparisons)        */
 #define GS_ZLOG_TINY 0x400   /* complex, testing: a Z log of one sweep per     */
                              /* matrix, so that the QR kernel applies the log  */
                              /* to Z itself before almost every sweep (single: */
@@ -120,10 +120,12 @@ int gs_schur_z(gs_handle* h, int64_t n, double* A, int64_t lda, double* T, int64
  * maxinner is ignored (the reference's real driver has none).
  * Orders above gs_batched_max_n(0) take the large-matrix path unless
  * GS_PLAIN or GS_HESSENBERG is set: blocked Hessenberg reduction and Q
- * formation with FP64 MFMA GEMM updates, then the same double-shift QR
- * iteration with each sweep chased in LDS-resident chunks whose reflectors
- * are applied to the rest of H and to Z by the whole GPU (same per-element
- * update order as the unblocked sweep).  GS_PLAIN runs the unblocked
+ * formation with FP64 MFMA GEMM updates, then the QR iteration with each
+ * sweep chased in LDS-resident chunks whose reflectors are applied to the
+ * rest of H and to Z by the whole GPU: below order 256 the same double-shift
+ * iteration (same per-element update order as the unblocked sweep), from 256
+ * up multishift sweeps of eight double shifts, each counted as eight
+ * iterations, with T's diagonal in an order of their own.  GS_PLAIN runs the unblocked
  * single-workgroup kernel instead. */
 int gs_schur_d(gs_handle* h, int64_t n, double* A, int64_t lda, double* T, int64_t ldt, double* Z, int64_t ldz,
                double* W, int flags, int64_t maxiter, int64_t maxinner, int32_t* info);
@@ -183,10 +185,8 @@ int gs_schur_batched_z_noalloc(gs_handle* h, int64_t count, const int32_t* n, co
  * _xsolve/_safe_lu_solve! util.jl:603-751).  Z may be NULL (vectors of T).
  * V is n x n complex (ldv).  normalize = 0 returns the max-abs1-scaled
  * vectors before _enormalize!.  Orders up to 4096 (GS_E_UNSUPPORTED above):
- * one workgroup per matrix up to 1024 (T in LDS up to 128 complex / 192
- * real, read from global memory above); above 1024 one matrix at a time
- * over the whole GPU, with n x n workspaces (real 40 n^2 bytes, complex
- * 64 n^2) held by the handle. */
+ * one wavefront per column of every matrix over the whole GPU, with
+ * workspaces held by the handle. */
 int gs_trevc_z(gs_handle* h, int64_t n, const double* T, int64_t ldt, const double* Z, int64_t ldz, double* V,
                int64_t ldv, int left, int normalize, int flags);
 int gs_trevc_d(gs_handle* h, int64_t n, const double* T, int64_t ldt, const double* Z, int64_t ldz, double* V,
@@ -344,7 +344,7 @@ int gs_last_stats(const gs_handle* h, int64_t* out, int len);
  *   kind 2      GEMM of the large real path: a, b, c = m, n, k, d = 2 m n k
  *   kind 3      phase of the large real path: a = 0 copy + scale,
  *               1 Hessenberg, 2 Q formation, 3 QR iterations, 4 finish
- *   kind 4      batched complex: the Z log applied after a bin's QR kernel
+ *   kind 4      batched: the Z log applied after a bin's QR kernel
  *               (fields as kind 0 / 1)
  * Writes at most max_records records and returns the number available. */
 #define GS_LAUNCH_REC 6
