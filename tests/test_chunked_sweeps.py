@@ -689,3 +689,144 @@ def test_complex_two_wave_sweep(ZW, case):
     sweep_seq(H1, Z1, istart1, istart, iend, v0, v1)
     sweep_win2(H2, Z2, istart1, istart, iend, v0, v1, ZW)
     assert np.array_equal(H1, H2) and np.array_equal(Z1, Z2)
+
+
+def _ms_first(H, I, s):
+    """first column of (H - s1)(H - s2), s = (r1r, r1i, r2r, r2i), 0-based I"""
+    r1r, r1i, r2r, r2i = s
+    h21 = H[I + 1, I]
+    sx = abs(H[I, I] - r2r) + abs(r2i) + abs(h21)
+    h21 = h21 / sx
+    v = np.array([h21 * H[I, I + 1] + (H[I, I] - r1r) * ((H[I, I] - r2r) / sx) - r1i * (r2i / sx),
+                  h21 * (H[I, I] + H[I + 1, I + 1] - r1r - r2r), h21 * H[I + 2, I + 1]])
+    return v / np.abs(v).sum()
+
+
+def _ms_apply(M, idx, rows, r3):
+    """a 3-element reflector on elements idx .. of lines: rows (left) or columns of M"""
+    tau, v2, v3, nr = r3
+    x = [M[idx + i, :] if rows else M[:, idx + i] for i in range(nr)]
+    ss = x[0] + v2 * x[1] + (v3 * x[2] if nr == 3 else 0.0)
+    for i, f in zip(range(nr), (tau, tau * v2, tau * v3)):
+        x[i][...] = x[i] - ss * f
+
+
+def _ms_times(H, I, E, shifts, SP, t0, t1, lo, hi):
+    """times t0 .. t1 of the train on rows and columns lo .. hi (0-based, both
+    in) of H, in place; returns the reflectors per time and bulge"""
+    log = {}
+    for t in range(t0, t1 + 1):
+        act = []
+        for j, s in enumerate(shifts):
+            k = I + t - SP * j
+            if not I <= k <= E - 1:
+                continue
+            nr = min(3, E - k + 1)
+            x = _ms_first(H, I, s) if k == I else [H[k, k - 1], H[k + 1, k - 1], H[k + 2, k - 1] if nr == 3 else 0.0]
+            tau, beta, v2, v3 = dreflector(nr, x[0], x[1], x[2] if nr == 3 else 0.0)
+            act.append((k, nr, beta))
+            log[t, j] = (tau, v2, v3, nr)
+        for (k, nr, beta), r3 in zip(act, (log[t, j] for j in range(len(shifts)) if (t, j) in log)):
+            if k > I:
+                H[k:k + nr, k - 1] = 0.0
+                H[k, k - 1] = beta
+            _ms_apply(H[:, k:hi + 1], k, True, r3)
+        for (k, nr, beta), r3 in zip(act, (log[t, j] for j in range(len(shifts)) if (t, j) in log)):
+            _ms_apply(H[lo:min(k + 3, E) + 1, :], k, False, r3)
+    return log
+
+
+def _ms_lines(M, rows, log, I, E, SP, NB, t0, t1, LB=8):
+    """ms_lines: bulge j one block of LB times behind bulge j - 1; the element
+    ranges that the bulges touch between two barriers must be disjoint"""
+    nblk = (t1 - t0 + LB) // LB
+    for u in range(nblk + NB - 1):
+        used = set()
+        for j in range(NB):
+            q = u - j
+            if not 0 <= q < nblk:
+                continue
+            lo, hi = max(t0 + LB * q, SP * j), min(t0 + LB * q + LB - 1, t1, E - 1 - I + SP * j)
+            el = set(range(I + lo - SP * j, I + hi - SP * j + 3)) if lo <= hi else set()
+            assert not el & used
+            used |= el
+            for t in range(lo, hi + 1):
+                _ms_apply(M, I + t - SP * j, rows, log[t, j])
+
+
+@pytest.mark.parametrize("NB,NW,I,E", [(8, 89, 0, 199), (8, 89, 5, 68), (8, 89, 3, 130), (4, 30, 0, 69), (4, 30, 7, 47),
+                                       (2, 16, 1, 12)])
+def test_multishift_chunks(NB, NW, I, E):
+    """lms_kernel: the train in chunks (window, new columns, the lines outside
+    two windows) equals the train on the whole matrix bit for bit, writes
+    disjoint regions in one launch, and up to rounding equals NB double-shift
+    sweeps one after the other."""
+    SP, n = 3, E + 6
+    ST = NW - SP * (NB - 1) - 4
+    rng = np.random.default_rng(7 * NB + E)
+    H, Z = _hessenberg(rng.standard_normal((n, n)))
+    if I > 0:
+        H[I, I - 1] = 0.0
+    H[E + 1, E] = 0.0
+    w = np.linalg.eigvals(H[E - 2 * NB + 1:E + 1, E - 2 * NB + 1:E + 1]) if E - I >= 2 * NB else rng.standard_normal(2 * NB)
+    cw, re = [z for z in w if z.imag > 0], [z.real for z in w if z.imag == 0]
+    shifts = [(z.real, z.imag, z.real, -z.imag) for z in cw]
+    shifts += [(a, 0.0, b, 0.0) for a, b in zip(re[::2], re[1::2])]
+    assert len(shifts) == NB
+    nt = E - I + SP * (NB - 1)
+    # whole matrix
+    H1, Z1 = H.copy(), Z.copy()
+    log = _ms_times(H1, I, E, shifts, SP, 0, nt - 1, 0, n - 1)
+    for t in range(nt):
+        for j in range(NB):
+            if (t, j) in log:
+                _ms_apply(Z1, I + t - SP * j, False, log[t, j])
+    # chunks
+    H2, Z2 = H.copy(), Z.copy()
+    nch, prev = -(-nt // ST), None
+    for c in range(nch + 1):
+        done = np.zeros((n, n), dtype=int)
+        cur = None
+        if c < nch:
+            t0, t1 = c * ST, min(c * ST + ST, nt) - 1
+            wb, we = max(I, I + t0 - SP * (NB - 1) - 1), min(E, I + t1 + 3)
+            assert we - wb + 1 <= NW
+        if prev:
+            p0, p1, pb, pe, plog = prev
+            right0 = (we if c < nch else pe) + 1
+            regions = [(slice(pb, pe + 1), slice(right0, n), True), (slice(0, pb), slice(pb, pe + 1), False)]
+            if c < nch:
+                assert we - pe <= 64
+                regions.append((slice(pb, pe + 1), slice(pe + 1, we + 1), True))  # the new columns, first
+            for rs, cs, rows in regions[::-1]:
+                # lines of elements pb .. pe with two zeros behind
+                L = np.zeros((pe + 3, cs.stop - cs.start)) if rows else np.zeros((rs.stop - rs.start, pe + 3))
+                if rows:
+                    L[pb:pe + 1, :] = H2[rs, cs]
+                else:
+                    L[:, pb:pe + 1] = H2[rs, cs]
+                _ms_lines(L, rows, {k: v[:3] + (3,) for k, v in plog.items()}, I, E, SP, NB, p0, p1)
+                H2[rs, cs] = L[pb:pe + 1, :] if rows else L[:, pb:pe + 1]
+                if not (rows and c < nch and cs.start == pe + 1 and cs.stop == we + 1):
+                    done[rs, cs] += 1
+            L = np.hstack([Z2, np.zeros((n, 3))])
+            _ms_lines(L, False, {k: v[:3] + (3,) for k, v in plog.items()}, I, E, SP, NB, p0, p1)
+            Z2 = L[:, :n].copy()
+        if c < nch:
+            done[wb:we + 1, wb:we + 1] += 1
+            if prev:
+                done[pb:wb, pe + 1:we + 1] += 1
+            Wn = H2.copy()
+            plog = _ms_times(Wn, I, E, shifts, SP, t0, t1, wb, we)
+            H2[wb:we + 1, wb:we + 1] = Wn[wb:we + 1, wb:we + 1]
+            cur = (t0, t1, wb, we, plog)
+        assert done.max() <= 1
+        prev = cur
+    assert np.array_equal(H1, H2) and np.array_equal(Z1, Z2)
+    # one sweep after the other
+    H3, Z3 = H.copy(), Z.copy()
+    for s in shifts:
+        unblocked_sweep(H3, Z3, I + 1, I + 1, E + 1, tuple(_ms_first(H3, I, s)))
+    assert np.abs(Z1 @ H1 @ Z1.T - Z3 @ H3 @ Z3.T).max() <= 1e-12 * n * np.abs(H).max()
+    # (rounding-level differences grow along a sweep, here below 1e-9)
+    assert np.abs(H1 - H3).max() <= 1e-7 * np.abs(H).max()
