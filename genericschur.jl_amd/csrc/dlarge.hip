@@ -37,7 +37,13 @@
 
 namespace gs {
 
-constexpr int LNB = 64;  // Hessenberg panel width
+// Hessenberg panel width.  A panel column is one workgroup's serial work that
+// grows with the columns before it in the panel, and bounds the phase; wider
+// panels only make the GEMM updates fewer and better filled.  Measured,
+// Hessenberg phase with 64 / 32 / 16 columns: n = 501 31.4 / 20.1 / 15.8 ms,
+// n = 1500 110.5 / 72.4 / 57.2, n = 4096 479 / 329 / 262 (Q formation 0.9 / 0.9
+// / 1.6, 2.7 / 3.1 / 5.3 and 10 / - / - ms; the n = 4096 solve 1.95 / 1.79 / 1.77 s).
+constexpr int LNB = 16;
 constexpr int LW = 64;   // bulge-chase window (rows and columns)
 constexpr int LKC = LW - 4;  // bulge steps per chunk
 constexpr int LWL = LW + 1;  // odd LDS pitch of a window column (bank spread)
