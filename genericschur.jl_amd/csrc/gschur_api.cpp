@@ -1047,7 +1047,9 @@ static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda
   const size_t es = cplx ? 16 : 8;
   const size_t ed = es / 8;
   const bool dev = (flags & GS_DEVICE_PTRS) != 0;
-  const int kflags = (flags & (GS_WANTZ | GS_SCALE | GS_HESSENBERG | GS_CHECK_SUBDIAG | GS_QR_BAND)) | env_qr_band();
+  const int kflags = (flags & (GS_WANTZ | GS_SCALE | GS_HESSENBERG | GS_CHECK_SUBDIAG | GS_QR_BAND | GS_ZDIRECT |
+                               GS_ZLOG_TINY)) |
+                     env_qr_band();
   // device operands, packed with ld = n when staged
   double *dA, *dT, *dZ, *dW;
   int32_t* dInfo;
@@ -1152,8 +1154,8 @@ static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda
     // order 1024 2.84 -> 2.50 s; orders 256 and 512 slower, 0.216 -> 0.242
     // and 0.434 -> 0.471 s, the replay's row chains outweighing the chains
     // saved)
-    const bool zlg = (kflags & GS_WANTZ) && !(flags & GS_ZDIRECT) && (n >= 768 || (flags & GS_ZLOG_TINY));
-    const int64_t lcap = zlg ? zlog_capacity((int)n, (flags & GS_ZLOG_TINY) != 0) : 0;
+    const bool zlg = (kflags & GS_WANTZ) && !(kflags & GS_ZDIRECT) && (n >= 768 || (kflags & GS_ZLOG_TINY));
+    const int64_t lcap = zlg ? zlog_capacity((int)n, (kflags & GS_ZLOG_TINY) != 0) : 0;
     if (zlg) HIPCHK(h, h->bLog.ensure(16 * (size_t)lcap));
     struct Meta {
       int32_t order, n;

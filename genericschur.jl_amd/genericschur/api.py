@@ -164,10 +164,11 @@ def gschur_(A, wantZ=True, scale=True, maxiter=None, maxinner=None, plain=False,
     Real matrices above the LDS-resident orders take the blocked large-matrix
     path unless plain=True (the unblocked single-workgroup kernel).  With
     timing=True the large path records per-phase and per-GEMM durations
-    (genericschur._lib.last_launches()).  Complex matrices above the
-    LDS-resident orders log Z's updates and apply the log after the sweeps;
-    zdirect=True updates Z during the sweeps instead, zlog_tiny=True makes
-    the log hold one sweep (comparisons; the results are the same)."""
+    (genericschur._lib.last_launches()).  Orders up to 48 (complex) / 62
+    (real) and complex ones from 768 log Z's updates and apply the log after
+    the sweeps; zdirect=True updates Z during the sweeps instead,
+    zlog_tiny=True makes the log hold one sweep (comparisons; the results are
+    the same)."""
     if _is_torch(A):
         raise TypeError("use gschur_device / gschur_batched_device for device tensors")
     A = np.asarray(A)

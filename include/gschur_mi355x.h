@@ -53,15 +53,17 @@ typedef struct gs_handle gs_handle;
                              /* (up to 80 KB per matrix) instead of the        */
                              /* default windowed kernel (H in HBM, a 32 x 32   */
                              /* chase window in LDS); same arithmetic           */
-#define GS_ZDIRECT 0x200     /* complex (batched, and single from order 768):  */
-                             /* apply each chunk's reflectors to Z in HBM      */
+#define GS_ZDIRECT 0x200     /* apply each chunk's reflectors to Z in HBM      */
                              /* during the QR sweeps instead of logging them   */
                              /* and applying the log to Z after the sweeps     */
-                             /* (Z's rows in registers, or over the GPU);      */
-                             /* same arithmetic and order (comparisons)        */
-#define GS_ZLOG_TINY 0x400   /* complex, testing: a Z log of one sweep per     */
-                             /* matrix, so that the QR kernel applies the log  */
-                             /* to Z itself before almost every sweep (single: */
+                             /* (Z's rows in registers, or over the GPU).  For */
+                             /* calls that log: batches (real: bins up to 128),*/
+                             /* single matrices up to 48 complex / 62 real and */
+                             /* complex ones from 768; same arithmetic and     */
+                             /* order (comparisons)                            */
+#define GS_ZLOG_TINY 0x400   /* testing: a Z log of one sweep per matrix, so   */
+                             /* that the QR kernel applies the log to Z itself */
+                             /* before almost every sweep (single complex:     */
                              /* the log at any order above the LDS range)      */
 #define GS_SORT 0x800       /* Hermitian eigensolver: eigenvalues ascending, */
                              /* eigenvectors alike (sorteig! with eigsortby)  */

@@ -209,10 +209,11 @@ def test_log_replay_order_edges(gs, cplx, n):
 def test_resident_qr_order_edges(gs, oracle, cplx, n):
     """QR with the matrix held in LDS, at the edges of its pitch classes and of
     its range: the checks against the oracle for a matrix alone, the same bits
-    in a batch that takes the windowed kernels (complex: beside larger orders;
-    real: above the widest class's launch size), with Z updated in place, with
-    a one-sweep log, and T without Z.  The matrices deflate in the middle,
-    are scaled to near underflow, and cycle (exceptional shifts)."""
+    in a batch that takes the windowed kernels (complex: the work queue of more
+    than 256 matrices with larger orders among them; real: above the widest
+    class's launch size), with Z updated in place, with a one-sweep log, and T
+    without Z.  The matrices deflate in the middle, are scaled to near
+    underflow, and cycle (exceptional shifts)."""
     rng = gen.stream(34, 100, n)
     A = gen.ginibre_complex(n, rng) if cplx else gen.ginibre_real(n, rng)
     B = A.copy()
@@ -221,8 +222,12 @@ def test_resident_qr_order_edges(gs, oracle, cplx, n):
     S1 = [gs.gschur(M) for M in mats]
     for M, S in zip(mats[:2], S1):
         _check(oracle, M, S)
+    for kw in ({"zdirect": True}, {"zlog_tiny": True}):
+        for M, a in zip(mats, S1):
+            b = gs.gschur(M, **kw)
+            assert np.array_equal(a.T, b.T) and np.array_equal(a.Z, b.Z) and np.array_equal(a.values, b.values)
     if cplx:
-        rest = [gen.ginibre_complex(60, rng)]
+        rest = [gen.ginibre_complex(60, rng) for _ in range(256)]
     else:
         rest = [A] * 4097 if n in (49, 62) else []
     for kw in ({}, {"zdirect": True}, {"zlog_tiny": True}):
@@ -230,12 +235,15 @@ def test_resident_qr_order_edges(gs, oracle, cplx, n):
         assert np.all(ib == 0)
         for a, b in zip(S1, Sb):
             assert np.array_equal(a.T, b.T) and np.array_equal(a.Z, b.Z) and np.array_equal(a.values, b.values)
-        rest = rest[:1]
-    Sb, _ = gs.gschur_batched(mats)
-    for a, M, b in zip(S1, mats, Sb):
+        if not cplx:
+            rest = rest[:1]
+    for kw in ({}, {"zdirect": True}, {"zlog_tiny": True}):
+        Sb, _ = gs.gschur_batched(mats, **kw)
+        for a, b in zip(S1, Sb):
+            assert np.array_equal(a.T, b.T) and np.array_equal(a.Z, b.Z)
+    for a, M in zip(S1, mats):
         N = gs.gschur(M, wantZ=False)
         assert np.array_equal(a.T, N.T) and np.array_equal(a.values, N.values)
-        assert np.array_equal(a.T, b.T) and np.array_equal(a.Z, b.Z)
 
 
 @pytest.mark.parametrize("n", [49, 58, 59, 60, 87, 88, 89, 99])
