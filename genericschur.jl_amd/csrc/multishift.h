@@ -122,6 +122,28 @@ GS_DEV void ms_lines(double* buf, const double* lg, int t0, int t1, int I, int E
   }
 }
 
+// First column of (H - s1)(H - s2) (GenericSchur.jl:851-876) from H's leading
+// entries and the shifts sh (r1r, r1i, r2r, r2i), scaled to unit 1-norm.  The
+// block is unreduced when the sweep begins, but the bulges after the first
+// meet the entries that those before them have left: a column that has
+// vanished gives zeros (an identity reflector: that bulge moves nothing), not
+// a quotient by zero.
+__host__ GS_DEV void ms_first(double h11, double h12, double h21, double h22, double h32, const double* sh, double& v0,
+                              double& v1, double& v2) {
+  v0 = v1 = v2 = 0.0;
+  double sx = fabs(h11 - sh[2]) + fabs(sh[3]) + fabs(h21);
+  if (sx == 0.0) return;
+  h21 = h21 / sx;
+  const double w0 = h21 * h12 + (h11 - sh[0]) * ((h11 - sh[2]) / sx) - sh[1] * (sh[3] / sx);
+  const double w1 = h21 * (h11 + h22 - sh[0] - sh[2]);
+  const double w2 = h21 * h32;
+  sx = fabs(w0) + fabs(w1) + fabs(w2);
+  if (sx == 0.0) return;
+  v0 = w0 / sx;
+  v1 = w1 / sx;
+  v2 = w2 / sx;
+}
+
 // Times t0 .. t1 of the train in the window win (rows and columns wb .. we,
 // entry (r, c) at win[(r - wb) + (c - wb) MWP]), wavefront j with bulge j;
 // the reflectors (tau, v2, v3) to lg[3 ((t - t0) MNB + j)].  Per time: the
@@ -135,7 +157,6 @@ GS_DEV void ms_chase(double* win, double* lg, const double* sh, int t0, int t1, 
   const int lane = threadIdx.x & 63;
   const int j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   auto W = [&](int r, int c) -> double& { return win[(r - wb) + (c - wb) * MWP]; };
-  const double r1r = sh[4 * j], r1i = sh[4 * j + 1], r2r = sh[4 * j + 2], r2i = sh[4 * j + 3];
   double nv0 = 0.0, nv1 = 0.0, nv2 = 0.0;
   int k = I + t0 - MSP * j;
   if (k > I && k <= E - 1) {
@@ -191,18 +212,7 @@ GS_DEV void ms_chase(double* win, double* lg, const double* sh, int t0, int t1, 
       }
     } else if (act) {
       if (k == I) {
-        // first column of (H - s1)(H - s2) (GenericSchur.jl:851-876)
-        const double h11 = W(I, I), h12 = W(I, I + 1), h22 = W(I + 1, I + 1), h32 = W(I + 2, I + 1);
-        double h21 = W(I + 1, I);
-        double sx = fabs(h11 - r2r) + fabs(r2i) + fabs(h21);
-        h21 = h21 / sx;
-        nv0 = h21 * h12 + (h11 - r1r) * ((h11 - r2r) / sx) - r1i * (r2i / sx);
-        nv1 = h21 * (h11 + h22 - r1r - r2r);
-        nv2 = h21 * h32;
-        sx = fabs(nv0) + fabs(nv1) + fabs(nv2);
-        nv0 /= sx;
-        nv1 /= sx;
-        nv2 /= sx;
+        ms_first(W(I, I), W(I, I + 1), W(I + 1, I), W(I + 1, I + 1), W(I + 2, I + 1), sh + 4 * j, nv0, nv1, nv2);
       }
       double beta = nv0;
       v2 = nv1;

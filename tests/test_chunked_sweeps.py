@@ -9,6 +9,10 @@ compare the result with the unblocked sweep of the reference
 operations: H and Z must be bitwise equal, and the regions that the large
 path's workgroups write in one launch must be disjoint.  CPU only.
 """
+import os
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -830,3 +834,40 @@ def test_multishift_chunks(NB, NW, I, E):
     assert np.abs(Z1 @ H1 @ Z1.T - Z3 @ H3 @ Z3.T).max() <= 1e-12 * n * np.abs(H).max()
     # (rounding-level differences grow along a sweep, here below 1e-9)
     assert np.abs(H1 - H3).max() <= 1e-7 * np.abs(H).max()
+
+
+MS_FIRST_MAIN = r"""
+#include <cstdio>
+#include "multishift.h"
+int main() {
+  double x[9];
+  while (scanf("%lf %lf %lf %lf %lf %lf %lf %lf %lf", x, x + 1, x + 2, x + 3, x + 4, x + 5, x + 6, x + 7, x + 8) == 9) {
+    double v0, v1, v2;
+    gs::ms_first(x[0], x[1], x[2], x[3], x[4], x + 5, v0, v1, v2);
+    printf("%.17g %.17g %.17g\n", v0, v1, v2);
+  }
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="compiles the kernels' header for the host")
+def test_multishift_first_column(tmp_path):
+    """The first column of a bulge of the train (multishift.h, compiled for the
+    host): the model's where it exists, and zeros, never NaN, where the bulges
+    before it have made it vanish."""
+    src = tmp_path / "first.hip"
+    src.write_text(MS_FIRST_MAIN)
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "genericschur.jl_amd", "csrc")
+    exe = str(tmp_path / "first")
+    subprocess.run(["hipcc", "--offload-host-only", "-O1", "-std=c++17", "-I", csrc, str(src), "-o", exe], check=True)
+    rng = np.random.default_rng(11)
+    rows = [list(rng.standard_normal(9)) for _ in range(20)]
+    zero = [[0.5, 2.0, 0.0, 1.0, 3.0, 0.25, 0.0, 0.5, 0.0],   # h21 = 0 and h11 the second shift
+            [0.5, 2.0, 0.0, 1.0, 3.0, 0.5, 0.0, 0.25, 0.0]]   # h21 = 0 and h11 the first shift
+    text = "".join(" ".join(f"{v:.17g}" for v in r) + chr(10) for r in rows + zero)
+    out = subprocess.run([exe], input=text, text=True, capture_output=True, check=True).stdout
+    got = np.array([[float(v) for v in line.split()] for line in out.splitlines()])
+    for r, g in zip(rows, got):
+        H = np.array([[r[0], r[1], 0.0], [r[2], r[3], 0.0], [0.0, r[4], 0.0]])
+        assert np.allclose(g, _ms_first(H, 0, r[5:]), rtol=1e-13, atol=0)
+    assert np.array_equal(got[len(rows):], np.zeros((2, 3)))
