@@ -218,3 +218,25 @@ def test_multishift_orders(gs, n):
             assert np.max(d) <= 1e4 * n * eps * np.linalg.norm(A, 2)
     with pytest.raises(gs.UnconvergedException):
         gs.gschur(gen.ginibre_real(n, gen.stream(26, 101, n)), maxiter=20)
+
+
+def test_multishift_nan_fails_as_fast(gs):
+    """A NaN never deflates: the iteration ends at its limit, and a sweep over
+    NaN takes no longer than one over numbers (the shifts' own QR iteration,
+    which cannot converge on it, is not tried)."""
+    import time
+    n = 256
+    A = gen.ginibre_real(n, gen.stream(27, 100, n))
+    B = A.copy()
+    B[3, 5] = np.nan
+    times = []
+    for M in (A, B):
+        t = []
+        for _ in range(4):
+            t0 = time.perf_counter()
+            with pytest.raises(gs.UnconvergedException):
+                gs.gschur(M, maxiter=160)
+            t.append(time.perf_counter() - t0)
+        times.append(min(t))
+    print(f"20 sweeps: {1e3 * times[0]:.1f} ms, with a NaN {1e3 * times[1]:.1f} ms", flush=True)
+    assert times[1] <= 2.5 * times[0]
