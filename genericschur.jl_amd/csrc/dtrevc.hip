@@ -489,6 +489,15 @@ template <int R, class VEC> GS_DEV void enormalize_w(VEC& v, int n) {
 // so within a run of nonzero subdiagonal entries (one entry, for a
 // quasi-triangular T) the distance from the end where the walk enters it
 // decides.
+template <class SUB> GS_DEV int dtrevc_kind(const SUB& sub, int j, bool left) {
+  int d = 0;
+  if (left) {
+    while (sub(j - 1 - d) != 0.0) ++d;
+    return (d & 1) ? 2 : (sub(j) != 0.0 ? 1 : 0);
+  }
+  while (sub(j + d) != 0.0) ++d;
+  return (d & 1) ? 2 : (sub(j - 1) != 0.0 ? -1 : 0);
+}
 __global__ void __launch_bounds__(256) dtrevc_norms_kernel(TrevcArgs a) {
   const TrevcMat<double> t = trevc_mat<double>(a, blockIdx.y);
   const int n = t.n;
@@ -501,14 +510,7 @@ __global__ void __launch_bounds__(256) dtrevc_norms_kernel(TrevcArgs a) {
   auto sub = [&](int i) { return (i >= 0 && i + 1 < n) ? t.T[(i + 1) + (int64_t)i * t.ldt] : 0.0; };
   t.cn[j] = s;
   t.sub[j] = sub(j);
-  int d = 0;
-  if (a.left) {
-    while (sub(j - 1 - d) != 0.0) ++d;
-    t.kind[j] = (d & 1) ? 2 : (sub(j) != 0.0 ? 1 : 0);
-  } else {
-    while (sub(j + d) != 0.0) ++d;
-    t.kind[j] = (d & 1) ? 2 : (sub(j - 1) != 0.0 ? -1 : 0);
-  }
+  t.kind[j] = dtrevc_kind(sub, j, a.left != 0);
 }
 
 // workgroup (t, matrix) solves column n-1-t (right) or t (left): the longest
@@ -542,55 +544,28 @@ template <int R, bool LEFT> __global__ void __launch_bounds__(64) dtrevc_solve_k
   }
 }
 
-template <int R> __global__ void __launch_bounds__(64) dtrevc_finish_kernel(TrevcArgs a) {
-  extern __shared__ double smem[];
-  const TrevcMat<double> t = trevc_mat<double>(a, blockIdx.y);
-  const int n = t.n, lane = threadIdx.x & 63, ki = blockIdx.x;
-  if (ki >= n) return;
-  const bool left = a.left != 0;
-  const int kd = t.kind[ki];
-  if (kd == 2) return;
-  WaveVec<R> y;
-  wavevec_bind(y.v, smem);
-  const int lo = left ? ki : 0, hi = left ? n : ki + 1;
-  zd* vo = t.V + (int64_t)ki * t.ldv;
+// Scaling and normalization of column ki, and its store with a pair's partner.
+// y: the column of Z X (whole), or without Z of X (entries lo .. hi - 1).  edge:
+// a column of Z itself, which the reference only normalizes.
+template <int R, class VEC> GS_DEV void dtrevc_store(const TrevcMat<double>& t, VEC& y, int ki, int kd, bool left,
+                                                     bool normalize, bool edge) {
+  const int n = t.n, lane = threadIdx.x & 63;
+  const bool conj = !left && kd == -1;
+  auto flip = [&] {
+#pragma unroll
+    for (int q = 0; q < R; ++q) y.v[q] = zconj(y.v[q]);
+  };
   if (t.Z) {
-    if ((!left && ki == 0 && kd == 0) || (left && ki == n - 1 && kd == 0)) {
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = lane + 64 * q;
-        y.v[q] = (r < n) ? zr(t.Z[r + (int64_t)ki * t.ldz]) : zr(0.0);
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = lane + 64 * q;
-        y.v[q] = (r < n) ? vo[r] : zr(0.0);
-      }
+    if (!edge) {
       scale_by_max<R>(y, 0, n, false);
-      if (!left && kd == -1) {
-#pragma unroll
-        for (int q = 0; q < R; ++q) y.v[q] = zconj(y.v[q]);
-      }
+      if (conj) flip();
     }
   } else {
-    const zd* xo = t.X + (int64_t)ki * n;
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int i = lane + 64 * q;
-      y.v[q] = (i >= lo && i < hi) ? xo[i] : zr(0.0);
-    }
-    if (kd == 0) {
-      scale_by_max<R>(y, lo, hi, false);
-    } else {
-      if (!left) {
-#pragma unroll
-        for (int q = 0; q < R; ++q) y.v[q] = zconj(y.v[q]);
-      }
-      scale_by_max<R>(y, lo, hi, true);
-    }
+    if (conj) flip();
+    scale_by_max<R>(y, left ? ki : 0, left ? n : ki + 1, kd != 0);
   }
-  if (a.normalize) enormalize_w<R>(y, n);
+  if (normalize) enormalize_w<R>(y, n);
+  zd* vo = t.V + (int64_t)ki * t.ldv;
   zd* po = t.V + (int64_t)(left ? ki + 1 : ki - 1) * t.ldv;
 #pragma unroll
   for (int q = 0; q < R; ++q) {
@@ -602,6 +577,91 @@ template <int R> __global__ void __launch_bounds__(64) dtrevc_finish_kernel(Trev
       if (kd != 0) po[r] = zconj(z);
     }
   }
+}
+
+GS_DEV bool dtrevc_edge(int n, int ki, int kd, bool left) { return kd == 0 && ki == (left ? n - 1 : 0); }
+
+template <int R> __global__ void __launch_bounds__(64) dtrevc_finish_kernel(TrevcArgs a) {
+  extern __shared__ double smem[];
+  const TrevcMat<double> t = trevc_mat<double>(a, blockIdx.y);
+  const int n = t.n, lane = threadIdx.x & 63, ki = blockIdx.x;
+  if (ki >= n) return;
+  const bool left = a.left != 0;
+  const int kd = t.kind[ki];
+  if (kd == 2) return;
+  WaveVec<R> y;
+  wavevec_bind(y.v, smem);
+  const int lo = left ? ki : 0, hi = left ? n : ki + 1;
+  const bool edge = dtrevc_edge(n, ki, kd, left);
+  const zd* vo = t.V + (int64_t)ki * t.ldv;
+  const zd* xo = t.X + (int64_t)ki * n;
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int r = lane + 64 * q;
+    zd v = zr(0.0);
+    if (t.Z) {
+      if (r < n) v = edge ? zr(t.Z[r + (int64_t)ki * t.ldz]) : vo[r];
+    } else {
+      if (r >= lo && r < hi) v = xo[r];
+    }
+    y.v[q] = v;
+  }
+  dtrevc_store<R>(t, y, ki, kd, left, a.normalize != 0, edge);
+}
+
+// Orders up to kTrevcSmallN: the columns of a matrix by the wavefronts of one
+// workgroup, T in LDS (pitch NM + 1), the back-transform and the scaling in the
+// solving wavefront's registers.
+template <int NM, bool LEFT> __global__ void __launch_bounds__(1024) dtrevc_small_kernel(TrevcArgs a) {
+  extern __shared__ double smem[];  // DFac[NM] per wavefront
+  constexpr int P = NM + 1;
+  __shared__ double Ts[P * NM], cn[NM], sub[NM];
+  __shared__ int kind[NM];
+  const TrevcMat<double> t = trevc_mat<double, false>(a, blockIdx.x);
+  const int n = t.n, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  trevc_stage<P>(t, false, Ts, cn);
+  if ((int)threadIdx.x < n) {
+    auto sb = [&](int i) { return (i >= 0 && i + 1 < n) ? Ts[(i + 1) + i * P] : 0.0; };
+    sub[threadIdx.x] = sb(threadIdx.x);
+    kind[threadIdx.x] = dtrevc_kind(sb, threadIdx.x, LEFT);
+  }
+  __syncthreads();
+  const double ulp = GS_EPS;
+  const double smallnum = GS_FMIN * ((double)n / ulp);  // vectors.jl:146,475
+  const double bignum = (1.0 - ulp) / smallnum;
+  const ColG<double> Tc{Ts, P};
+  DFac* const fac = reinterpret_cast<DFac*>(smem) + NM * wave;
+  for (int b = wave; b < n; b += blockDim.x >> 6) {
+    const int ki = LEFT ? b : n - 1 - b;
+    const int kd = __builtin_amdgcn_readfirstlane(kind[ki]);
+    if (kd == 2) continue;
+    WaveVec<1> y;
+    if (!LEFT) dsolve_right<1>(Tc, sub, cn, ki, kd, smallnum, bignum, y, fac);
+    else dsolve_left<1>(Tc, sub, cn, n, ki, kd, smallnum, bignum, y, fac);
+    const int lo = LEFT ? ki : 0, hi = LEFT ? n : ki + 1;
+    if (!(lane >= lo && lane < hi)) y.v[0] = zr(0.0);
+    const bool edge = dtrevc_edge(n, ki, kd, LEFT);
+    if (t.Z) {
+      if (edge) y.v[0] = lane < n ? zr(t.Z[lane + (int64_t)ki * t.ldz]) : zr(0.0);
+      else y.v[0] = trevc_back_small(t, y, lo, hi - 1);
+    }
+    dtrevc_store<1>(t, y, ki, kd, LEFT, a.normalize != 0, edge);
+  }
+}
+
+static hipError_t launch_dtrevc_small(const TrevcArgs& a, int nmax, hipStream_t s) {
+  const int nw = trevc_small_waves(a.count);
+  if (nmax <= 16) {
+    const size_t lds = 16 * sizeof(DFac) * nw;
+    if (a.left) hipLaunchKernelGGL((dtrevc_small_kernel<16, true>), dim3(a.count), dim3(64 * nw), lds, s, a);
+    else hipLaunchKernelGGL((dtrevc_small_kernel<16, false>), dim3(a.count), dim3(64 * nw), lds, s, a);
+  } else {
+    const size_t lds = 32 * sizeof(DFac) * nw;
+    if (a.left) hipLaunchKernelGGL((dtrevc_small_kernel<32, true>), dim3(a.count), dim3(64 * nw), lds, s, a);
+    else hipLaunchKernelGGL((dtrevc_small_kernel<32, false>), dim3(a.count), dim3(64 * nw), lds, s, a);
+  }
+  return hipGetLastError();
 }
 
 template <int R> static hipError_t launch_dtrevc_r(const TrevcArgs& a, int nmax, hipStream_t s) {
@@ -621,6 +681,7 @@ template <int R> static hipError_t launch_dtrevc_r(const TrevcArgs& a, int nmax,
 }
 
 hipError_t launch_dtrevc(const TrevcArgs& a, int nmax, hipStream_t s) {
+  if (nmax <= kTrevcSmallN) return launch_dtrevc_small(a, nmax, s);
   switch (trevc_class(nmax)) {
     case 1: return launch_dtrevc_r<1>(a, nmax, s);
     case 2: return launch_dtrevc_r<2>(a, nmax, s);
@@ -639,7 +700,7 @@ int trevc_max_n() { return 4096; }
 // (left), and 8 n + 8 n + 4 n for norms, subdiagonal and kinds; each array
 // 256-byte aligned.  A group ends where the next matrix needs another class,
 // would take the workspace above kGroupBytes, or fills the grid's z
-// dimension.
+// dimension; the small orders, without workspace, are one group.
 constexpr size_t kGroupBytes = size_t(1) << 30;
 constexpr int kGroupCount = 32768;
 static size_t seg(size_t bytes) { return (bytes + 255) & ~size_t(255); }
@@ -647,8 +708,8 @@ static size_t seg(size_t bytes) { return (bytes + 255) & ~size_t(255); }
 void trevc_groups(const int32_t* n, const int32_t* order, int64_t count, bool cplx, TrevcPlan& p) {
   const size_t es = cplx ? 16 : 8;
   p.groups.clear();
-  p.wsn.assign((size_t)count, 0);
-  p.wsnn.assign((size_t)count, 0);
+  p.wsn.clear();
+  p.wsnn.clear();
   p.bytes = 0;
   for (int64_t q = 0; q < count;) {
     if (n[order[q]] <= 0) break;  // descending: only empty matrices remain
@@ -658,12 +719,14 @@ void trevc_groups(const int32_t* n, const int32_t* order, int64_t count, bool cp
     const int cls = trevc_class(g.nmax);
     int64_t sn = 0, snn = 0;
     int64_t k = q;
-    for (; k < count && k - q < kGroupCount; ++k) {
+    const bool small = g.nmax <= kTrevcSmallN;
+    while (small && k < count && n[order[k]] > 0) ++k;
+    for (; !small && k < count && k - q < kGroupCount; ++k) {
       const int64_t m = n[order[k]];
-      if (m <= 0 || trevc_class((int)m) != cls) break;
+      if (m <= kTrevcSmallN || trevc_class((int)m) != cls) break;
       if (k > q && (16 + es) * (size_t)(snn + m * m) > kGroupBytes) break;
-      p.wsn[k] = sn;
-      p.wsnn[k] = snn;
+      p.wsn.push_back(sn);
+      p.wsnn.push_back(snn);
       sn += m;
       snn += m * m;
     }
@@ -671,6 +734,7 @@ void trevc_groups(const int32_t* n, const int32_t* order, int64_t count, bool cp
     g.sn = sn;
     g.snn = snn;
     p.groups.push_back(g);
+    if (small) break;  // the last: without workspace
     p.bytes = std::max(p.bytes, seg(16 * (size_t)snn) + seg(es * (size_t)snn) + 2 * seg(8 * (size_t)sn) +
                                     seg(4 * (size_t)sn));
     q = k;
@@ -693,8 +757,10 @@ hipError_t launch_trevc(bool cplx, TrevcArgs a, const TrevcPlan& p, void* ws, hi
     w += seg(8 * (size_t)g.sn);
     a.wkind = reinterpret_cast<int*>(w);
     a.order = order + g.first;
-    a.wsn = wsn + g.first;
-    a.wsnn = wsnn + g.first;
+    if (g.nmax > kTrevcSmallN) {
+      a.wsn = wsn + g.first;
+      a.wsnn = wsnn + g.first;
+    }
     a.count = (int)g.count;
     const hipError_t e = cplx ? launch_ztrevc(a, g.nmax, s) : launch_dtrevc(a, g.nmax, s);
     if (e != hipSuccess) return e;

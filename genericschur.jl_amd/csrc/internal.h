@@ -149,12 +149,13 @@ struct TrevcGroup {
 };
 struct TrevcPlan {
   std::vector<TrevcGroup> groups;
-  std::vector<int64_t> wsn, wsnn;
+  std::vector<int64_t> wsn, wsnn;  // of the leading matrices, which take a workspace
   size_t bytes = 0;  // workspace
 };
 void trevc_groups(const int32_t* n, const int32_t* order, int64_t count, bool cplx, TrevcPlan& p);
 int trevc_max_n();
-// a: order, wsn, wsnn whole device arrays; ws holds p.bytes of device memory
+// a: order, wsn, wsnn whole device arrays (wsn, wsnn of p's length); ws holds
+// p.bytes of device memory
 hipError_t launch_trevc(bool cplx, TrevcArgs a, const TrevcPlan& p, void* ws, hipStream_t s);
 // one group (a.order .. a.wkind the group's own)
 hipError_t launch_ztrevc(const TrevcArgs& a, int nmax, hipStream_t s);

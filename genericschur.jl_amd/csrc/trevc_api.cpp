@@ -48,19 +48,24 @@ int run_trevc(gs_handle* h, bool cplx, int64_t count, const int32_t* n, const in
   DevBuf& meta = handle_buf(h, 0);
   TrevcPlan plan;
   trevc_groups(n, order.data(), count, cplx, plan);
-  const size_t mbytes = sizeof(int32_t) * 2 * count + sizeof(int64_t) * 3 * count;
+  const int64_t nws = (int64_t)plan.wsn.size();
+  const size_t mbytes = sizeof(int32_t) * 2 * count + sizeof(int64_t) * (count + 2 * nws);
   if ((e = meta.ensure(mbytes)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
   char* mp = static_cast<char*>(meta.p);
   int64_t* d_off = reinterpret_cast<int64_t*>(mp);
-  int32_t* d_n = reinterpret_cast<int32_t*>(d_off + 3 * count);
+  int32_t* d_n = reinterpret_cast<int32_t*>(d_off + count + 2 * nws);
   int32_t* d_order = d_n + count;
   std::vector<char> hm(mbytes);
-  const size_t c8 = sizeof(int64_t) * count, c4 = sizeof(int32_t) * count;
-  std::memcpy(hm.data(), off, c8);
-  std::memcpy(hm.data() + c8, plan.wsn.data(), c8);
-  std::memcpy(hm.data() + 2 * c8, plan.wsnn.data(), c8);
-  std::memcpy(hm.data() + 3 * c8, n, c4);
-  std::memcpy(hm.data() + 3 * c8 + c4, order.data(), c4);
+  char* hp = hm.data();
+  auto put = [&](const void* src, size_t bytes) {
+    if (bytes > 0) std::memcpy(hp, src, bytes);
+    hp += bytes;
+  };
+  put(off, sizeof(int64_t) * count);
+  put(plan.wsn.data(), sizeof(int64_t) * nws);
+  put(plan.wsnn.data(), sizeof(int64_t) * nws);
+  put(n, sizeof(int32_t) * count);
+  put(order.data(), sizeof(int32_t) * count);
   if ((e = hipMemcpyAsync(meta.p, hm.data(), mbytes, hipMemcpyHostToDevice, s)) != hipSuccess)
     return handle_fail_hip(h, e, "hipMemcpyAsync");
   const double *dT = T, *dZ = Z;
@@ -104,9 +109,9 @@ int run_trevc(gs_handle* h, bool cplx, int64_t count, const int32_t* n, const in
   a.ldz = single ? ldz : 0;
   a.ldv = single ? ldv : 0;
   a.wsn = d_off + count;
-  a.wsnn = d_off + 2 * count;
+  a.wsnn = d_off + count + nws;
   DevBuf& ws = handle_buf(h, 4);
-  if ((e = ws.ensure(plan.bytes)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
+  if (plan.bytes > 0 && (e = ws.ensure(plan.bytes)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
   if ((e = launch_trevc(cplx, a, plan, ws.p, s)) != hipSuccess) return handle_fail_hip(h, e, "kernel launch");
   if (!dev) {
     if (single) {

@@ -11,7 +11,8 @@
 //   4. back-transform Z X as FP64 MFMA tiles (trevc_back_kernel);
 //   5. one wavefront per column scales and normalises in V.
 //
-// The list is processed in classes of orders that need the same number R of
+// The orders up to kTrevcSmallN go through one launch of their own.  The rest of
+// the list is processed in classes of orders that need the same number R of
 // entries per lane.  Bound by the latency of the substitutions, of which one
 // matrix has n in flight and a batch n per matrix.  Before, one workgroup of
 // 4 wavefronts per matrix solved its n columns in turn with T's triangle in
@@ -42,10 +43,11 @@ template <class E> struct TrevcMat {
   double* sub; // n (real)
   int* kind;   // n (real)
 };
-template <class E> GS_DEV TrevcMat<E> trevc_mat(const TrevcArgs& a, int q) {
+// WS: with the workspace segments.
+template <class E, bool WS = true> GS_DEV TrevcMat<E> trevc_mat(const TrevcArgs& a, int q) {
   const int m = a.order[q];
   const int n = a.n[m];
-  const int64_t o = a.off[m], w = a.wsn[q], ww = a.wsnn[q];
+  const int64_t o = a.off[m];
   TrevcMat<E> t;
   t.n = n;
   t.T = reinterpret_cast<const E*>(a.T) + o;
@@ -54,11 +56,14 @@ template <class E> GS_DEV TrevcMat<E> trevc_mat(const TrevcArgs& a, int q) {
   t.ldt = a.ldt > 0 ? a.ldt : n;
   t.ldz = a.ldz > 0 ? a.ldz : n;
   t.ldv = a.ldv > 0 ? a.ldv : n;
-  t.X = reinterpret_cast<zd*>(a.wX) + ww;
-  t.Tt = reinterpret_cast<E*>(a.wT) + ww;
-  t.cn = a.wcn + w;
-  t.sub = a.wsub + w;
-  t.kind = a.wkind + w;
+  if constexpr (WS) {
+    const int64_t w = a.wsn[q], ww = a.wsnn[q];
+    t.X = reinterpret_cast<zd*>(a.wX) + ww;
+    t.Tt = reinterpret_cast<E*>(a.wT) + ww;
+    t.cn = a.wcn + w;
+    t.sub = a.wsub + w;
+    t.kind = a.wkind + w;
+  }
   return t;
 }
 
@@ -184,6 +189,50 @@ template <class E> __global__ void __launch_bounds__(256) trevc_back_kernel(Trev
         const int gr = r0 + wr + 16 * i + (lane & 15), gc = c0 + wc + 16 * j + (lane >> 4) + 4 * r;
         if (gr < n && gc < n) t.V[gr + (int64_t)gc * t.ldv] = zmk(re[i][j][r], im[i][j][r]);
       }
+}
+
+// Orders up to this take one launch of a workgroup per matrix (the small
+// kernels of ztrevc.hip and dtrevc.hip) instead of the four or five over the
+// columns, whose launches cost a small matrix more than its solves, and a large
+// batch the solutions' way through memory.  Measured, complex, five launches /
+// one: one matrix n = 2 35 / 26 us, n = 16 39 / 33, n = 24 45 / 42, n = 32 47 / 55;
+// 16384 of n = 16 1.41 / 0.94 ms, of n = 32 3.16 / 2.08 (real 1.64 / 1.02 and
+// 3.77 / 2.06).
+constexpr int kTrevcSmallN = 32;
+
+// Wavefronts of a small matrix's workgroup: one per column or two where the
+// matrices are fewer than the CUs, down to four where they fill the GPU.
+// Measured, 16 / 8 / 4: one complex matrix n = 32 55 / 62 / 89 us, 1000 of n =
+// 4..24 99 / 97 / 105, 16384 of n = 16 1.05 / 0.97 / 0.94 ms (real 1.35 / 1.15 /
+// 1.02).
+inline int trevc_small_waves(int count) { return count <= 256 ? 16 : (count <= 1024 ? 8 : 4); }
+
+// A small matrix in LDS with pitch P: T, and its strictly upper column norms
+// by one lane per column.  Every thread of the workgroup calls it.
+template <int P, class E> GS_DEV void trevc_stage(const TrevcMat<E>& t, bool abs1, E* Ts, double* cn) {
+  constexpr int NM = P - 1;
+  const int n = t.n, r = threadIdx.x % NM;
+  for (int c = threadIdx.x / NM; c < n; c += blockDim.x / NM)
+    if (r < n) Ts[r + c * P] = t.T[r + (int64_t)c * t.ldt];
+  __syncthreads();
+  if ((int)threadIdx.x < n) {
+    double s = 0.0;
+    for (int i = 0; i < (int)threadIdx.x; ++i) s += tmag(Ts[i + threadIdx.x * P], abs1);
+    cn[threadIdx.x] = s;
+  }
+}
+
+// y = Z x over the support lo .. hi of x, row lane of the product in lane.
+template <class E, class VEC> GS_DEV zd trevc_back_small(const TrevcMat<E>& t, const VEC& x, int lo, int hi) {
+  const E* z = t.Z + min((int)(threadIdx.x & 63), t.n - 1);
+  zd y = zr(0.0);
+#pragma unroll 8
+  for (int k = lo; k <= hi; ++k) {
+    const E a = z[(int64_t)k * t.ldz];
+    const zd b = x.get(k);
+    y = y + a * b;
+  }
+  return y;
 }
 
 // entries per lane of the class an order belongs to

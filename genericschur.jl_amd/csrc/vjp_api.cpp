@@ -41,21 +41,26 @@ extern "C" int gs_eig_vjp_batched_d(gs_handle* h, int64_t count, const int32_t* 
   DevBuf& meta = handle_buf(h, 4);
   TrevcPlan plan;
   trevc_groups(n, order.data(), count, false, plan);
-  const size_t mbytes = sizeof(int64_t) * 4 * count + sizeof(int32_t) * 2 * count;
+  const int64_t nws = (int64_t)plan.wsn.size();
+  const size_t mbytes = sizeof(int64_t) * (2 * count + 2 * nws) + sizeof(int32_t) * 2 * count;
   if ((e = meta.ensure(mbytes + 64)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
   char* mp = static_cast<char*>(meta.p);
   int64_t* d_off = reinterpret_cast<int64_t*>(mp);
   int64_t* d_woff = d_off + count;
-  int32_t* d_n = reinterpret_cast<int32_t*>(d_off + 4 * count);
+  int32_t* d_n = reinterpret_cast<int32_t*>(d_off + 2 * count + 2 * nws);
   int32_t* d_order = d_n + count;
   std::vector<char> hm(mbytes);
-  const size_t c8 = sizeof(int64_t) * count, c4 = sizeof(int32_t) * count;
-  std::memcpy(hm.data(), off, c8);
-  std::memcpy(hm.data() + c8, woff.data(), c8);
-  std::memcpy(hm.data() + 2 * c8, plan.wsn.data(), c8);
-  std::memcpy(hm.data() + 3 * c8, plan.wsnn.data(), c8);
-  std::memcpy(hm.data() + 4 * c8, n, c4);
-  std::memcpy(hm.data() + 4 * c8 + c4, order.data(), c4);
+  char* hp = hm.data();
+  auto put = [&](const void* src, size_t bytes) {
+    if (bytes > 0) std::memcpy(hp, src, bytes);
+    hp += bytes;
+  };
+  put(off, sizeof(int64_t) * count);
+  put(woff.data(), sizeof(int64_t) * count);
+  put(plan.wsn.data(), sizeof(int64_t) * nws);
+  put(plan.wsnn.data(), sizeof(int64_t) * nws);
+  put(n, sizeof(int32_t) * count);
+  put(order.data(), sizeof(int32_t) * count);
   if ((e = hipMemcpyAsync(meta.p, hm.data(), mbytes, hipMemcpyHostToDevice, s)) != hipSuccess)
     return handle_fail_hip(h, e, "hipMemcpyAsync");
   DevBuf& bVR = handle_buf(h, 5);
@@ -96,10 +101,10 @@ extern "C" int gs_eig_vjp_batched_d(gs_handle* h, int64_t count, const int32_t* 
   t.normalize = 1;
   t.ldt = t.ldz = t.ldv = 0;
   t.wsn = d_off + 2 * count;
-  t.wsnn = d_off + 3 * count;
+  t.wsnn = d_off + 2 * count + nws;
   // right and left eigenvectors, the second side reusing the workspace
   DevBuf& ws = handle_buf(h, 13);
-  if ((e = ws.ensure(plan.bytes)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
+  if (plan.bytes > 0 && (e = ws.ensure(plan.bytes)) != hipSuccess) return handle_fail_hip(h, e, "hipMalloc");
   for (int left = 0; left < 2; ++left) {
     t.left = left;
     t.V = static_cast<double*>(left ? bVL.p : bVR.p);

@@ -528,6 +528,56 @@ template <int R> __global__ void __launch_bounds__(64) ztrevc_finish_kernel(Trev
   }
 }
 
+// Orders up to kTrevcSmallN: the columns of a matrix by the wavefronts of one
+// workgroup, T in LDS (pitch NM + 1), the back-transform and the scaling in the
+// solving wavefront's registers.
+template <int NM, bool LEFT> __global__ void __launch_bounds__(1024) ztrevc_small_kernel(TrevcArgs a) {
+  extern __shared__ double smem[];  // ZFac[64] per wavefront
+  constexpr int P = NM + 1;
+  __shared__ zd Ts[P * NM];
+  __shared__ double cn[NM];
+  const TrevcMat<zd> t = trevc_mat<zd, false>(a, blockIdx.x);
+  const int n = t.n, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  trevc_stage<P>(t, LEFT, Ts, cn);
+  __syncthreads();
+  const ColG<zd> Tc{Ts, P};
+  ZFac* const fac = reinterpret_cast<ZFac*>(smem) + 64 * wave;
+  for (int b = wave; b < n; b += blockDim.x >> 6) {
+    const int kk = LEFT ? b : n - 1 - b;
+    const zd lam = Tc(kk, kk);
+    const double smin = fmax(GS_EPS * zabs1(lam), GS_FMIN * (double)n);  // vectors.jl:61,386
+    WaveVec<1> x;
+    x.v[0] = zr(0.0);
+    if (!LEFT) {
+      if (lane < kk) x.v[0] = -Tc(lane, kk);
+    } else {
+      if (lane > kk && lane < n) x.v[0] = -zconj(Tc(kk, lane));
+    }
+    double vscale;
+    if (!LEFT) vscale = (kk > 0) ? usolve_w<1>(Tc, cn, kk, lam, smin, x, fac) : 1.0;
+    else vscale = (kk < n - 1) ? cusolve_w<1>(Tc, cn, kk + 1, n - 1 - kk, lam, smin, x, fac) : 1.0;
+    x.set(kk, zr(vscale));
+    if (!(LEFT ? (lane >= kk && lane < n) : (lane <= kk))) x.v[0] = zr(0.0);
+    if (t.Z) x.v[0] = trevc_back_small(t, x, LEFT ? kk : 0, LEFT ? n - 1 : kk);
+    normalize_col<1>(x, n, a.normalize != 0);
+    if (lane < n) t.V[lane + (int64_t)kk * t.ldv] = x.v[0];
+  }
+}
+
+static hipError_t launch_ztrevc_small(const TrevcArgs& a, int nmax, hipStream_t s) {
+  const int nw = trevc_small_waves(a.count);
+  const size_t lds = 64 * sizeof(ZFac) * nw;
+  if (nmax <= 16) {
+    if (a.left) hipLaunchKernelGGL((ztrevc_small_kernel<16, true>), dim3(a.count), dim3(64 * nw), lds, s, a);
+    else hipLaunchKernelGGL((ztrevc_small_kernel<16, false>), dim3(a.count), dim3(64 * nw), lds, s, a);
+  } else {
+    if (a.left) hipLaunchKernelGGL((ztrevc_small_kernel<32, true>), dim3(a.count), dim3(64 * nw), lds, s, a);
+    else hipLaunchKernelGGL((ztrevc_small_kernel<32, false>), dim3(a.count), dim3(64 * nw), lds, s, a);
+  }
+  return hipGetLastError();
+}
+
 template <int R> static hipError_t launch_ztrevc_r(const TrevcArgs& a, int nmax, hipStream_t s) {
   const size_t lds = wavevec_lds_bytes<R>();
   const int nt = (nmax + 63) / 64;
@@ -545,6 +595,7 @@ template <int R> static hipError_t launch_ztrevc_r(const TrevcArgs& a, int nmax,
 }
 
 hipError_t launch_ztrevc(const TrevcArgs& a, int nmax, hipStream_t s) {
+  if (nmax <= kTrevcSmallN) return launch_ztrevc_small(a, nmax, s);
   switch (trevc_class(nmax)) {
     case 1: return launch_ztrevc_r<1>(a, nmax, s);
     case 2: return launch_ztrevc_r<2>(a, nmax, s);

@@ -220,13 +220,14 @@ def test_batched_vectors_with_large_order(gs, oracle):
                 assert np.abs(Vg - Vo).max() <= 1e-7, (cplx, left, m)
 
 
-@pytest.mark.parametrize("n,cplx", [(50, False), (50, True), (1100, False), (1100, True)])
+@pytest.mark.parametrize("n,cplx", [(24, False), (24, True), (50, False), (50, True), (1100, False), (1100, True)])
 def test_vectors_unnormalized(gs, oracle, n, cplx):
     """normalize = 0: the solutions back-transformed and scaled to largest
     entry 1 (max abs, or abs1 for the real pairs and the complex kernel),
     before _enormalize! — the form eigen! feeds to the balancing
-    back-transform (pirates.jl:86-110).  Small orders on the one-workgroup
-    kernels, 1100 on the whole-GPU path; entrywise against the oracle."""
+    back-transform (pirates.jl:86-110).  Order 24 in the one launch of the small
+    orders, 50 with the vectors in registers, 1100 with them in LDS; entrywise
+    against the oracle."""
     A, T, Z, w = _schur_lapack(n, cplx, 500 + n)
     for left in (False, True):
         Vg = gs.geigvecs(S(T, Z, w), left=left, normalize=False)
@@ -237,13 +238,14 @@ def test_vectors_unnormalized(gs, oracle, n, cplx):
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("left", [False, True])
 def test_class_edges_batched(gs, cplx, left):
-    """Orders at the edges of the launch classes (entries per lane), the back
-    transform's tiles and the 64-row factor chunks, in one batch with an empty
-    matrix: the batch gives the single calls' bits, and every vector satisfies
-    its eigenvalue equation (residual at most 50 n eps ||A||_F, unit vectors)."""
+    """Orders at the edges of the launch classes (one launch for small orders;
+    entries per lane), the back transform's tiles and the 64-row factor
+    chunks, in one batch with an empty matrix: the batch gives the single
+    calls' bits, and every vector satisfies its eigenvalue equation (residual
+    at most 50 n eps ||A||_F, unit vectors)."""
     import ctypes
     from genericschur import _lib
-    orders = (1, 2, 3, 15, 63, 64, 65, 0, 127, 128, 129, 130, 200, 256, 257, 300)
+    orders = (1, 2, 3, 15, 16, 17, 31, 32, 33, 63, 64, 65, 0, 127, 128, 129, 130, 200, 256, 257, 300)
     mats = []
     for n in orders:
         rng = gen.stream(41, 100, n)
@@ -268,3 +270,20 @@ def test_class_edges_batched(gs, cplx, left):
         res = np.linalg.norm(M @ X - X * w, axis=0)
         assert res.max() <= 50 * n * eps * np.linalg.norm(A)
         assert np.abs(np.linalg.norm(X, axis=0) - 1).max() <= 50 * eps
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("left", [False, True])
+def test_small_orders_without_Z(gs, cplx, left):
+    """Vectors of T itself (no Z) around the small orders' limits: the
+    eigenvalue equation, and zeros outside T's triangle (a pair's column reaches
+    one row further)."""
+    eps = np.finfo(np.float64).eps
+    for n in (1, 2, 3, 16, 17, 32, 33):
+        rng = gen.stream(42, 100, n)
+        F = gs.gschur(gen.ginibre_complex(n, rng) if cplx else gen.ginibre_real(n, rng))
+        X = gs.geigvecs(S(F.T, np.zeros((0, 0), dtype=F.T.dtype), F.values), left=left)
+        print(f"case vectors of T n={n} cplx={cplx} left={left}", flush=True)
+        M, w = (F.T.conj().T, F.values.conj()) if left else (F.T, F.values)
+        assert np.linalg.norm(M @ X - X * w, axis=0).max() <= 50 * n * eps * np.linalg.norm(F.T)
+        assert np.all((np.triu(X, 2) if left else np.tril(X, -2)) == 0)
