@@ -511,6 +511,15 @@ static bool bin_zlog(bool cplx, const Bin& b, int kflags) {
   return b.nmax >= 2;
 }
 
+// Matrices of a complex plan above the LDS-resident QR kernels' orders (no bin
+// holds orders on both sides).
+static int64_t windowed_count(const std::vector<Bin>& bins) {
+  int64_t c = 0;
+  for (const Bin& b : bins)
+    if (b.nmax > zqr_res_max_n()) c += b.count;
+  return c;
+}
+
 // Whether a complex plan's QR iterations run as one work-queue launch: not
 // where every order fits the LDS-resident kernels (one QR launch per bin;
 // 16384 matrices n = 4..24 3.8 against 6.9 ms, n = 33..48 34.3 against 39.7),
@@ -677,6 +686,7 @@ static hipError_t launch_plan(gs_handle* h, const PlanDev& pd, const double* A, 
     if ((e = launch_hq(bi)) != hipSuccess) return e;
     if ((e = hipEventRecord(h->evlead[bi], bstream(bins[bi]))) != hipSuccess) return e;
   }
+  const bool coop = windowed_count(bins) <= kCoopCount;
   bool waited[kBranches] = {false, false, false, false};
   for (size_t bi = 0; bi < bins.size(); ++bi) {
     const Bin& b = bins[bi];
@@ -697,7 +707,7 @@ static hipError_t launch_plan(gs_handle* h, const PlanDev& pd, const double* A, 
     if (flags & GS_QR_BAND)
       e = p->is_complex ? launch_zqr(a, b.nmax, b.nt_qr, s) : launch_dqr(a, b.nmax, b.nt_qr, s);
     else
-      e = p->is_complex ? launch_zqrw(a, b.nmax, s) : launch_dqrw(a, b.nmax, s);
+      e = p->is_complex ? launch_zqrw(a, b.nmax, coop, s) : launch_dqrw(a, b.nmax, s);
     if (e != hipSuccess) return e;
     if (timed && (e = hipEventRecord(h->tev[6 * bi + 3], s)) != hipSuccess) return e;
     if (timed && (e = hipEventRecord(h->tev[6 * bi + 4], s)) != hipSuccess) return e;
@@ -1143,7 +1153,7 @@ static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda
       if (kflags & GS_QR_BAND)
         le = cplx ? launch_zqr(a, (int)n, ntqr, h->stream) : launch_dqr(a, (int)n, ntqr, h->stream);
       else
-        le = cplx ? launch_zqrw(a, (int)n, h->stream) : launch_dqrw(a, (int)n, h->stream);
+        le = cplx ? launch_zqrw(a, (int)n, true, h->stream) : launch_dqrw(a, (int)n, h->stream);
       if (le == hipSuccess && zlg) le = cplx ? launch_zlog(a, (int)n, h->stream) : launch_dlog(a, (int)n, h->stream);
     }
   } else if (use_win) {

@@ -75,11 +75,13 @@ hipError_t launch_zqr(const BatchArgs& a, int nmax, int nt, hipStream_t s);
 // QR launch of matrices of order at most nmax: up to z/dqr_res_max_n() one
 // wavefront per matrix with H in LDS, above windowed with H and Z in HBM (a
 // launch's matrices all on one side of that order)
-// complex launches up to this size take the 512-thread windowed form
+// complex launches, coop: in the 512-thread windowed form, for calls of at most
+// kCoopCount matrices above that order (one to a CU), over all their launches,
+// which run side by side
 constexpr int kCoopCount = 256;
 int zqr_res_max_n();
 int dqr_res_max_n();
-hipError_t launch_zqrw(const BatchArgs& a, int nmax, hipStream_t s);
+hipError_t launch_zqrw(const BatchArgs& a, int nmax, bool coop, hipStream_t s);
 // The persistent form of launch_zqrw: `slots` workgroups take the matrices
 // order[first .. first + count) from the work queue a.qctr, in order.
 hipError_t launch_zqrw_queue(const BatchArgs& a, int slots, hipStream_t s);

@@ -1931,17 +1931,18 @@ template <bool FAST> static void launch_zqrr(const BatchArgs& a, int nmax, hipSt
   else hipLaunchKernelGGL((zqrr_kernel<FAST, 49>), dim3(a.count), dim3(64), 0, s, a);
 }
 
-// Launches of at most one matrix per CU take the 512-thread form (one matrix,
+// Calls of at most one matrix per CU take the 512-thread form (one matrix,
 // whole call with Z: n = 96 11.96 against 12.91 ms, n = 64 5.92 / 5.94; 256
-// matrices n = 73..96 13.84 / 13.97; 400 18.9 against 14.4).
-hipError_t launch_zqrw(const BatchArgs& a, int nmax, hipStream_t s) {
+// matrices n = 73..96 13.84 / 13.97; 400 18.9 against 14.4; 500 n = 49..96 in
+// three launches of at most 256 side by side 17.0 / 14.4).
+hipError_t launch_zqrw(const BatchArgs& a, int nmax, bool coop, hipStream_t s) {
   if (a.count <= 0) return hipSuccess;
   if (nmax <= zqr_res_max_n()) {
     if (a.flags & 0x1000) launch_zqrr<false>(a, nmax, s);
     else launch_zqrr<true>(a, nmax, s);
     return hipGetLastError();
   }
-  if (a.count <= kCoopCount && !(a.flags & 0x1000))
+  if (coop && !(a.flags & 0x1000))
     hipLaunchKernelGGL((zqrw2_kernel<true, 512>), dim3(a.count), dim3(512), 0, s, a);
   else if (a.flags & 0x1000)
     hipLaunchKernelGGL((zqrw2_kernel<false>), dim3(a.count), dim3(128), 0, s, a);

@@ -52,3 +52,37 @@ def test_small_vectors_one_launch(gs, kernels, cplx, left):
         S = gs.gschur(A)
         k = kernels(lambda: gs.geigvecs(S, left=left))
         assert len(k) >= 3 if n > 32 else (len(k) == 1 and "trevc_small" in k[0]), k
+
+
+def _device_batch(ns, cplx):
+    import numpy as np
+    import torch
+    ns = np.ascontiguousarray(ns, dtype=np.int32)
+    off = np.zeros(len(ns), dtype=np.int64)
+    off[1:] = np.cumsum(ns[:-1].astype(np.int64) ** 2)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    A = torch.randn((2 if cplx else 1) * int((ns.astype(np.int64) ** 2).sum()), generator=g, device="cuda",
+                    dtype=torch.float64)
+    T, Z = torch.zeros_like(A), torch.zeros_like(A)
+    W = torch.zeros(2 * int(ns.sum()), device="cuda", dtype=torch.float64)
+    return ns, off, A, T, Z, W, torch.zeros(len(ns), device="cuda", dtype=torch.int32)
+
+
+@pytest.mark.parametrize("count", [85, 86])
+def test_noalloc_cooperative_form_by_call(gs, kernels, count):
+    """The 512-thread windowed form where the call (not one of its launches,
+    which run side by side) has at most a matrix above order 48 per CU."""
+    import ctypes
+    from genericschur import _lib
+    ns, off, A, T, Z, W, info = _device_batch([20] * 300 + [96] * count + [80] * count + [64] * (256 - 2 * 85), True)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    h = _lib.handle()
+
+    def call():
+        rc = _lib.lib().gs_schur_batched_z_noalloc(h, len(ns), ctypes.c_void_p(ns.ctypes.data),
+                                                   ctypes.c_void_p(off.ctypes.data), p(A), p(T), p(Z), p(W), p(info),
+                                                   _lib.GS_SCALE)
+        _lib.check(rc, h, "gs_schur_batched_z_noalloc")
+    k = kernels(call)
+    assert any("zqrw2_kernel<true, 512>" in x for x in k) == (count == 85), k
+    assert any("zqrw2_kernel<true, 128>" in x for x in k) == (count == 86), k
