@@ -1024,18 +1024,20 @@ static hipError_t run_large(gs_handle* h, int64_t n, double* dA, int64_t lda, do
 
 // Threads of the windowed QR kernel for one matrix above the LDS-resident
 // orders.  Measured, whole call without / with Z, 512 against 1024 threads:
-// n = 130 20.7 / 23.0 against 22.4 / 24.6 ms, n = 400 216 / 248 against 263 /
-// 279, n = 1000 1862 / 2109 against 1864 / 2116, n = 1500 (more chains than
+// n = 130 20.7 / 23.0 against 22.4 / 24.6 ms, n = 400 171 / 198 against 222 /
+// 238, n = 1000 1862 / 2109 against 1864 / 2116, n = 1500 (more chains than
 // seven wavefronts finish behind the chase) 6371 / 7109 against 5798 / 6576.
-// GSCHUR_WIN_NT overrides (512 or 1024).
-static int win_nt(int n) {
+// With Z updated in place (zdir), which adds Z's rows to the chains, that point
+// comes earlier: n = 500 349 against 364, n = 600 634 / 615, n = 700 879 / 850, n =
+// 767 1169 / 1083.  GSCHUR_WIN_NT overrides (512 or 1024).
+static int win_nt(int n, bool zdir) {
   static const int force = [] {
     const char* e = std::getenv("GSCHUR_WIN_NT");
     const int v = e ? std::atoi(e) : 0;
     return (v == 512 || v == 1024) ? v : 0;
   }();
   if (force) return force;
-  return n <= 1000 ? 512 : 1024;
+  return n <= (zdir ? 550 : 1000) ? 512 : 1024;
 }
 
 static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda, double* T, int64_t ldt, double* Z,
@@ -1212,7 +1214,7 @@ static int run_single(gs_handle* h, bool cplx, int64_t n, double* A, int64_t lda
       a.loff = zlg ? reinterpret_cast<const int64_t*>(mp + offsetof(Meta, loff)) : nullptr;
       a.llen = zlg ? reinterpret_cast<int64_t*>(mp + offsetof(Meta, llen)) : nullptr;
       a.zlog_min = 0;
-      le = launch_zqrw_single(a, win_nt((int)n), h->stream);
+      le = launch_zqrw_single(a, win_nt((int)n, (kflags & GS_WANTZ) && !zlg), h->stream);
       if (le == hipSuccess && zlg)
         le = launch_zlog_rows((int)n, dZ, n, static_cast<const double*>(h->bLog.p),
                               reinterpret_cast<const int64_t*>(mp + offsetof(Meta, llen)), h->stream);

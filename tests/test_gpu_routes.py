@@ -86,3 +86,13 @@ def test_noalloc_cooperative_form_by_call(gs, kernels, count):
     k = kernels(call)
     assert any("zqrw2_kernel<true, 512>" in x for x in k) == (count == 85), k
     assert any("zqrw2_kernel<true, 128>" in x for x in k) == (count == 86), k
+
+
+@pytest.mark.parametrize("n,wantZ,zdirect,nt", [(550, True, False, 512), (551, True, False, 1024), (551, False, False, 512),
+                                                (768, True, False, 512), (768, True, True, 1024)])
+def test_single_complex_threads(gs, kernels, n, wantZ, zdirect, nt):
+    """Threads of one complex matrix's QR kernel: 1024 already above order 550
+    where Z is updated in place (without the log, which starts at 768)."""
+    A = gen.ginibre_complex(n, gen.stream(53, 1, n))
+    k = kernels(lambda: gs.gschur(A, wantZ=wantZ, zdirect=zdirect))
+    assert any(f"zqrw2_kernel<true, {nt}>" in x for x in k), k
