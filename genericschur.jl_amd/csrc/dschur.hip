@@ -1120,8 +1120,9 @@ hipError_t launch_dshift(const double* H, int64_t ld, LState* st, hipStream_t s)
 // After a bin's QR launch: each matrix's Z log applied to Z, one wavefront per
 // 64 rows and one row per lane with its NC entries in registers (zlog_kernel's
 // form, dlog_row's operations; a sweep's last, two-element step is logged with
-// v3 = 0 and runs as a three-element one).  1208 matrices n = 97..128 take 4.5
-// ms and 1094 n = 65..96 1.2 ms, against 8.7 ms together with Z in LDS.
+// v3 = 0 and runs as a three-element one).  Against Z in LDS (below): 2000
+// matrices n = 33..64 0.33 + 0.24 (two bins) against 0.40 ms, 1094 n = 65..96
+// 1.22 against 1.16 ms, 500 n = 81..96 0.585 against 0.595.
 template <int NC> __global__ void __launch_bounds__(64) dlog_kernel(BatchArgs a) {
   constexpr int NT = (2 + 3 * NC + 63) / 64;  // a record has at most 2 + 3 (n - 1) doubles
   constexpr int NE = (4 * NC + 63) / 64;      // lane registers of a sweep's steps
@@ -1210,14 +1211,122 @@ template <int NC> __global__ void __launch_bounds__(64) dlog_kernel(BatchArgs a)
   }
 }
 
+// The same for orders 97 .. 128, whose rows do not fit the registers without
+// spills: one workgroup of two wavefronts per matrix with all of Z in LDS (row r,
+// column c at zs[(c - 1) n + r]), each thread replaying the log on one row.  Each
+// wavefront stages a record in its own LDS buffer and loads the next one into
+// registers while it replays the current one.  1208 matrices n = 97..128 3.4 ms,
+// dlog_kernel<128> 4.4 ms.
+constexpr int DLREC = 384;  // >= 2 + 3 (n - 1) for n <= 128
+__global__ void __launch_bounds__(128) dlog_lds_kernel(BatchArgs a) {
+  extern __shared__ double dzs[];
+  __shared__ double rbuf[2][DLREC];  // a separate array: its reads do not wait on the row writes
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int b = blockIdx.x;
+  if (b >= a.count) return;
+  const int m = a.order[a.first + b];
+  const int n = a.n[m];
+  if (n <= 0 || wave * 64 >= n) return;
+  const int64_t len = a.llen[m];
+  if (len <= 0) return;
+  double* Z = a.Z + a.off[m];
+  const double* lg = a.zlog + a.loff[m];
+  const int r = min(tid, n - 1);  // threads past the last row repeat it, unstored
+  const bool live = tid < n;
+  double t[DLREC / 64];
+  auto fetch = [&](int64_t p) {
+#pragma unroll
+    for (int j = 0; j < DLREC / 64; ++j) t[j] = lg[min(p + lane + 64 * j, len - 1)];
+  };
+  fetch(0);
+  for (int c0 = 0; c0 < n; c0 += 8) {
+    double v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = Z[r + (int64_t)min(c0 + i, n - 1) * n];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (c0 + i < n && live) dzs[(c0 + i) * n + r] = v[i];
+  }
+  double* row = dzs + r;
+  const int st = n;
+  double* rec = rbuf[wave];
+  for (int64_t pos = 0; pos < len;) {
+#pragma unroll
+    for (int j = 0; j < DLREC / 64; ++j) rec[lane + 64 * j] = t[j];
+    wsync();
+    const double h0 = rec[0];
+    const bool rotation = h0 < 0.0;
+    const int i1 = __builtin_amdgcn_readfirstlane(rotation ? (int)(-h0) : (int)h0);
+    const int ie = __builtin_amdgcn_readfirstlane(rotation ? 0 : (int)rec[1]);
+    const int64_t rl = rotation ? 3 : 2 + 3 * (int64_t)(ie - i1);
+    if (pos + rl < len) fetch(pos + rl);
+    if (live) {
+      if (rotation) {
+        double a1 = row[(i1 - 1) * st], a2 = row[i1 * st];
+        drot_fixed(a1, a2, rec[1], rec[2]);
+        row[(i1 - 1) * st] = a1;
+        row[i1 * st] = a2;
+      } else {
+        const double* e = rec + 2;
+        double c0 = row[(i1 - 1) * st], c1 = row[i1 * st];
+        // groups of eight steps: the group's row entries (which its own steps
+        // do not write first) are read before any of its writes
+        int k = i1;
+        for (; k + 7 < ie - 1; k += 8) {
+          double bb[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) bb[j] = row[(k + j + 1) * st];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            drefl3_fixed(c0, c1, bb[j], e[3 * (k + j - i1)], e[3 * (k + j - i1) + 1], e[3 * (k + j - i1) + 2]);
+            row[(k + j - 1) * st] = c0;
+            c0 = c1;
+            c1 = bb[j];
+          }
+        }
+        for (; k < ie - 1; ++k) {
+          double bb = row[(k + 1) * st];
+          drefl3_fixed(c0, c1, bb, e[3 * (k - i1)], e[3 * (k - i1) + 1], e[3 * (k - i1) + 2]);
+          row[(k - 1) * st] = c0;
+          c0 = c1;
+          c1 = bb;
+        }
+        drefl2_fixed(c0, c1, e[3 * (ie - 1 - i1)], e[3 * (ie - 1 - i1) + 1]);
+        row[(ie - 2) * st] = c0;
+        row[(ie - 1) * st] = c1;
+      }
+    }
+    wsync();  // the record buffer is rewritten for the next record
+    pos += rl;
+  }
+  if (live) {
+    for (int c0 = 0; c0 < n; c0 += 8) {
+      double v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = dzs[min(c0 + i, n - 1) * n + r];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (c0 + i < n) Z[r + (int64_t)(c0 + i) * n] = v[i];
+    }
+  }
+}
+
 hipError_t launch_dlog(const BatchArgs& a, int nmax, hipStream_t s) {
   if (a.count <= 0 || !a.zlog) return hipSuccess;
   const dim3 g(a.count, (nmax + 63) / 64);
-  if (nmax <= 32) hipLaunchKernelGGL(dlog_kernel<32>, g, dim3(64), 0, s, a);
-  else if (nmax <= 64) hipLaunchKernelGGL(dlog_kernel<64>, g, dim3(64), 0, s, a);
-  else if (nmax <= 96) hipLaunchKernelGGL(dlog_kernel<96>, g, dim3(64), 0, s, a);
-  else if (nmax <= 128) hipLaunchKernelGGL(dlog_kernel<128>, g, dim3(64), 0, s, a);
-  else return hipErrorInvalidValue;
+  if (nmax <= 32) {
+    hipLaunchKernelGGL(dlog_kernel<32>, g, dim3(64), 0, s, a);
+  } else if (nmax <= 64) {
+    hipLaunchKernelGGL(dlog_kernel<64>, g, dim3(64), 0, s, a);
+  } else if (nmax <= 96) {
+    hipLaunchKernelGGL(dlog_kernel<96>, g, dim3(64), 0, s, a);
+  } else if (nmax <= 128) {
+    const size_t lds = (size_t)nmax * nmax * sizeof(double);
+    (void)hipFuncSetAttribute((const void*)dlog_lds_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(dlog_lds_kernel, dim3(a.count), dim3(128), lds, s, a);
+  } else {
+    return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 

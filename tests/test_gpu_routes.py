@@ -96,3 +96,10 @@ def test_single_complex_threads(gs, kernels, n, wantZ, zdirect, nt):
     A = gen.ginibre_complex(n, gen.stream(53, 1, n))
     k = kernels(lambda: gs.gschur(A, wantZ=wantZ, zdirect=zdirect))
     assert any(f"zqrw2_kernel<true, {nt}>" in x for x in k), k
+
+
+@pytest.mark.parametrize("n,name", [(96, "dlog_kernel<96>"), (97, "dlog_lds_kernel"), (128, "dlog_lds_kernel")])
+def test_real_replay_form(gs, kernels, n, name):
+    """The real Z log's replay: Z's rows in registers up to order 96, Z in LDS above."""
+    A = [gen.ginibre_real(n, gen.stream(54, 1, n))] * 2
+    assert any(name in x for x in kernels(lambda: gs.gschur_batched(A)))
