@@ -35,7 +35,7 @@ struct Bin {
   int nt_hq;  // threads per workgroup of the Hessenberg+Z launch
   int nt_qr;  // threads per workgroup of the QR launch
   int branch; // graph branch (stream) the bin runs on
-  int zlog;   // tuned Z log of the QR launch: 1 on, 0 off, -1 the default rule
+  bool zlog;  // the QR launch logs its Z updates (where the call logs)
   double work;
 };
 
@@ -372,6 +372,44 @@ static std::string plan_key(bool cplx, int64_t count, const int32_t* n, const in
   return k;
 }
 
+// Matrices of a complex plan above the LDS-resident QR kernels' orders (no bin
+// holds orders on both sides).
+static int64_t windowed_count(const std::vector<Bin>& bins) {
+  int64_t c = 0;
+  for (const Bin& b : bins)
+    if (b.nmax > zqr_res_max_n()) c += b.count;
+  return c;
+}
+
+// Whether a plan has matrices above the resident orders, and so few that they
+// take the 512-thread form, all of them in one QR launch: at most one to a CU,
+// which it fills, so that beside smaller matrices some CUs have to stay free
+// (1000 n = 4..64, 242 of them above 48, 7.4 ms, queued 7.0).
+static bool coop_plan(bool cplx, const std::vector<Bin>& bins) {
+  const int64_t w = cplx ? windowed_count(bins) : 0;
+  return w > 0 && w <= (bins.back().nmax > zqr_res_max_n() ? kCoopCount : kCoopCount / 4 * 3);
+}
+
+// Whether a complex plan's QR iterations run as one work-queue launch: where
+// there are more matrices above the LDS-resident orders than the 512-thread form
+// takes, in one launch beside the resident bins' (200 matrices n = 49..96 12.1
+// against 13.7 ms queued, 250 n = 2..99 13.0 / 15.9, 300 n = 24..60 5.4 / 5.9,
+// 16384 n = 4..24 and one n = 49 4.3 / 7.0).  A queue holds the small orders too:
+// they fill its tail (2500 matrices n = 24..60 8.5 ms; those up to 48 in resident
+// launches beside the queue 11.2, the 8192 of n = 8..96 50.4 against 53.6).
+static bool plan_queue(const Tuning& t, bool cplx, const std::vector<Bin>& bins) {
+  return cplx && qr_queue(t, cplx) && windowed_count(bins) > 0 && !coop_plan(cplx, bins);
+}
+
+// The largest real order whose QR launch logs its Z updates; complex bins log
+// at every order.  Measured with each launch alone, QR + replay against in
+// place: complex n = 4..24 (1000 matrices) 0.83 against 0.90 ms, and with
+// every larger order of 8192 matrices n ~ U{8..96} in place up to 72 the batch
+// takes 56.3 ms, with the log 50.4 ms; real n = 4..24 0.72 against 0.79 ms,
+// n = 16..32 1.14 against 1.23 ms, n = 129..141 (1000 matrices, whose rows have
+// no replay kernel) 30.2 ms in place.
+constexpr int kDlogMaxN = 128;
+
 // Host part of a plan: size bins of width bin_width, the largest bin first
 // and the largest matrix first inside a bin (order[]), each bin's launch
 // shape and graph branch, and the eigenvalue offsets woff[].  Orders must
@@ -407,8 +445,6 @@ static void plan_bins(const Tuning& tn, bool cplx, int64_t count, const int32_t*
     bin.nmax = std::max(1, n[v.front()]);
     bin.nmin = n[v.back()];
     bin.nt_hq = bin_nt_hq(tn, cplx, bin.nmax);
-    const Tuning::Row* r = tune_row(tn, bin.nmax);
-    bin.zlog = r ? r->zlog : -1;
     bin.nt_qr = default_nt_qr(cplx, bin.nmax);
     bin.work = 0;
     for (int32_t i : v) bin.work += (double)n[i] * n[i] * n[i];
@@ -416,17 +452,40 @@ static void plan_bins(const Tuning& tn, bool cplx, int64_t count, const int32_t*
     bins.push_back(bin);
     order.insert(order.end(), v.begin(), v.end());
   }
-  // bins to graph branches, heaviest first onto the least loaded branch
-  std::vector<int> idx(bins.size());
-  for (size_t i = 0; i < idx.size(); ++i) idx[i] = (int)i;
-  std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) { return bins[x].work > bins[y].work; });
+  for (Bin& b : bins) {
+    const Tuning::Row* r = tune_row(tn, b.nmax);
+    b.zlog = r && r->zlog >= 0 ? r->zlog == 1 : b.nmax >= 2;
+  }
+  // Bins to graph branches, the longest first onto the least loaded branch.  A
+  // complex bin lasts at least as long as its largest matrix, about n^2 sweep
+  // steps one after another (n = 96 12 ms; the GPU does the n^3 of about 56000
+  // such steps in their time).  Where the bins above the resident orders share
+  // a QR launch (coop_plan), that is branch 0, and the resident bins follow one
+  // another on branch 1 while they are shorter: the runtime maps the branches to
+  // fewer queues, and two long chains in one queue wait for each other (250 n =
+  // 2..99 as four branches 19.8 ms, as two 13.0).
+  std::vector<double> cost(bins.size());
+  for (size_t i = 0; i < bins.size(); ++i) {
+    const Bin& b = bins[i];
+    cost[i] = cplx ? std::max((double)b.nmax * b.nmax, b.work / 56000.0) : b.work;
+  }
   double load[kBranches] = {0, 0, 0, 0};
+  size_t nwin = 0;
+  if (coop_plan(cplx, bins))
+    for (; nwin < bins.size() && bins[nwin].nmax > zqr_res_max_n(); ++nwin) {
+      bins[nwin].branch = nwin & 1;  // its Hessenberg launch
+      load[0] = std::max(load[0], cost[nwin]);
+    }
+  std::vector<int> idx;
+  for (size_t i = nwin; i < bins.size(); ++i) idx.push_back((int)i);
+  std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) { return cost[x] > cost[y]; });
   for (int i : idx) {
-    int best = 0;
-    for (int b = 1; b < kBranches; ++b)
-      if (load[b] < load[best]) best = b;
+    int best = nwin ? 1 : 0;
+    if (!nwin || load[1] + cost[i] > load[0])
+      for (int b = best + 1; b < kBranches; ++b)
+        if (load[b] < load[best]) best = b;
     bins[i].branch = best;
-    load[best] += bins[i].work;
+    load[best] += cost[i];
   }
 }
 
@@ -490,15 +549,6 @@ static int build_plan(gs_handle* h, bool cplx, int64_t count, const int32_t* n, 
   return GS_OK;
 }
 
-// The largest real order whose QR launch logs its Z updates; complex bins log
-// at every order.  Measured with each launch alone, QR + replay against in
-// place: complex n = 4..24 (1000 matrices) 0.83 against 0.90 ms, and with
-// every larger order of 8192 matrices n ~ U{8..96} in place up to 72 the batch
-// takes 56.3 ms, with the log 50.4 ms; real n = 4..24 0.72 against 0.79 ms,
-// n = 16..32 1.14 against 1.23 ms, n = 129..141 (1000 matrices, the replay's
-// row no longer fits the registers) 30.6 against 30.2 ms.
-constexpr int kDlogMaxN = 128;
-
 // Whether the batched QR launches of this call log their Z updates
 // (windowed kernels, Z wanted, not GS_ZDIRECT).
 static bool uses_zlog(int kflags) { return (kflags & GS_WANTZ) && !(kflags & (GS_QR_BAND | GS_ZDIRECT)); }
@@ -506,33 +556,7 @@ static bool uses_zlog(int kflags) { return (kflags & GS_WANTZ) && !(kflags & (GS
 static bool bin_zlog(bool cplx, const Bin& b, int kflags) {
   if (!uses_zlog(kflags)) return false;
   if (!cplx && b.nmax > kDlogMaxN) return false;
-  if (kflags & GS_ZLOG_TINY) return true;
-  if (b.zlog >= 0) return b.zlog == 1;
-  return b.nmax >= 2;
-}
-
-// Matrices of a complex plan above the LDS-resident QR kernels' orders (no bin
-// holds orders on both sides).
-static int64_t windowed_count(const std::vector<Bin>& bins) {
-  int64_t c = 0;
-  for (const Bin& b : bins)
-    if (b.nmax > zqr_res_max_n()) c += b.count;
-  return c;
-}
-
-// Whether a complex plan's QR iterations run as one work-queue launch: not
-// where every order fits the LDS-resident kernels (one QR launch per bin;
-// 16384 matrices n = 4..24 3.8 against 6.9 ms, n = 33..48 34.3 against 39.7),
-// nor where the matrices are too few for the queue's small workgroups to fill
-// the CUs (200 matrices n = 49..96 12.7 per bin against 14.1 ms).  A larger plan
-// with larger orders queues the small ones too: they fill the queue's tail
-// (2500 matrices n = 24..60 8.5 ms; those up to 48 in resident launches beside
-// the queue 11.2, the 8192 of n = 8..96 50.4 against 53.6).
-static bool plan_queue(const Tuning& t, bool cplx, const std::vector<Bin>& bins) {
-  if (!qr_queue(t, cplx) || bins.empty() || bins[0].nmax <= zqr_res_max_n()) return false;
-  int64_t count = 0;
-  for (const Bin& b : bins) count += b.count;
-  return count > kCoopCount;
+  return (kflags & GS_ZLOG_TINY) || b.zlog;
 }
 
 // Work-queue form of a complex batch (tuning queue = 1): the bins'
@@ -665,10 +689,19 @@ static hipError_t launch_plan(gs_handle* h, const PlanDev& pd, const double* A, 
   for (const Bin& b : bins) used[b.branch] = true;
   for (int i = 0; i < kBranches; ++i)
     if (used[i] && (e = hipStreamWaitEvent(h->branch[i], h->evfork, 0)) != hipSuccess) return e;
+  // the bins above the resident orders of a coop_plan share a QR launch (not
+  // where they differ in logging; timed, every bin has its own)
+  const bool coop = coop_plan(p->is_complex, bins);
+  size_t nwin = 0;
+  if (coop && !timed && !(flags & GS_QR_BAND)) {
+    while (nwin < bins.size() && bins[nwin].nmax > zqr_res_max_n()) ++nwin;
+    for (size_t bi = 1; bi < nwin; ++bi)
+      if (bin_zlog(true, bins[bi], flags) != bin_zlog(true, bins[0], flags)) nwin = 0;
+  }
   // the leading (largest) bins' Hessenberg launches run first, alone: the
   // largest bin's chain (Hessenberg, QR, Z log) is the batch's longest, and
   // started later it would finish last with the GPU half idle
-  const int lead = (int)std::min<size_t>((size_t)hq_lead(tn, p->is_complex), bins.size());
+  const int lead = nwin ? 0 : (int)std::min<size_t>((size_t)hq_lead(tn, p->is_complex), bins.size());
   auto bstream = [&](const Bin& b) { return timed ? h->stream : h->branch[b.branch]; };
   auto launch_hq = [&](size_t bi) -> hipError_t {
     const Bin& b = bins[bi];
@@ -686,9 +719,27 @@ static hipError_t launch_plan(gs_handle* h, const PlanDev& pd, const double* A, 
     if ((e = launch_hq(bi)) != hipSuccess) return e;
     if ((e = hipEventRecord(h->evlead[bi], bstream(bins[bi]))) != hipSuccess) return e;
   }
-  const bool coop = windowed_count(bins) <= kCoopCount;
+  for (size_t bi = 0; bi < nwin; ++bi)
+    if ((e = launch_hq(bi)) != hipSuccess) return e;
+  if (nwin > 0) {
+    hipStream_t s = h->branch[0];
+    if (nwin > 1) {
+      if ((e = hipEventRecord(h->evlead[0], h->branch[1])) != hipSuccess) return e;
+      if ((e = hipStreamWaitEvent(s, h->evlead[0], 0)) != hipSuccess) return e;
+    }
+    const bool log = zl && bin_zlog(true, bins[0], flags);
+    a.first = bins[0].first;
+    a.count = (int)windowed_count(bins);
+    a.zlog = log ? zlog : nullptr;
+    if ((e = launch_zqrw(a, bins[0].nmax, true, s)) != hipSuccess) return e;
+    for (size_t bi = 0; log && bi < nwin; ++bi) {
+      a.first = bins[bi].first;
+      a.count = bins[bi].count;
+      if ((e = launch_zlog(a, bins[bi].nmax, s)) != hipSuccess) return e;
+    }
+  }
   bool waited[kBranches] = {false, false, false, false};
-  for (size_t bi = 0; bi < bins.size(); ++bi) {
+  for (size_t bi = nwin; bi < bins.size(); ++bi) {
     const Bin& b = bins[bi];
     hipStream_t s = bstream(b);
     if ((int)bi >= lead) {

@@ -76,8 +76,7 @@ hipError_t launch_zqr(const BatchArgs& a, int nmax, int nt, hipStream_t s);
 // wavefront per matrix with H in LDS, above windowed with H and Z in HBM (a
 // launch's matrices all on one side of that order)
 // complex launches, coop: in the 512-thread windowed form, for calls of at most
-// kCoopCount matrices above that order (one to a CU), over all their launches,
-// which run side by side
+// kCoopCount matrices above that order (one to a CU), over all their launches
 constexpr int kCoopCount = 256;
 int zqr_res_max_n();
 int dqr_res_max_n();

@@ -70,11 +70,12 @@ def _device_batch(ns, cplx):
 
 @pytest.mark.parametrize("count", [85, 86])
 def test_noalloc_cooperative_form_by_call(gs, kernels, count):
-    """The 512-thread windowed form where the call (not one of its launches,
-    which run side by side) has at most a matrix above order 48 per CU."""
+    """The 512-thread windowed form where the call (not one of its launches)
+    has at most a matrix above order 48 to a CU (three to four CUs beside
+    smaller ones)."""
     import ctypes
     from genericschur import _lib
-    ns, off, A, T, Z, W, info = _device_batch([20] * 300 + [96] * count + [80] * count + [64] * (256 - 2 * 85), True)
+    ns, off, A, T, Z, W, info = _device_batch([20] * 300 + [96] * count + [80] * count + [64] * (192 - 2 * 85), True)
     p = lambda t: ctypes.c_void_p(t.data_ptr())
     h = _lib.handle()
 
@@ -103,3 +104,44 @@ def test_real_replay_form(gs, kernels, n, name):
     """The real Z log's replay: Z's rows in registers up to order 96, Z in LDS above."""
     A = [gen.ginibre_real(n, gen.stream(54, 1, n))] * 2
     assert any(name in x for x in kernels(lambda: gs.gschur_batched(A)))
+
+
+# (orders, whether the work queue, the 512-thread form and the resident form run)
+ROUTES = [([64] * 256, False, True, False),
+          ([64] * 257, True, False, False),
+          ([64] * 192 + [20] * 10, False, True, True),
+          ([64] * 193 + [20] * 10, True, False, False),
+          ([49] + [20] * 1000, False, True, True),
+          ([48] * 300, False, False, True)]
+
+
+@pytest.mark.parametrize("case", range(len(ROUTES)))
+def test_complex_batch_routes(gs, kernels, case):
+    """Complex batches at the lines between the forms."""
+    orders, queue, coop, resident = ROUTES[case]
+    ns, off, A, T, Z, W, info = _device_batch(orders, True)
+    k = kernels(lambda: gs.gschur_batched_device(ns, off, A, T, Z, W, info, True))
+    assert int(info.abs().sum()) == 0
+    got = [any(x in y for y in k) for x in ("zqrw2_queue_kernel", "zqrw2_kernel<true, 512>", "zqrr_kernel")]
+    assert got == [queue, coop, resident], k
+
+
+def test_complex_batch_one_windowed_launch(gs, kernels):
+    """Bins above the resident orders in one 512-thread launch, with the results
+    of one launch per bin (as when timed) and of the queue (the same matrices
+    among more), bit for bit."""
+    import torch
+    from genericschur import _lib
+    orders = [99, 97, 80, 60, 49, 48, 30, 5, 1] * 20
+    ns, off, A, T, Z, W, info = _device_batch(orders, True)
+    gs.gschur_batched_device(ns, off, A, T, Z, W, info, True)
+    T1, Z1, W1 = torch.zeros_like(T), torch.zeros_like(Z), torch.zeros_like(W)
+    gs.gschur_batched_device(ns, off, A, T1, Z1, W1, info, True, timing=True)
+    qr = [r for r in _lib.last_launches() if r["kind"] == "qr"]
+    assert sum(r["nmax"] > 48 for r in qr) >= 2 and sum(r["count"] for r in qr) == len(orders)
+    assert torch.equal(T, T1) and torch.equal(Z, Z1) and torch.equal(W, W1)
+    ns2, off2, A2, T2, Z2, W2, info2 = _device_batch(orders + [60] * 300, True)
+    A2[:A.numel()] = A
+    assert any("queue" in x for x in kernels(lambda: gs.gschur_batched_device(ns2, off2, A2, T2, Z2, W2, info2, True)))
+    m = A.numel()
+    assert torch.equal(T, T2[:m]) and torch.equal(Z, Z2[:m]) and torch.equal(W, W2[:W.numel()])
