@@ -401,14 +401,30 @@ static bool plan_queue(const Tuning& t, bool cplx, const std::vector<Bin>& bins)
   return cplx && qr_queue(t, cplx) && windowed_count(bins) > 0 && !coop_plan(cplx, bins);
 }
 
-// The largest real order whose QR launch logs its Z updates; complex bins log
-// at every order.  Measured with each launch alone, QR + replay against in
-// place: complex n = 4..24 (1000 matrices) 0.83 against 0.90 ms, and with
-// every larger order of 8192 matrices n ~ U{8..96} in place up to 72 the batch
-// takes 56.3 ms, with the log 50.4 ms; real n = 4..24 0.72 against 0.79 ms,
-// n = 16..32 1.14 against 1.23 ms, n = 129..141 (1000 matrices, whose rows have
-// no replay kernel) 30.2 ms in place.
+// The largest real order whose QR launch logs its Z updates (n = 129..141, 1000
+// matrices, whose rows have no replay kernel: 30.2 ms in place).
 constexpr int kDlogMaxN = 128;
+// Complex: queued plans of at most kQueueLogCount matrices above the resident
+// orders log from kQueueLogMinN up only, since the smaller orders' replays are a
+// chain of launches behind a queue that does not fill the GPU (400 matrices n =
+// 49..96 14.7 ms with every order logged, 13.8 without; 1000 n = 8..96, 530 of
+// them above 48, 16.0 / 15.3; 600 n = 49..96 15.4 / 15.7; 1000 17.0 / 17.6).
+constexpr int kQueueLogCount = 560;
+constexpr int kQueueLogMinN = 81;
+
+// Whether a bin's QR launch logs its Z updates by default.  Real: up to
+// kDlogMaxN (n = 4..24 0.72 against 0.79 ms in place, n = 16..32 1.14 / 1.23).
+// Complex: resident launches always (1000 matrices n = 4..24 0.83 against 0.90
+// ms); the 512-thread form never, whose chains wait for the chase in any case
+// (200 n = 49..96 12.1 in place, 13.7 logged); queued ones as above, all of them
+// from kQueueLogCount on (8192 n = 8..96 50.4 against 56.3 ms with the log from
+// 73 up).
+static bool default_zlog(bool cplx, const Bin& b, bool queue, bool coop, int64_t windowed) {
+  if (b.nmax < 2) return false;
+  if (!cplx) return b.nmax <= kDlogMaxN;
+  if (queue) return windowed > kQueueLogCount || b.nmax >= kQueueLogMinN;
+  return b.nmax <= zqr_res_max_n() || !coop;
+}
 
 // Host part of a plan: size bins of width bin_width, the largest bin first
 // and the largest matrix first inside a bin (order[]), each bin's launch
@@ -452,9 +468,11 @@ static void plan_bins(const Tuning& tn, bool cplx, int64_t count, const int32_t*
     bins.push_back(bin);
     order.insert(order.end(), v.begin(), v.end());
   }
+  const int64_t windowed = cplx ? windowed_count(bins) : 0;
+  const bool queue = plan_queue(tn, cplx, bins), coop = coop_plan(cplx, bins);
   for (Bin& b : bins) {
     const Tuning::Row* r = tune_row(tn, b.nmax);
-    b.zlog = r && r->zlog >= 0 ? r->zlog == 1 : b.nmax >= 2;
+    b.zlog = r && r->zlog >= 0 ? r->zlog == 1 : default_zlog(cplx, b, queue, coop, windowed);
   }
   // Bins to graph branches, the longest first onto the least loaded branch.  A
   // complex bin lasts at least as long as its largest matrix, about n^2 sweep
@@ -471,7 +489,7 @@ static void plan_bins(const Tuning& tn, bool cplx, int64_t count, const int32_t*
   }
   double load[kBranches] = {0, 0, 0, 0};
   size_t nwin = 0;
-  if (coop_plan(cplx, bins))
+  if (coop)
     for (; nwin < bins.size() && bins[nwin].nmax > zqr_res_max_n(); ++nwin) {
       bins[nwin].branch = nwin & 1;  // its Hessenberg launch
       load[0] = std::max(load[0], cost[nwin]);

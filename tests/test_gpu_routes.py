@@ -106,24 +106,29 @@ def test_real_replay_form(gs, kernels, n, name):
     assert any(name in x for x in kernels(lambda: gs.gschur_batched(A)))
 
 
-# (orders, whether the work queue, the 512-thread form and the resident form run)
-ROUTES = [([64] * 256, False, True, False),
-          ([64] * 257, True, False, False),
-          ([64] * 192 + [20] * 10, False, True, True),
-          ([64] * 193 + [20] * 10, True, False, False),
-          ([49] + [20] * 1000, False, True, True),
-          ([48] * 300, False, False, True)]
+# (orders, whether the work queue, the 512-thread form, the resident form, and a replay of orders above 48 run)
+ROUTES = [([64] * 256, False, True, False, False),
+          ([64] * 257, True, False, False, False),
+          ([64] * 192 + [20] * 10, False, True, True, False),
+          ([64] * 193 + [20] * 10, True, False, False, False),
+          ([81] * 257, True, False, False, True),
+          ([64] * 560, True, False, False, False),
+          ([64] * 561, True, False, False, True),
+          ([49] + [20] * 1000, False, True, True, False),
+          ([48] * 300, False, False, True, False)]
 
 
 @pytest.mark.parametrize("case", range(len(ROUTES)))
 def test_complex_batch_routes(gs, kernels, case):
     """Complex batches at the lines between the forms."""
-    orders, queue, coop, resident = ROUTES[case]
+    orders, queue, coop, resident, replay = ROUTES[case]
     ns, off, A, T, Z, W, info = _device_batch(orders, True)
     k = kernels(lambda: gs.gschur_batched_device(ns, off, A, T, Z, W, info, True))
     assert int(info.abs().sum()) == 0
     got = [any(x in y for y in k) for x in ("zqrw2_queue_kernel", "zqrw2_kernel<true, 512>", "zqrr_kernel")]
     assert got == [queue, coop, resident], k
+    assert any("zlog_kernel<" + c in y for y in k for c in ("64", "80", "96")) == replay, k
+    assert any("zlog_kernel<32" in y or "zlog_kernel<48" in y for y in k) == resident, k
 
 
 def test_complex_batch_one_windowed_launch(gs, kernels):

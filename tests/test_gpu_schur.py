@@ -105,16 +105,20 @@ def test_batched_matches_single(gs):
         assert np.array_equal(S.T, S1.T) and np.array_equal(S.Z, S1.Z) and np.array_equal(S.values, S1.values)
 
 
-def test_zlog_matches_direct(gs, oracle):
-    """The Z log: Z updated after the QR sweeps from the logged reflectors
-    and scalings (default), during the sweeps (GS_ZDIRECT), and with a log of
-    one sweep, so that the QR kernel applies it to Z in HBM before nearly
+@pytest.mark.parametrize("queued", [False, True])
+def test_zlog_matches_direct(gs, oracle, queued):
+    """The Z log, one launch per bin and through the work queue (more matrices
+    above order 48 than its line): Z updated after the QR sweeps from the
+    logged reflectors and scalings (default), during the sweeps (GS_ZDIRECT),
+    and with a log of one sweep, so that the QR kernel applies it to Z in HBM before nearly
     every sweep (GS_ZLOG_TINY).  T does not depend on how Z is updated, and
     the three forms apply the same operations to Z in the same order with
     the same rounding: all bitwise equal.  The log form also passes the
     Schur invariants."""
     eps = np.finfo(np.float64).eps
     mats = gen.workload2(seed=7, count=64)
+    if queued:
+        mats += gen.workload2(seed=8, count=600, nmin=49, nmax=64)
     mats += [gen.toeplitz_grcar(40).astype(np.complex128), np.eye(12, dtype=np.complex128)]
     Sl, il = gs.gschur_batched(mats)
     Sd, idd = gs.gschur_batched(mats, zdirect=True)
@@ -191,7 +195,8 @@ def test_log_replay_order_edges(gs, cplx, n):
     """The Z log's replay at the edges of its register classes, groups of
     eight steps and blocks of 64 rows: T, Z and the values bitwise those of
     the updates in place.  The matrices deflate in the middle (sweeps that
-    start late) and, real, leave 2 x 2 blocks to rotate."""
+    start late) and, real, leave 2 x 2 blocks to rotate.  Complex orders also
+    through the work queue, beside enough matrices that every order logs."""
     rng = gen.stream(33, 100, n)
     mats = [gen.ginibre_complex(n, rng) if cplx else gen.ginibre_real(n, rng) for _ in range(3)]
     B = mats[0].copy()
@@ -202,6 +207,13 @@ def test_log_replay_order_edges(gs, cplx, n):
     assert np.all(il == 0)
     for a, d in zip(Sl, Sd):
         assert np.array_equal(a.T, d.T) and np.array_equal(a.Z, d.Z) and np.array_equal(a.values, d.values)
+    if cplx:
+        rest = [gen.ginibre_complex(49, rng)] * 561
+        for kw in ({}, {"zlog_tiny": True}):
+            Sq, iq = gs.gschur_batched(mats + rest, **kw)
+            assert np.all(iq == 0)
+            for q, d in zip(Sq, Sd):
+                assert np.array_equal(q.T, d.T) and np.array_equal(q.Z, d.Z) and np.array_equal(q.values, d.values)
 
 
 @pytest.mark.parametrize("cplx,n", [(True, n) for n in (2, 3, 15, 16, 17, 24, 25, 31, 32, 33, 47, 48, 49)] +
