@@ -474,6 +474,7 @@ template <int R, class VEC> GS_DEV void enormalize_w(VEC& v, int n) {
       bi = oi;
     }
   }
+  bi = min(bi, n - 1);  // no entry compared (NaN throughout): any of them, within the vector
   const zd vi0 = v.get(bi);
   const zd tt = ((1.0 / nrm) * zconj(vi0)) / sqrt(zabs2(vi0));
 #pragma unroll

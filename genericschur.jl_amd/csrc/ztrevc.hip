@@ -447,6 +447,7 @@ template <int R, class VEC> GS_DEV void normalize_col(VEC& v, int n, bool enorm)
       bi = oi;
     }
   }
+  bi = min(bi, n - 1);  // no entry compared (NaN throughout): any of them, within the vector
   const zd vi0 = v.get(bi);
   const double s = 1.0 / nrm;
   const zd tt = (s * zconj(vi0)) / sqrt(zabs2(vi0));

@@ -287,3 +287,23 @@ def test_small_orders_without_Z(gs, cplx, left):
         M, w = (F.T.conj().T, F.values.conj()) if left else (F.T, F.values)
         assert np.linalg.norm(M @ X - X * w, axis=0).max() <= 50 * n * eps * np.linalg.norm(F.T)
         assert np.all((np.triu(X, 2) if left else np.tril(X, -2)) == 0)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("n", [20, 60, 300])
+def test_vectors_nan(gs, cplx, n):
+    """A NaN in T spoils the vectors that depend on it and no others, in the one
+    launch, in registers and in LDS (where no entry of a vector is the largest,
+    the normalization takes one within it)."""
+    rng = np.random.default_rng(91)
+    T = np.triu(rng.standard_normal((n, n))) + np.diag(3.0 * np.arange(n))
+    if cplx:
+        T = T + 1j * np.triu(rng.standard_normal((n, n)), 1)
+    T[5, 10] = np.nan
+    Z = np.linalg.qr(rng.standard_normal((n, n)))[0].astype(T.dtype)
+    for left in (False, True):
+        print(f"case NaN n={n} cplx={cplx} left={left}", flush=True)
+        V = gs.geigvecs(S(T, Z, np.diag(T)), left=left)
+        bad = np.isnan(V).any(axis=0)
+        assert np.array_equal(np.nonzero(bad)[0], np.arange(6) if left else np.arange(10, n))
+        assert np.all(np.isnan(V[:, bad])) and np.abs(np.linalg.norm(V[:, ~bad], axis=0) - 1).max() <= 1e-13
