@@ -108,6 +108,18 @@ def test_families_batched(gs, oracle, cplx):
     report(f"batched {'complex' if cplx else 'real'}", tally)
 
 
+def test_families_multishift(gs, oracle):
+    """Real orders with multishift sweeps (from 256), whose diagonal order is
+    their own: the invariants, the acceptance bounds and the eigenvalues."""
+    for name, A, normal in families(300, False, seed=5):
+        print(f"case {name} n=300", flush=True)
+        S = gs.gschur(A)
+        checks.schur_invariants(A, S.T, S.Z, S.values, TOL, normal=normal)
+        assert checks.rel_backward(A, S.T, S.Z) <= 50 * 300 * EPS and checks.rel_orth(S.Z) <= 50 * 300 * EPS
+        To, Zo, wo, cond, _ = oracle_result(oracle, A)
+        checks.eigen_parity(A, S.values, wo, cond)
+
+
 @pytest.mark.parametrize("cplx,n", [(True, 40), (True, 130), (False, 40), (False, 160)])
 def test_families_plain(gs, oracle, cplx, n):
     """The plain unblocked global-memory kernel (GS_PLAIN)."""
