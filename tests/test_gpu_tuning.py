@@ -52,9 +52,11 @@ def test_table_parity_and_single_match(gs, oracle, tuned, cplx):
 
 def test_queue_matches_bins(gs, tuned):
     """One work-queue QR launch over all bins runs the same per-matrix code as
-    the per-bin launches: identical bits (with the Z log on some bins)."""
+    the per-bin launches: identical bits (with the Z log on some bins).  The
+    queue needs more than 192 matrices above order 48 beside smaller ones."""
     h = tuned
-    mats = gen.workload2(seed=4, count=300)
+    mats = gen.workload2(seed=4, count=600)
+    assert sum(A.shape[0] > 48 for A in mats) > 192
     print("case queue vs bins", flush=True)
     tuning.set_section(h, True, dict(TABLE["complex"], queue=0))
     S0, i0 = gs.gschur_batched(mats)

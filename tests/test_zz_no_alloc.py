@@ -2,9 +2,10 @@
 against gs_schur_batched_z on the same device data: T, Z, the values and
 info bit for bit equal (both run the same kernels; the no-allocation form
 updates Z in place, which the Z-log tests show equal to the Z log bit for
-bit), on two calls in a row, the second with a smaller batch of other
-orders, so that the scratch array's leftovers from the first call must not
-matter.  Also: more matrices than the scratch array holds are rejected."""
+bit), on calls in a row, the second with a smaller batch of other orders, so
+that the scratch array's leftovers from the first call must not matter, the
+third with enough matrices that the allocating form takes the work queue.
+Also: more matrices than the scratch array holds are rejected."""
 import ctypes
 
 import numpy as np
@@ -41,7 +42,7 @@ def _call(fn_name, ns, off, A, T, Z, W, info, flags):
 def test_noalloc_matches_batched(gs):
     from genericschur import _lib
     import torch
-    for step, (seed, count, nmin, nmax) in enumerate(((21, 300, 8, 96), (22, 97, 3, 40))):
+    for step, (seed, count, nmin, nmax) in enumerate(((21, 300, 8, 96), (22, 97, 3, 40), (23, 600, 8, 96))):
         mats = gen.workload2(seed=seed, count=count, nmin=nmin, nmax=nmax)
         ns, off, flat = gs.pack(mats, np.complex128)
         print(f"case noalloc call {step}: {count} matrices, n in [{ns.min()}, {ns.max()}]", flush=True)
