@@ -502,13 +502,15 @@ template <int NT> __global__ void __launch_bounds__(NT) lctrl_kernel(LQArgs a) {
       s.phase = 0;
       continue;
     }
-    // a multishift sweep (its shifts come from dshift_kernel); it counts as MNB
-    // iterations, and an iteration that stalls takes the exceptional shifts
+    // a multishift sweep (its shifts come from dshift_kernel), one iteration
+    // against maxiter: its eight double shifts and the double-shift sweeps of the
+    // small blocks are more than the shifts taken one at a time (order 300: 55 x 8
+    // + 354 against 536), and a limit that those meet has to be met; an iteration
+    // that stalls takes the exceptional shifts
     s.iterqr += 1;
     s.nb = 0;
     if (a.msmin > 0 && iend - istart + 1 >= a.msmin && s.iterqr != 10 && s.iterqr != 20) {
       s.nb = MNB;
-      s.iter += MNB - 1;
       s.nsweep += MNB;
       s.nstep += MNB * (int64_t)(iend - istart);
       s.mx = istart;
@@ -1013,7 +1015,7 @@ hipError_t large_schur_d(const LargeArgs& a, LargeWork& w, hipStream_t s, LargeT
     seen_iend = last.iend;
     if (status != 0) break;
     if (last.nb > 0) {
-      if ((e = launch_dshift(H, ldt, q.st, s)) != hipSuccess) return fail(e);
+      if ((e = launch_dshift(H, ldt, q.st, q.maxiter, s)) != hipSuccess) return fail(e);
       const int nch = ms_chunks(last.istart, last.iend);
       for (int c = 0; c <= nch; ++c) {
         hipLaunchKernelGGL(lms_kernel, dim3(1 + std::min(3 * nwork, 255)), dim3(64 * MNB), MS_LDS, s, q, c);

@@ -1063,10 +1063,10 @@ hipError_t launch_dqrw(const BatchArgs& a, int nmax, hipStream_t s) {
 // Shifts of a multishift sweep: the eigenvalues of the trailing 2 MNB x 2 MNB
 // block of the active block, by the resident QR, complex ones in their conjugate
 // pairs, the real ones two by two.  Where the QR does not converge, those that
-// it found, and the block's diagonal in the others' places; a block that is not
-// finite, which would run to its limit in every sweep, is not tried (order 256
-// with one NaN, 100 sweeps: 626 -> 55 ms).  One wavefront.
-__global__ void __launch_bounds__(64) dshift_kernel(const double* H, int64_t ld, LState* st) {
+// it found, and the block's diagonal in the others' places.  A block with a NaN
+// never deflates: it ends the iteration as the limit would (order 256 with one
+// NaN, a limit of 800: 626 ms while every sweep ran the QR on it).  One wavefront.
+__global__ void __launch_bounds__(64) dshift_kernel(const double* H, int64_t ld, LState* st, int64_t maxiter) {
   constexpr int M = 2 * MNB, RP = M + 1;
   __shared__ double hs[RP * M];
   __shared__ double lg[3 * RP + 2];
@@ -1074,19 +1074,22 @@ __global__ void __launch_bounds__(64) dshift_kernel(const double* H, int64_t ld,
   __shared__ int redi[2];
   if (st->status != 0 || st->nb == 0) return;
   const int i0 = st->iend - M;  // 0-based
-  bool finite = true;
+  bool nan = false;
   for (int e = threadIdx.x; e < M * M; e += 64) {
     const int c = e / M, r = e - c * M;
     const double h = r <= c + 1 ? H[(i0 + r) + (int64_t)(i0 + c) * ld] : 0.0;
-    finite = finite && isfinite(h);
+    nan = nan || isnan(h);
     hs[r + c * RP] = h;
   }
   if (threadIdx.x < M) w[threadIdx.x] = zr(H[(i0 + threadIdx.x) + (int64_t)(i0 + threadIdx.x) * ld]);
   __syncthreads();
   const FullLayout lay{RP};
   int64_t nsweep = 0, nstep = 0;
-  if (!wave_any(!finite))
+  if (wave_any(nan)) {
+    if (threadIdx.x == 0) st->iter = maxiter;
+  } else {
     d_qr<64, FullLayout, true, RP>(hs, lay, M, nullptr, 0, false, lg, redi, w, 30 * M, nsweep, nstep, nullptr);
+  }
   __syncthreads();
   if (threadIdx.x != 0) return;
   int nc = 0, nr = 0;  // bulges with complex shifts, from the front; real ones, from the back
@@ -1112,8 +1115,8 @@ __global__ void __launch_bounds__(64) dshift_kernel(const double* H, int64_t ld,
   }
 }
 
-hipError_t launch_dshift(const double* H, int64_t ld, LState* st, hipStream_t s) {
-  hipLaunchKernelGGL(dshift_kernel, dim3(1), dim3(64), 0, s, H, ld, st);
+hipError_t launch_dshift(const double* H, int64_t ld, LState* st, int64_t maxiter, hipStream_t s) {
+  hipLaunchKernelGGL(dshift_kernel, dim3(1), dim3(64), 0, s, H, ld, st, maxiter);
   return hipGetLastError();
 }
 

@@ -19,10 +19,12 @@ namespace gs {
 
 // Smallest order with multishift sweeps.  They deflate the eigenvalues in an
 // order of their own, so T's diagonal is another one of the matrix's valid
-// ones than the double-shift iteration's; the orders near the LDS-resident
-// range, where they gain least, keep that iteration's.  Measured, whole call
-// with Z: n = 160 25.9 against 31.1 ms, n = 200 33.5 / 45.8, n = 256 44.5 / 64.4,
-// n = 501 105 / 188, n = 1500 528 / 1317.
+// ones than the double-shift iteration's.  They are faster from the LDS-resident
+// range on, so the line is not the measurements': it keeps the double-shift
+// iteration's order, which is the oracle's slot by slot and is held by the
+// tests up to n = 160, for the orders below 256.  Measured, QR phase with Z,
+// multishift against double-shift sweeps: n = 160 16.2 / 22.4 ms, n = 200 21.5 /
+// 30.9, n = 256 29.1 / 48.4, n = 501 71.5 / 155, n = 1500 405 / 1191.
 constexpr int MSMINN = 256;
 // Smallest active block with multishift sweeps.  Measured, QR phase: n = 300
 // 36.0 ms from 64 rows, 35.7 from 48, 36.2 from 80; n = 200 21.4, 23.9, 23.8.
@@ -303,6 +305,6 @@ GS_DEV void ms_chase(double* win, double* lg, const double* sh, int t0, int t1, 
   }
 }
 
-hipError_t launch_dshift(const double* H, int64_t ld, LState* st, hipStream_t s);
+hipError_t launch_dshift(const double* H, int64_t ld, LState* st, int64_t maxiter, hipStream_t s);
 
 }  // namespace gs

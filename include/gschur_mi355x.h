@@ -126,9 +126,9 @@ int gs_schur_z(gs_handle* h, int64_t n, double* A, int64_t lda, double* T, int64
  * sweep chased in LDS-resident chunks whose reflectors are applied to the
  * rest of H and to Z by the whole GPU: below order 256 the same double-shift
  * iteration (same per-element update order as the unblocked sweep), from 256
- * up multishift sweeps of eight double shifts, each counted as eight
- * iterations, with T's diagonal in an order of their own.  GS_PLAIN runs the unblocked
- * single-workgroup kernel instead. */
+ * up multishift sweeps of eight double shifts, each counted as one
+ * iteration, with T's diagonal in an order of their own.  GS_PLAIN runs the
+ * unblocked single-workgroup kernel instead. */
 int gs_schur_d(gs_handle* h, int64_t n, double* A, int64_t lda, double* T, int64_t ldt, double* Z, int64_t ldz,
                double* W, int flags, int64_t maxiter, int64_t maxinner, int32_t* info);
 

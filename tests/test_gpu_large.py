@@ -221,9 +221,9 @@ def test_multishift_orders(gs, n):
 
 
 def test_multishift_nan_fails_as_fast(gs):
-    """A NaN never deflates: the iteration ends at its limit, and a sweep over
-    NaN takes no longer than one over numbers (the shifts' own QR iteration,
-    which cannot converge on it, is not tried)."""
+    """A NaN never deflates: the iteration ends as at its limit, and in no more
+    time than a matrix of numbers takes to reach it (the shifts' own QR
+    iteration, which cannot converge on a NaN, is not tried)."""
     import time
     n = 256
     A = gen.ginibre_real(n, gen.stream(27, 100, n))
@@ -235,8 +235,27 @@ def test_multishift_nan_fails_as_fast(gs):
         for _ in range(4):
             t0 = time.perf_counter()
             with pytest.raises(gs.UnconvergedException):
-                gs.gschur(M, maxiter=160)
+                gs.gschur(M, maxiter=40)
             t.append(time.perf_counter() - t0)
         times.append(min(t))
-    print(f"20 sweeps: {1e3 * times[0]:.1f} ms, with a NaN {1e3 * times[1]:.1f} ms", flush=True)
+    print(f"to the limit {1e3 * times[0]:.1f} ms, with a NaN {1e3 * times[1]:.1f} ms", flush=True)
     assert times[1] <= 2.5 * times[0]
+    with pytest.raises(gs.UnconvergedException):
+        gs.gschur(B)
+
+
+@pytest.mark.parametrize("n", [256, 300, 501])
+def test_multishift_iteration_limit(gs, n):
+    """An iteration limit that double-shift sweeps (the plain kernel: each sweep
+    and each deflation is one) just meet is met by multishift sweeps too."""
+    from genericschur import _lib
+    for A in (gen.ginibre_real(n, gen.stream(28, 100, n)), gen.haar_orthogonal(n, gen.stream(28, 101, n)),
+              gen.toeplitz_grcar(n)):
+        P = gs.gschur(A, plain=True)
+        blocks = n - int(np.count_nonzero(np.diag(P.T, -1)))
+        limit = int(_lib.last_stats()[0]) + blocks
+        print(f"case iteration limit n={n}: {limit}", flush=True)
+        gs.gschur(A, plain=True, maxiter=limit)
+        with pytest.raises(gs.UnconvergedException):
+            gs.gschur(A, plain=True, maxiter=limit - 1)
+        gs.gschur(A, maxiter=limit)
