@@ -40,9 +40,11 @@ namespace gs {
 // Hessenberg panel width.  A panel column is one workgroup's serial work that
 // grows with the columns before it in the panel, and bounds the phase; wider
 // panels only make the GEMM updates fewer and better filled.  Measured,
-// Hessenberg phase with 64 / 32 / 16 columns: n = 501 31.4 / 20.1 / 15.8 ms,
-// n = 1500 110.5 / 72.4 / 57.2, n = 4096 479 / 329 / 262 (Q formation 0.9 / 0.9
-// / 1.6, 2.7 / 3.1 / 5.3 and 10 / - / - ms; the n = 4096 solve 1.95 / 1.79 / 1.77 s).
+// Hessenberg phase with 64 / 32 / 16 columns: n = 501 31.3 / 20.1 / 15.8 ms,
+// n = 1500 110.8 / 72.5 / 57.1, n = 4096 485 / 324 / 260.  The price: Q formation
+// 0.9 / 0.9 / 1.6, 2.7 / 3.2 / 5.3 and 10.1 / 13.4 / 23.7 ms, and the products at
+// n = 4096 at 13.3 / 9.3 / 4.8 TFLOP/s (21 / 30 / 58 ms together); the n = 4096
+// solve 1.94 / 1.76 / 1.66 s.
 constexpr int LNB = 16;
 constexpr int LW = 64;   // bulge-chase window (rows and columns)
 constexpr int LKC = LW - 4;  // bulge steps per chunk

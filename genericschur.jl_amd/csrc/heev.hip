@@ -975,8 +975,8 @@ template <class T> static hipError_t launch_heev_big_t(const HeevArgs& a, bool c
                        wantz ? Zr : nullptr, (int64_t)n);
     int* infob = a.info ? a.info + b : nullptr;
     int* sweepsb = a.sweeps ? a.sweeps + b : nullptr;
-    // the recurrence by one thread writing its rotations to HBM, their replay
-    // onto Q's rows over the whole GPU (values only: the recurrence alone)
+    // the recurrence by one wavefront writing its rotations to HBM, their replay
+    // onto Q's rows over the whole GPU beside it (values only: the recurrence alone)
     if ((e = st_rounds<T>(n, a.maxsweeps, dref, eref, wantz ? Zr : nullptr, n, (int64_t)n, rec, cap, npos, state,
                           infob, sweepsb, s)) != hipSuccess)
       return e;

@@ -187,8 +187,11 @@ int gs_schur_batched_z_noalloc(gs_handle* h, int64_t count, const int32_t* n, co
  * _xsolve/_safe_lu_solve! util.jl:603-751).  Z may be NULL (vectors of T).
  * V is n x n complex (ldv).  normalize = 0 returns the max-abs1-scaled
  * vectors before _enormalize!.  Orders up to 4096 (GS_E_UNSUPPORTED above):
- * one wavefront per column of every matrix over the whole GPU, with
- * workspaces held by the handle. */
+ * up to 32 one workgroup per matrix; above, one wavefront per column of every
+ * matrix over the whole GPU, with a workspace held by the handle, 24 bytes
+ * (real) or 32 (complex) per entry of the matrices that one group of launches
+ * takes, at most 1 GiB or one matrix's (512 MiB at order 4096, complex).
+ * gs_eig_vjp_batched_d holds another one. */
 int gs_trevc_z(gs_handle* h, int64_t n, const double* T, int64_t ldt, const double* Z, int64_t ldz, double* V,
                int64_t ldv, int left, int normalize, int flags);
 int gs_trevc_d(gs_handle* h, int64_t n, const double* T, int64_t ldt, const double* Z, int64_t ldz, double* V,
