@@ -220,6 +220,20 @@ def test_multishift_orders(gs, n):
         gs.gschur(gen.ginibre_real(n, gen.stream(26, 101, n)), maxiter=20)
 
 
+def test_multishift_orthogonality(gs):
+    """Z of multishift sweeps is no further from orthogonal than that of the
+    double-shift sweeps they replace, though they take 7 % more reflectors:
+    |Z^T Z - I| in the Frobenius norm, mean of 4 Ginibre matrices of order 400,
+    1.66e-13 (standard deviation of one 0.04), double-shift 2.16e-13, the bound
+    midway.  With the logged tau as the chase has it, 2.25e-13."""
+    n, errs = 400, []
+    for s in range(4):
+        print(f"case n={n} seed {s}", flush=True)
+        Z = gs.gschur(np.random.default_rng(177 * n + s).standard_normal((n, n))).Z.astype(np.longdouble)
+        errs.append(float(np.sqrt(((Z.T.dot(Z) - np.eye(n)) ** 2).sum())))
+    assert np.mean(errs) <= 1.9e-13
+
+
 def test_multishift_nan_fails_as_fast(gs):
     """A NaN never deflates: the iteration ends as at its limit, and in no more
     time than a matrix of numbers takes to reach it (the shifts' own QR
