@@ -71,6 +71,19 @@ GS_DEV bool ms_chunk_of(int I, int E, int c, MChunk& ck) {
 GS_DEV int ms_wb(int I, int t0) { return max(I, I + t0 - MSP * (MNB - 1) - 1); }
 GS_DEV int ms_we(int I, int E, int t1) { return min(E, I + t1 + 3); }
 
+// tau fitted to the vector (1, v2, v3) as rounded: a Newton step towards
+// 2 / (1 + v2^2 + v3^2).  What the reflector formulas leave of it is most of
+// what Z loses.  n = 400, |Z^T Z - I| 1.63e-13 with the step, 2.25 without, 2.16
+// by double-shift sweeps (7 % fewer reflectors); |A Z - Z T| / |A| 0.98, 1.28 and
+// 1.23e-14.  Fitting the log's tau only, so that Z takes another reflector than
+// T, gives 1.66e-13 and 1.12e-14, and eigenvector residuals 10 % above the
+// double-shift ones instead of 15 % below.  Two more dependent operations of a
+// step; n = 1500 462 ms with it, 465 without.
+GS_DEV double ms_fit(double tau, double v2, double v3) {
+  const double vv = fma(v3, v3, fma(v2, v2, 1.0));
+  return fma(tau, fma(-0.5 * tau, vv, 1.0), tau);
+}
+
 // One 3-element reflector on a line.
 GS_DEV void ms_apply(double& x0, double& x1, double& x2, double tau, double v2, double v3) {
   const double ss = x0 + v2 * x1 + v3 * x2;
@@ -191,7 +204,7 @@ GS_DEV void ms_chase(double* win, double* lg, const double* sh, int t0, int t1, 
       double beta = nv0;
       v2 = nv1;
       v3 = nv2;
-      tau = dreflector3_wave(beta, v2, v3);
+      tau = ms_fit(dreflector3_wave(beta, v2, v3), v2, v3);
       tau2 = tau * v2;
       tau3 = tau * v3;
       const bool l0 = lane == 0;
@@ -225,6 +238,7 @@ GS_DEV void ms_chase(double* win, double* lg, const double* sh, int t0, int t1, 
         tau = dreflector_fast(2, beta, v2, v3);
         v3 = 0.0;
       }
+      tau = ms_fit(tau, v2, v3);
       tau2 = tau * v2;
       tau3 = tau * v3;
       for (int c = k + lane; c <= we; c += 64) {
@@ -299,13 +313,7 @@ GS_DEV void ms_chase(double* win, double* lg, const double* sh, int t0, int t1, 
   }
   if (lane <= t1 - t0) {
     double* const g = lg + 3 * (lane * MNB + j);
-    // tau of the logged vector, one Newton step towards 2 / (1 + v2^2 + v3^2):
-    // the chase's comes from other rounded values, and what it misses is Z's
-    // loss of orthogonality.  n = 400: |Z^T Z - I| 1.66e-13 with the step, 2.25
-    // without, 2.16 by double-shift sweeps (7 % fewer reflectors); |A - Z T Z^T|
-    // / |A| 1.23, 1.72 and 1.68e-14; no time measurable.
-    const double vv = fma(l3, l3, fma(l2, l2, 1.0));
-    g[0] = fma(lt, fma(-0.5 * lt, vv, 1.0), lt);
+    g[0] = lt;
     g[1] = l2;
     g[2] = l3;
   }
