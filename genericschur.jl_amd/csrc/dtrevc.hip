@@ -701,7 +701,8 @@ int trevc_max_n() { return 4096; }
 // (left), and 8 n + 8 n + 4 n for norms, subdiagonal and kinds; each array
 // 256-byte aligned.  A group ends where the next matrix needs another class,
 // would take the workspace above kGroupBytes, or fills the grid's z
-// dimension; the small orders, without workspace, are one group.
+// dimension; the small orders, without workspace, are one group, or, up to
+// kTrevcJoin of them, part of the group of orders 33 to 64 if there is one.
 constexpr size_t kGroupBytes = size_t(1) << 30;
 constexpr int kGroupCount = 32768;
 static size_t seg(size_t bytes) { return (bytes + 255) & ~size_t(255); }
@@ -712,6 +713,9 @@ void trevc_groups(const int32_t* n, const int32_t* order, int64_t count, bool cp
   p.wsn.clear();
   p.wsnn.clear();
   p.bytes = 0;
+  int64_t nsmall = 0;
+  for (int64_t q = 0; q < count; ++q) nsmall += n[q] > 0 && n[q] <= kTrevcSmallN;
+  const bool join = nsmall <= kTrevcJoin;
   for (int64_t q = 0; q < count;) {
     if (n[order[q]] <= 0) break;  // descending: only empty matrices remain
     TrevcGroup g;
@@ -724,7 +728,7 @@ void trevc_groups(const int32_t* n, const int32_t* order, int64_t count, bool cp
     while (small && k < count && n[order[k]] > 0) ++k;
     for (; !small && k < count && k - q < kGroupCount; ++k) {
       const int64_t m = n[order[k]];
-      if (m <= kTrevcSmallN || trevc_class((int)m) != cls) break;
+      if (m <= (join ? 0 : kTrevcSmallN) || trevc_class((int)m) != cls) break;
       if (k > q && (16 + es) * (size_t)(snn + m * m) > kGroupBytes) break;
       p.wsn.push_back(sn);
       p.wsnn.push_back(snn);

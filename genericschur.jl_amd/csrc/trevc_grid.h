@@ -11,8 +11,8 @@
 //   4. back-transform Z X as FP64 MFMA tiles (trevc_back_kernel);
 //   5. one wavefront per column scales and normalises in V.
 //
-// The orders up to kTrevcSmallN go through one launch of their own.  The rest of
-// the list is processed in classes of orders that need the same number R of
+// The orders up to kTrevcSmallN go through one launch of their own, unless they
+// are few beside orders 33 to 64 (kTrevcJoin).  The rest of the list is processed in classes of orders that need the same number R of
 // entries per lane.  Bound by the latency of the substitutions, of which one
 // matrix has n in flight and a batch n per matrix.  Before, one workgroup of
 // 4 wavefronts per matrix solved its n columns in turn with T's triangle in
@@ -207,6 +207,14 @@ template <class E> __global__ void __launch_bounds__(256, 2) trevc_back_kernel(T
 // 3.77 / 2.06).
 constexpr int kTrevcSmallN = 32;
 
+// Small matrices of a list that go through the grid launches of its orders 33
+// to 64 all the same, if it has any: up to this many cost those less than a
+// launch of their own.  Measured, own launch / joined, right vectors, beside 8
+// matrices: 16 complex of n = 17..32 93 / 61 us, 256 105 / 102, 512 130 / 141
+// (real 96 / 64, 111 / 84, 137 / 112; n = 2..16 75 / 62, 82 / 76, 94 / 95);
+// beside 300: 200 / 168, 210 / 202, 237 / 249.
+constexpr int64_t kTrevcJoin = 256;
+
 // Wavefronts of a small matrix's workgroup: one per column or two where the
 // matrices are fewer than the CUs, down to four where they fill the GPU.
 // Measured, 16 / 8 / 4: one complex matrix n = 32 55 / 62 / 89 us, 1000 of n =
@@ -229,16 +237,24 @@ template <int P, class E> GS_DEV void trevc_stage(const TrevcMat<E>& t, bool abs
   }
 }
 
-// y = Z x over the support lo .. hi of x, row lane of the product in lane.
+// y = Z x over the support lo .. hi of x, row lane of the product in lane, each
+// sum an fma chain of its own in the columns' order: the MFMA tiles' bits.
 template <class E, class VEC> GS_DEV zd trevc_back_small(const TrevcMat<E>& t, const VEC& x, int lo, int hi) {
+  constexpr bool CPLX = sizeof(E) == sizeof(zd);
   const E* z = t.Z + min((int)(threadIdx.x & 63), t.n - 1);
-  zd y = zr(0.0);
+  zd y = zr(0.0), y2 = zr(0.0);
 #pragma unroll 8
   for (int k = lo; k <= hi; ++k) {
     const E a = z[(int64_t)k * t.ldz];
     const zd b = x.get(k);
-    y = y + a * b;
+    if constexpr (CPLX) {
+      y = zmk(fma(a.x, b.x, y.x), fma(a.x, b.y, y.y));
+      y2 = zmk(fma(a.y, b.y, y2.x), fma(a.y, b.x, y2.y));
+    } else {
+      y = y + a * b;
+    }
   }
+  if constexpr (CPLX) y = zmk(y.x - y2.x, y.y + y2.y);
   return y;
 }
 

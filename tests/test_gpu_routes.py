@@ -54,6 +54,29 @@ def test_small_vectors_one_launch(gs, kernels, cplx, left):
         assert len(k) >= 3 if n > 32 else (len(k) == 1 and "trevc_small" in k[0]), k
 
 
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("small,large,own", [(256, [33, 64], False), (257, [33, 64], True), (256, [65], True)])
+def test_small_vectors_joined(gs, kernels, cplx, small, large, own):
+    """Up to 256 matrices of orders up to 32 go with the list's orders 33 to 64,
+    if there are any; either way with the single calls' bits."""
+    import ctypes
+    import numpy as np
+    from genericschur import _lib
+    ns = [int(n) for n in gen.stream(56, small, len(large)).integers(1, 33, size=small)] + large + [0]
+    r = gen.stream(56, 1, small)
+    Ss, _ = gs.gschur_batched([gen.ginibre_complex(n, r) if cplx else gen.ginibre_real(n, r) for n in ns])
+    n_, off, T = gs.pack([S.T for S in Ss], np.complex128 if cplx else np.float64)
+    _, _, Z = gs.pack([S.Z for S in Ss], T.dtype)
+    V = np.zeros(T.shape, dtype=np.complex128)
+    h = _lib.handle()
+    p = lambda a: ctypes.c_void_p(a.ctypes.data)
+    f = _lib.lib().gs_trevc_batched_z if cplx else _lib.lib().gs_trevc_batched_d
+    k = kernels(lambda: _lib.check(f(h, len(n_), p(n_), p(off), p(T), p(Z), p(V), 0, 1, 0), h, "gs_trevc_batched"))
+    assert any("trevc_small" in x for x in k) == own, k
+    for S, X in list(zip(Ss, gs.unpack(n_, off, V)))[:-1:16]:
+        assert np.array_equal(X, gs.geigvecs(S))
+
+
 def _device_batch(ns, cplx):
     import numpy as np
     import torch
